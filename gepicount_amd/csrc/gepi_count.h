@@ -118,7 +118,7 @@ __global__ void __launch_bounds__(POPC_THREADS) k_count_popc(CountArgs g) {
         for (int kk = split; kk < end; kk += 4) popc_step<1>(sA, sB, ty, tx, kk, acc);
     }
 
-    const FilterConsts fc = filter_consts(g.st, g.n0, g.n1);
+    const FilterConsts fc = filter_consts(g.st, g);
 #pragma unroll
     for (int i = 0; i < 2; i++) {
 #pragma unroll
@@ -264,7 +264,7 @@ __global__ void __launch_bounds__(MF_THREADS, 2) k_count_mfma(CountArgs g) {
 
     /* epilogue: lane holds D[4*lg + r][l16] of each 16x16 block, i.e. A
      * variant 32wa + 16i + 4lg + r against B variant 32wb + 16j + l16.     */
-    const FilterConsts fc = filter_consts(g.st, g.n0, g.n1);
+    const FilterConsts fc = filter_consts(g.st, g);
     const bool c0_high = g.cls0_high != 0; /* class 0 held in the high part */
 #pragma unroll
     for (int i = 0; i < 2; i++) {
@@ -543,7 +543,7 @@ __device__ __forceinline__ void count_f4_tile(const CountArgs &g, int64_t tile) 
 
     /* epilogue: lane holds D[4*lg + r][l16] of each 16x16 block, i.e. A
      * variant 32wa + 16i + 4lg + r against B variant 16wb + l16.           */
-    const FilterConsts fc = filter_consts(g.st, g.n0, g.n1);
+    const FilterConsts fc = filter_consts(g.st, g);
 #pragma unroll
     for (int i = 0; i < 2; i++) {
 #pragma unroll
@@ -805,7 +805,7 @@ __device__ __forceinline__ void count_f4_run(const Src &src) {
 
         /* the filter's constants are read before the next tile's loads are
          * issued: waits on global loads are in issue order */
-        const FilterConsts fc = filter_consts(g.st, g.n0, g.n1);
+        const FilterConsts fc = filter_consts(g.st, g);
         /* next job (written before this tile's first barrier) and its first
          * super-step, in flight during the filter */
         const F4Job nj = uniform_job(s_job[(t + 1) & 1]);
@@ -1108,7 +1108,7 @@ __device__ __forceinline__ void count_f4w_unit(const CountArgs &g, int64_t unit,
         u_end = nu_live;
     }
 
-    const FilterConsts fc = filter_consts(g.st, g.n0, g.n1);
+    const FilterConsts fc = filter_consts(g.st, g);
     __syncthreads(); /* the stage counter is cleared, the park region claimed */
     const bool parks = PARK && sh.park_slot != PARK_NONE;
     PairListG pl{&sh.n_park, parks ? g.park + (int64_t)sh.park_slot * g.park_cap : nullptr,

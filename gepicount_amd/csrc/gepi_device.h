@@ -40,7 +40,8 @@ struct ScanState {
     double thr_score;          /* admission key: (thr_score, thr_idx), inclusive   */
     uint64_t thr_idx;
     float filt_k;              /* entropy filter coefficient, 0 = admit everything */
-    uint32_t thr_pad[59];
+    float filt_t;              /* entropy: the threshold in nats, rounded down     */
+    uint32_t thr_pad[58];
     uint32_t overflow;         /* candidate buffer overflowed in this band          */
     uint32_t pad2;
     unsigned long long count;  /* records in the active candidate buffer           */
@@ -80,6 +81,8 @@ struct CountArgs {
     int32_t f32;              /* fp4: class sizes for which the filter may work on
                                * the fp32 counts (f32_counts)                    */
     int32_t n0, n1;           /* class sizes (bounds of y and z: Fisher filter)   */
+    float h0, h1;             /* chi-square coefficient per nat: h0 + h1 min(y, z)
+                               * (chi2_slope)                                     */
     ScanState *st;
     Pend *pend;
     unsigned long long pcap;
@@ -269,6 +272,8 @@ __device__ __forceinline__ void stage_flush(const CountArgs &g, PendStage &ps) {
 struct FilterConsts {
     double thr_s; /* admission score threshold                                 */
     float kf;     /* entropy: chi-square coefficient, 0 = admit everything      */
+    float k0, k1; /* entropy: another, k0 + k1 min(y, z); the larger one counts */
+    float h0, h1; /* Fisher: the same per nat                                   */
     float a_s;    /* Fisher: -(thr + 1e-6) ln 10 - ln(4 n0 n1) / 2 + 0.9189,
                    * less a float error margin                                 */
 };
@@ -279,11 +284,16 @@ struct FilterConsts {
  * counter that every workgroup updates, so each workgroup waited for that
  * line before its filter (20,000 x 2,048, 2^15 workgroups: 3.24 ms against
  * 1.85 ms).                                                                */
-__device__ __forceinline__ FilterConsts filter_consts(const ScanState *st, int32_t n0, int32_t n1) {
+__device__ __forceinline__ FilterConsts filter_consts(const ScanState *st, const CountArgs &g) {
     const auto *c = (const __attribute__((address_space(4))) ScanState *)(uintptr_t)st;
     FilterConsts fc;
     fc.thr_s = c->thr_score;
     fc.kf = c->filt_k;
+    fc.h0 = g.h0;
+    fc.h1 = g.h1;
+    fc.k0 = c->filt_t * g.h0;
+    fc.k1 = c->filt_t * g.h1;
+    const int32_t n0 = g.n0, n1 = g.n1;
     const double a = -(fc.thr_s + 1e-6) * 2.302585092994046;
     const double A = a - 0.5 * log(4.0 * (double)(n0 > 1 ? n0 : 1) * (double)(n1 > 1 ? n1 : 1)) +
                      0.9189;
@@ -356,8 +366,18 @@ __device__ __forceinline__ void push_mask(const CountArgs &g, PendStage &ps, con
  * information of the class x f table (nats) and chi2/m = D^2/(y z q),
  * D = wz - xy, q = xx(m - xx), Jensen on the KL divergence gives
  * I <= ln(1 + chi2/m), so I >= T requires D^2 >= expm1(T) * y * z * q.
- * Entropy: -I_bits <= thr needs T = -thr * ln 2 (kf = 2^-thr - 1, made on
- * the host side of the threshold update, rounded down).
+ * The second bound is I <= g(p) chi2/m with p = min(y, z)/m and g(p) =
+ * -ln(1-p) (1-p)/p, the largest ratio of KL(a||p) to (a-p)^2/(p(1-p)) over
+ * a (at the end a = 0; I is the mean of the KL terms of f = 0 and f = 1 and
+ * chi2/m that of the quadratic ones): I >= T requires D^2 >= T/g(p) * y z q.
+ * 1/g runs from 1 at p = 0 to 1.44 at 1/2 and is convex, so its tangent at
+ * the scan's class fraction, taken at min(y, z)/(n0+n1) <= p, is a lower
+ * bound (chi2_slope); the larger of the two coefficients is used.  Tables
+ * near the threshold have small T, so with even classes a table needs
+ * 1.44 times the chi-square to pass (entropy, top-1,000 of 20,000 x 2,048: 5.79 -> 3.69
+ * ms, Fisher 7.47 -> 5.99; large scan 120.4 -> 116.6).
+ * Entropy: -I_bits <= thr needs T = -thr * ln 2 (kf = 2^-thr - 1 and T made
+ * where the threshold is updated, rounded down).
  * Fisher: p >= P(obs) = C(y,w) C(z,x) / C(m,xx); e^{nH(k/n)} / sqrt(2n) <=
  * C(n,k) for the numerator and C(m,xx) <= e^{mH} sqrt(m / (2 pi xx (m-xx)))
  * (1 <= xx <= m-1; H in nats) give P(obs) >= e^{-mI} sqrt(2 pi (m-1) / m) /
@@ -496,18 +516,20 @@ __device__ __forceinline__ void filter_pair(const CountArgs &g, PendStage &ps, c
     const CT y = c[0][2][2], z = c[1][2][2];
     const CT m = tot ? tot[2][2] : y + z;
     const float mf = (float)m;
-    float K = fc.kf;
+    const float mn = (float)(y < z ? y : z);
+    float K = fmaxf(fc.kf, __builtin_fmaf(fc.k1, mn, fc.k0));
     if (FFUN == GEPI_FFUNC_FISHERPV) {
         K = 0.0f;
         if (fc.thr_s < 0.0) {
             /* T = (a - ln(4yz)/2 + 0.9189 - 1/m) / m at ln(4yz) <= ln(4 n0 n1)
-             * (a_s; y <= n0, z <= n1), and K = T (1 + T/2) <= expm1(T): both
-             * only lower K; 0.9189 - 1/m <= ln(2 pi (m-1)/m) / 2 comes from
+             * (a_s; y <= n0, z <= n1), and K = T (1 + T/2) <= expm1(T) or
+             * T (h0 + h1 min(y, z)) <= T/g(p): both only lower K; 0.9189 - 1/m <= ln(2 pi (m-1)/m) / 2 comes from
              * C(m, xx) <= e^{m H} sqrt(m / (2 pi xx (m - xx))), 1 <= xx <= m-1
              * (the other tables have P(obs) = 1 and D = 0) */
             const float r = __builtin_amdgcn_rcpf(m > 1 ? mf : 1.0f);
             const float T = (fc.a_s - r) * r;
-            if (T > 0.0f) K = T * (1.0f + 0.5f * T) * (1.0f - 2e-5f);
+            if (T > 0.0f)
+                K = T * fmaxf(1.0f + 0.5f * T, __builtin_fmaf(fc.h1, mn, fc.h0)) * (1.0f - 2e-5f);
         }
     }
     RowTest<CT> rt;

@@ -11,6 +11,7 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <cmath>
 #include <vector>
 
 #include "../../include/gepicount.h"
@@ -98,6 +99,24 @@ int grow(T **ptr, size_t *have, size_t need) {
     return GEPI_OK;
 }
 
+
+/* Coefficients of a lower bound of 1/g(p), p = min(y, z)/(y + z), over the
+ * tables of a scan with classes of n0 and n1 samples (y <= n0, z <= n1):
+ * 1/g(p) >= h0 + h1 min(y, z), the tangent of the convex 1/g at p0 =
+ * min(n0, n1)/(n0 + n1) (g as in gepi_device.h's filter), less 1e-6 for the
+ * roundings.                                                              */
+inline void chi2_slope(int32_t n0, int32_t n1, float *h0, float *h1) {
+    const double n = (double)n0 + n1, p = n > 0 ? std::min(n0, n1) / n : 0.0;
+    double h = 1.0, d = 0.5; /* 1/g and its slope at p = 0 */
+    if (p > 0.0) {
+        const double l = -std::log1p(-p), g = l * (1.0 - p) / p;
+        h = 1.0 / g;
+        /* the difference loses digits for small p, where it nears 1/2 */
+        d = p < 1e-4 ? 0.5 : (l / (p * p) - 1.0 / p) / (g * g);
+    }
+    *h0 = (float)(h - d * p - 1e-6);
+    *h1 = n > 0 ? (float)(d / n * (1.0 - 1e-6)) : 0.0f;
+}
 
 /* Sorts candidate records by the canonical key and writes the first
  * min(k, size) as results; returns how many were written.                   */

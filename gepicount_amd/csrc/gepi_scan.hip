@@ -624,6 +624,7 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
     ca.f32 = f32_counts(n0, n1) ? 1 : 0;
     ca.n0 = n0;
     ca.n1 = n1;
+    chi2_slope(n0, n1, &ca.h0, &ca.h1);
     ca.st = b.state;
     ca.pend = b.pend;
     ca.pcap = pcap;

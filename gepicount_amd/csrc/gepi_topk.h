@@ -223,16 +223,20 @@ __device__ __forceinline__ void adopt_threshold(ScanState *st, uint64_t key_hi, 
     const double thr = from_order_bits(key_hi);
     st->thr_score = thr;
     st->thr_idx = key_lo;
-    float kf = 0.0f;
+    float kf = 0.0f, kt = 0.0f;
     if (ffun == GEPI_FFUNC_ENTROPY) {
         double it = -thr - 1e-12;
         if (it > 0.0) {
             double k = expm1(it * 0.6931471805599453) * (1.0 - 1e-6);
             kf = (float)k;
             if ((double)kf > k) kf = nextafterf(kf, 0.0f);
+            const double t = it * 0.6931471805599453 * (1.0 - 1e-6);
+            kt = (float)t;
+            if ((double)kt > t) kt = nextafterf(kt, 0.0f);
         }
     }
     st->filt_k = kf;
+    st->filt_t = kt;
 }
 
 /* After a compaction: adopt the compacted buffer and the new threshold. */

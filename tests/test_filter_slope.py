@@ -1,0 +1,49 @@
+"""The filters' class-fraction coefficient (CPU, exact math).
+
+I <= g(p) chi2/m with p = min(y, z)/m, g(p) = -ln(1-p) (1-p)/p, and the
+tangent h0 + h1 min(y, z) <= 1/g(p) that the kernels use for tables of a
+scan with classes of n0 >= y and n1 >= z samples (chi2_slope, restated here
+with its float32 results).
+"""
+import math
+
+import numpy as np
+import pytest
+
+from test_filter_bounds import all_small_tables, chi2_over_m, mi_nats, tables
+
+
+def g(p):
+    return 1.0 - p / 2 if p < 1e-9 else -math.log1p(-p) * (1.0 - p) / p
+
+
+def slope(n0, n1):
+    n = n0 + n1
+    p = min(n0, n1) / n if n else 0.0
+    h, d = 1.0, 0.5
+    if p > 0.0:
+        h = 1.0 / g(p)
+        d = 0.5 if p < 1e-4 else (-math.log1p(-p) / (p * p) - 1.0 / p) / (g(p) * g(p))
+    return np.float32(h - d * p - 1e-6), np.float32(d / n * (1.0 - 1e-6)) if n else np.float32(0.0)
+
+
+def test_information_below_class_fraction_bound():
+    rng = np.random.default_rng(11)
+    for w, x, y, z in list(all_small_tables(14)) + list(tables(rng, 20000, 5000)):
+        b = g(min(y, z) / (y + z)) * chi2_over_m(w, x, y, z)
+        assert mi_nats(w, x, y, z) <= b + 1e-12 * max(1.0, b), (w, x, y, z)
+
+
+@pytest.mark.parametrize("n0,n1", [(0, 0), (0, 7), (1, 1), (1, 46339), (45, 44), (128, 128),
+                                   (465, 273), (1024, 1024), (5734, 2458), (2, 20000),
+                                   (23170, 23170), (6000, 14001)])
+def test_tangent_below_inverse(n0, n1):
+    h0, h1 = slope(n0, n1)
+    ys = np.unique(np.linspace(0, n0, 200).astype(int))
+    zs = np.unique(np.linspace(0, n1, 200).astype(int))
+    for y in ys:
+        for z in zs:
+            if y + z == 0:
+                continue
+            k = np.float32(h0 + np.float32(h1 * np.float32(min(y, z))))
+            assert float(k) <= 1.0 / g(min(y, z) / (y + z)), (n0, n1, y, z)
