@@ -64,12 +64,17 @@ struct gepi_panel {
     size_t park_bytes = 0;
     gepi::Cand *d_cand[2] = {nullptr, nullptr};
     gepi::Pend *d_pend = nullptr;
-    unsigned long long buf_cap = 0;  /* records in each candidate buffer */
+    unsigned long long buf_cap = 0;  /* records in the candidate buffer  */
+    unsigned long long buf2_cap = 0; /* records in the second one        */
     unsigned long long pend_cap = 0; /* records in the pending list       */
     gepi::ScanState *d_state = nullptr;
     uint64_t *d_small = nullptr;
     DeviceTables tabs;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
+    std::vector<hipEvent_t> band_ev; /* two per band of a planned scan */
+    /* pinned, mapped: the band reports and small result lists the device
+     * writes (HostMail) */
+    void *mail = nullptr;
 };
 
 

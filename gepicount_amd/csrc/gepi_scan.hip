@@ -24,6 +24,7 @@
  * synchronises once per band to read the state and size the next band; only
  * the final k records are copied to the host.
  */
+#include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -141,6 +142,15 @@ static __device__ __align__(256) unsigned char scratch[SCRATCH_BYTES];
 
 namespace {
 
+/* What a planned scan's kernels write for the host (pinned memory): a
+ * report per enqueued band, and the final records when they are few. */
+constexpr int PLAN_BANDS = 48;        /* bands enqueued between two waits       */
+constexpr int64_t MAIL_RECORDS = 2048;
+struct HostMail {
+    ItemReport report[PLAN_BANDS];
+    Cand rec[MAIL_RECORDS];
+};
+
 int panel_alloc(gepi_panel *p, int device, int64_t n_var, int32_t n_samples) {
     p->device = device;
     p->n_var = n_var;
@@ -154,6 +164,7 @@ int panel_alloc(gepi_panel *p, int device, int64_t n_var, int32_t n_samples) {
     HIP_TRY(hipMalloc(&p->d_small, sizeof(uint64_t) * 2 * SEL_SMALL));
     HIP_TRY(hipEventCreate(&p->ev0));
     HIP_TRY(hipEventCreate(&p->ev1));
+    HIP_TRY(hipHostMalloc(&p->mail, sizeof(HostMail), hipHostMallocDefault));
     return GEPI_OK;
 }
 
@@ -175,6 +186,8 @@ void panel_free(gepi_panel *p) {
     hipFree(p->tabs.lhi);
     hipFree(p->tabs.llo);
     hipFree(p->tabs.lfact);
+    for (hipEvent_t e : p->band_ev) hipEventDestroy(e);
+    if (p->mail) hipHostFree(p->mail);
     if (p->ev0) hipEventDestroy(p->ev0);
     if (p->ev1) hipEventDestroy(p->ev1);
     if (p->stream) hipStreamDestroy(p->stream);
@@ -332,7 +345,8 @@ inline bool wg_select(int path, unsigned long long count) {
 }
 
 TopkDesc topk_desc(const ScanBufs &b, int cur, unsigned long long cap, int64_t k,
-                   const gepi_params *par, int64_t t0, int64_t t1, int64_t n_a4) {
+                   const gepi_params *par, int64_t t0, int64_t t1, int64_t n_a4,
+                   ItemReport *report = nullptr) {
     TopkDesc d;
     memset(&d, 0, sizeof d);
     d.st = b.state;
@@ -340,7 +354,7 @@ TopkDesc topk_desc(const ScanBufs &b, int cur, unsigned long long cap, int64_t k
     d.cap = cap;
     d.drop_t0 = t0;
     d.drop_t1 = t1;
-    d.report = nullptr;
+    d.report = report;
     d.k = (uint32_t)k;
     d.ffun = par->ffun;
     d.n_a4 = (int32_t)n_a4;
@@ -354,6 +368,70 @@ thread_local void *g_progress_user = nullptr;
 double ms_since(std::chrono::steady_clock::time_point t) {
     return std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t).count();
 }
+
+/* ---- planned bands --------------------------------------------------------
+ * A scan's bands need no answer from the device between them: a band's
+ * count, exact and top-k launches find the threshold, the lists and an
+ * overflow flag in device memory, so all of them can be enqueued at once and
+ * their reports read at the end (bands that overflowed are redone; the order
+ * of bands does not change the result).  What has to be chosen beforehand is
+ * the size of each band, from how many evaluations its threshold lets
+ * through, and a threshold for the first one.
+ *
+ * Without association 2 m I (I in nats) of a table is close to chi-square
+ * with one degree of freedom, and P(p <= a) of a Fisher test is at most a.
+ * So the first band admits the quantile where GUESS times k of its
+ * evaluations are expected: few enough to be cheap, and if the k best are
+ * among them (nearly always: the count says so) the threshold was valid.  A
+ * scan that ends with fewer than k records is run again without it.
+ * Against bands that began with one tile admitting everything and grew
+ * fourfold, a host round trip (40 us) and a selection between two: 1,024 x
+ * 256 0.73 -> 0.13 ms (5 bands -> 1), 3,001 x 777 Fisher 1.44 -> 0.29, 20,000
+ * x 2,048 3.69 -> 2.38 (10 -> 3), 8,000 x 20,001 3.84 -> 2.50.               */
+constexpr double GUESS_ENTROPY = 8.0, GUESS_FISHER = 16.0;
+
+/* P(chi2_1 > t) and its inverse */
+inline double chi2_tail(double t) { return std::erfc(std::sqrt(0.5 * std::max(t, 0.0))); }
+double chi2_quantile(double p) {
+    double lo = 0.0, hi = 1400.0;
+    for (int i = 0; i < 60; i++) {
+        const double mid = 0.5 * (lo + hi);
+        (chi2_tail(mid) > p ? lo : hi) = mid;
+    }
+    return lo;
+}
+
+struct BandPlan {
+    bool entropy;
+    double evals_tile;  /* evaluations per tile                              */
+    double h;           /* chi-square coefficient per nat (chi2_slope)       */
+    double k;
+    double most;        /* survivors a band may have                         */
+    double factor = 1.0; /* survivors measured over survivors expected       */
+
+    /* Expected survivors per evaluation under the threshold that admits a
+     * share q: the filter's chi-square cut is h/2 of the quantile; Fisher's
+     * exact check of log10 P(obs) admits a few times the two-sided p.      */
+    double pass(double q) const {
+        q = std::min(q, 1.0);
+        return entropy ? chi2_tail(0.5 * h * chi2_quantile(q)) : std::min(1.0, 4.0 * q);
+    }
+    double survivors(int64_t tiles, double q) const {
+        return factor * (double)tiles * evals_tile * pass(q);
+    }
+    /* Tiles of the band that follows `done` tiles.  About 250,000 survivors
+     * cost what a band's fixed part does (100 us); at least three times what
+     * is done while the list holds them.                                    */
+    int64_t next(int64_t done, int64_t left) const {
+        const double q = 1.3 * k / ((double)done * evals_tile);
+        const double per = factor * evals_tile * pass(q);
+        const double cheap = std::max(250000.0 / per, 3.0 * (double)done);
+        const double tiles = std::min({cheap, most / per, 1048576.0, (double)left});
+        /* a remainder below a fifth of the band goes with it */
+        if ((double)left < 1.2 * tiles && (double)left * per < most) return left;
+        return std::max<int64_t>(1, (int64_t)tiles);
+    }
+};
 
 int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case,
              const gepi_params *par, gepi_result *tops, int64_t *n_tops,
@@ -479,8 +557,14 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
      * one-tile band admits at most TILE_EVALS_MAX, so cap >= k +
      * TILE_EVALS_MAX lets a band shrunk to one tile always complete.        */
     const unsigned long long cap_min = (unsigned long long)k + TILE_EVALS_MAX + 1024;
+    /* 4k or 2^23 records, but no more than a 64th of the evaluations: bands
+     * are sized for the lists, and a drop-in call allocates them anew (a
+     * list of 2^23 records cost 0.5 ms to allocate and free, with 80 bytes a
+     * record three fifths of a 1,020 x 89 call)                             */
     unsigned long long cap = std::max<unsigned long long>(
-        cap_min, (unsigned long long)std::max<int64_t>(4 * k, 1 << 23));
+        cap_min, std::min<unsigned long long>(
+                     (unsigned long long)std::max<int64_t>(4 * k, 1 << 23),
+                     std::max<unsigned long long>((unsigned long long)total_evals / 64, 1u << 18)));
     if (const char *env = getenv("GEPI_CAND_CAP")) {
         /* capacity override for exercising the overflow recovery in tests */
         cap = std::max<unsigned long long>((unsigned long long)std::max(atoll(env), 0ll), cap_min);
@@ -524,15 +608,13 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
         if (fp4 &&
             (rc = grow(&p->d_cw, &p->cw_bytes, cw.size() * sizeof(CompressWord))) != GEPI_OK)
             return rc;
-        if (cap > p->buf_cap) alloc += (int64_t)(2 * sizeof(Cand) * cap);
+        if (cap > p->buf_cap) alloc += (int64_t)(sizeof(Cand) * cap);
         if (pcap > p->pend_cap) alloc += (int64_t)(sizeof(Pend) * pcap);
         if (cap > p->buf_cap) {
             hipFree(p->d_cand[0]);
-            hipFree(p->d_cand[1]);
-            p->d_cand[0] = p->d_cand[1] = nullptr;
+            p->d_cand[0] = nullptr;
             p->buf_cap = 0;
             HIP_TRY(hipMalloc(&p->d_cand[0], sizeof(Cand) * cap));
-            HIP_TRY(hipMalloc(&p->d_cand[1], sizeof(Cand) * cap));
             p->buf_cap = cap;
         }
         if (pcap > p->pend_cap) {
@@ -547,7 +629,6 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
         b.perm = p->d_perm;
         b.cw = p->d_cw;
         b.cand[0] = p->d_cand[0];
-        b.cand[1] = p->d_cand[1];
         b.pend = p->d_pend;
         b.state = p->d_state;
         b.small = p->d_small;
@@ -595,17 +676,18 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
     }
     HIP_TRY(hipEventRecord(p->ev1, p->stream));
 
-    ScanState init;
-    memset(&init, 0, sizeof init);
-    init.thr_score = INFINITY;
-    init.thr_idx = ~0ull;
-    HIP_TRY(hipMemcpyAsync(b.state, &init, sizeof init, hipMemcpyHostToDevice, p->stream));
-    HIP_TRY(hipStreamSynchronize(p->stream));
-    {
+    /* state of a scan that admits everything scoring at most thr */
+    auto init_state = [&](double thr) {
+        float kf, kt;
+        threshold_coeffs(thr, par->ffun, kf, kt);
+        k_state_init<<<1, 256, 0, p->stream>>>(b.state, thr, kf, kt);
+        return hipGetLastError();
+    };
+    auto read_prepare = [&]() {
         float ms = 0;
         hipEventElapsedTime(&ms, p->ev0, p->ev1);
         st_local.ms_prepare = ms;
-    }
+    };
 
     int cur = 0; /* active candidate buffer */
     CountArgs ca;
@@ -671,54 +753,184 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
     const bool f32 = ca.f32 != 0;
     /* wave tiles: the kernel built with parking where the scan parks */
     const bool park = f4w_park;
-    while (t0 < n_tiles) {
-        const int64_t t1 = std::min<int64_t>(n_tiles, t0 + band);
-        ca.tile_begin = t0;
-        ca.n_tiles = (int32_t)(t1 - t0);
-        ea.cand = b.cand[cur];
-        k_reset_pending<<<1, 1, 0, p->stream>>>(b.state);
-        HIP_TRY(hipEventRecord(p->ev0, p->stream));
-        const unsigned grid = path == 3 ? (unsigned)((t1 - t0 + 1) / 2) : (unsigned)(t1 - t0);
+    /* the count kernel over tiles [c0, c1), its duration between the events */
+    auto launch_count = [&](int64_t c0, int64_t c1, hipEvent_t e0, hipEvent_t e1) {
+        ca.tile_begin = c0;
+        ca.n_tiles = (int32_t)(c1 - c0);
+        const unsigned grid = path == 3 ? (unsigned)((c1 - c0 + 1) / 2) : (unsigned)(c1 - c0);
+        auto go = [&](auto kernel, unsigned threads) {
+            hipExtLaunchKernelGGL(kernel, dim3(grid), dim3(threads), 0, p->stream, e0, e1, 0, ca);
+        };
         if (path == 3) {
             if (entropy && f32 && park)
-                k_count_f4w<GEPI_FFUNC_ENTROPY, true, true><<<grid, F4W_THREADS, 0, p->stream>>>(ca);
+                go(k_count_f4w<GEPI_FFUNC_ENTROPY, true, true>, F4W_THREADS);
             else if (entropy && f32)
-                k_count_f4w<GEPI_FFUNC_ENTROPY, true, false><<<grid, F4W_THREADS, 0, p->stream>>>(ca);
+                go(k_count_f4w<GEPI_FFUNC_ENTROPY, true, false>, F4W_THREADS);
             else if (entropy && park)
-                k_count_f4w<GEPI_FFUNC_ENTROPY, false, true><<<grid, F4W_THREADS, 0, p->stream>>>(ca);
+                go(k_count_f4w<GEPI_FFUNC_ENTROPY, false, true>, F4W_THREADS);
             else if (entropy)
-                k_count_f4w<GEPI_FFUNC_ENTROPY, false, false><<<grid, F4W_THREADS, 0, p->stream>>>(ca);
+                go(k_count_f4w<GEPI_FFUNC_ENTROPY, false, false>, F4W_THREADS);
             else if (f32)
-                k_count_f4w<GEPI_FFUNC_FISHERPV, true, true><<<grid, F4W_THREADS, 0, p->stream>>>(ca);
+                go(k_count_f4w<GEPI_FFUNC_FISHERPV, true, true>, F4W_THREADS);
             else
-                k_count_f4w<GEPI_FFUNC_FISHERPV, false, true><<<grid, F4W_THREADS, 0, p->stream>>>(ca);
+                go(k_count_f4w<GEPI_FFUNC_FISHERPV, false, true>, F4W_THREADS);
         } else if (path == 4) {
             if (entropy && f32)
-                k_count_f4<GEPI_FFUNC_ENTROPY, true><<<grid, F4_THREADS, 0, p->stream>>>(ca);
+                go(k_count_f4<GEPI_FFUNC_ENTROPY, true>, F4_THREADS);
             else if (entropy)
-                k_count_f4<GEPI_FFUNC_ENTROPY, false><<<grid, F4_THREADS, 0, p->stream>>>(ca);
+                go(k_count_f4<GEPI_FFUNC_ENTROPY, false>, F4_THREADS);
             else if (f32)
-                k_count_f4<GEPI_FFUNC_FISHERPV, true><<<grid, F4_THREADS, 0, p->stream>>>(ca);
+                go(k_count_f4<GEPI_FFUNC_FISHERPV, true>, F4_THREADS);
             else
-                k_count_f4<GEPI_FFUNC_FISHERPV, false><<<grid, F4_THREADS, 0, p->stream>>>(ca);
+                go(k_count_f4<GEPI_FFUNC_FISHERPV, false>, F4_THREADS);
         } else if (path == 2) {
             if (entropy)
-                k_count_mfma<GEPI_FFUNC_ENTROPY><<<grid, MF_THREADS, 0, p->stream>>>(ca);
+                go(k_count_mfma<GEPI_FFUNC_ENTROPY>, MF_THREADS);
             else
-                k_count_mfma<GEPI_FFUNC_FISHERPV><<<grid, MF_THREADS, 0, p->stream>>>(ca);
+                go(k_count_mfma<GEPI_FFUNC_FISHERPV>, MF_THREADS);
         } else {
             if (entropy)
-                k_count_popc<GEPI_FFUNC_ENTROPY><<<grid, POPC_THREADS, 0, p->stream>>>(ca);
+                go(k_count_popc<GEPI_FFUNC_ENTROPY>, POPC_THREADS);
             else
-                k_count_popc<GEPI_FFUNC_FISHERPV><<<grid, POPC_THREADS, 0, p->stream>>>(ca);
+                go(k_count_popc<GEPI_FFUNC_FISHERPV>, POPC_THREADS);
         }
-        HIP_TRY(hipGetLastError());
-        HIP_TRY(hipEventRecord(p->ev1, p->stream));
-        auto ts = std::chrono::steady_clock::now();
+    };
+    auto launch_exact = [&]() {
         if (entropy)
             k_exact<GEPI_FFUNC_ENTROPY><<<1024, 256, 0, p->stream>>>(ea);
         else
             k_exact<GEPI_FFUNC_FISHERPV><<<1024, 256, 0, p->stream>>>(ea);
+    };
+
+    /* ---- all bands enqueued at once (fp4, small k) ---- */
+    std::vector<Cand> host;
+    bool finished = false, prepare_read = false;
+    BandPlan plan;
+    plan.entropy = entropy;
+    plan.evals_tile = (double)evals_per_tile;
+    plan.h = (double)ca.h0 + (double)ca.h1 * std::min(n0, n1);
+    plan.k = (double)k;
+    plan.most = (double)pcap / 4;
+    const double guess = entropy ? GUESS_ENTROPY : GUESS_FISHER;
+    /* the share of n tiles' evaluations that the first threshold admits */
+    auto share = [&](int64_t n) { return guess * (double)k / ((double)n * evals_per_tile); };
+    /* the first band: a scan of up to about 5,000 variants whole, else one
+     * tile per workgroup the chip holds, as a pilot for the others' sizes */
+    int64_t first = n_tiles <= 6400 ? n_tiles : 1024;
+    if (first == n_tiles && n_tiles > 1024 && plan.survivors(first, share(first)) > 600000.0) first = 1024;
+    const bool hooks = forced_band || getenv("GEPI_CAND_CAP") || getenv("GEPI_PEND_CAP");
+    const bool planned = fp4 && n_ks > 0 && !hooks && !par->intermediate && par->max_grid_area <= 0 &&
+                         share(first) <= 0.02 && 1.5 * (guess + 1.0) * (double)k <= (double)cap &&
+                         (guess + 1.0) * (double)k <= (double)WG_SELECT_MAX &&
+                         plan.survivors(first, share(first)) <= plan.most;
+    if (planned) {
+        HostMail *mail = static_cast<HostMail *>(p->mail);
+        while (p->band_ev.size() < 2 * PLAN_BANDS) {
+            hipEvent_t e;
+            HIP_TRY(hipEventCreate(&e));
+            p->band_ev.push_back(e);
+        }
+        const double q = share(first);
+        HIP_TRY(init_state(entropy ? -chi2_quantile(q) / (2.0 * (n0 + n1)) * 1.4426950408889634
+                                   : std::log10(q)));
+        ea.cand = b.cand[0];
+        struct Job {
+            int64_t t0, t1;
+        };
+        std::vector<Job> jobs(1, Job{0, first}), redo;
+        int64_t upto = first; /* tiles given to jobs so far */
+        while (!jobs.empty()) {
+            const int nj = (int)std::min<size_t>(jobs.size(), PLAN_BANDS);
+            for (int j = 0; j < nj; j++) {
+                launch_count(jobs[j].t0, jobs[j].t1, p->band_ev[2 * j], p->band_ev[2 * j + 1]);
+                launch_exact();
+                k_topk_one<<<1, TOPK_THREADS, 0, p->stream>>>(topk_desc(
+                    b, 0, cap, k, par, jobs[j].t0, jobs[j].t1, n_a4, &mail->report[j]));
+            }
+            HIP_TRY(hipGetLastError());
+            /* the records, in case these bands are the last */
+            const bool last_jobs = upto == n_tiles && nj == (int)jobs.size();
+            const bool by_mail = k <= MAIL_RECORDS;
+            if (last_jobs && by_mail)
+                HIP_TRY(hipMemcpyAsync(mail->rec, b.cand[0], sizeof(Cand) * k, hipMemcpyDeviceToHost,
+                                       p->stream));
+            HIP_TRY(hipStreamSynchronize(p->stream));
+            if (!prepare_read) read_prepare();
+            prepare_read = true;
+            redo.clear();
+            for (int j = 0; j < nj; j++) {
+                const ItemReport &r = mail->report[j];
+                float ms = 0;
+                hipEventElapsedTime(&ms, p->band_ev[2 * j], p->band_ev[2 * j + 1]);
+                ms_count += ms;
+                bands++;
+                count = r.count;
+                if (r.pend_overflow || r.cand_overflow) {
+                    /* survivors or candidates lost (the band's candidates are
+                     * dropped already): redo it in pieces                   */
+                    (r.pend_overflow ? st_local.pend_overflows : st_local.cand_overflows)++;
+                    const int64_t n = jobs[j].t1 - jobs[j].t0, piece = std::max<int64_t>(1, n / 4);
+                    for (int64_t c = jobs[j].t0; c < jobs[j].t1; c += piece)
+                        redo.push_back(Job{c, std::min(jobs[j].t1, c + piece)});
+                } else {
+                    exact_total += r.pend_count;
+                }
+            }
+            if (upto < n_tiles) {
+                /* after the pilot: was its threshold sound, how many
+                 * survivors did it have, and the other bands             */
+                if (redo.empty() && count < (unsigned long long)k / 4) break;
+                plan.factor = std::min(64.0, std::max(0.25, (double)mail->report[0].pend_count /
+                                                                std::max(1.0, plan.survivors(first, q))));
+                for (; upto < n_tiles; upto = redo.back().t1)
+                    redo.push_back(Job{upto, upto + plan.next(upto, n_tiles - upto)});
+            }
+            redo.insert(redo.end(), jobs.begin() + nj, jobs.end());
+            jobs.swap(redo);
+            if (jobs.empty() && count == (unsigned long long)k) {
+                host.resize((size_t)k);
+                if (by_mail)
+                    memcpy(host.data(), mail->rec, sizeof(Cand) * (size_t)k);
+                else
+                    HIP_TRY(hipMemcpyAsync(host.data(), b.cand[0], sizeof(Cand) * k,
+                                           hipMemcpyDeviceToHost, p->stream));
+                HIP_TRY(hipStreamSynchronize(p->stream));
+                finished = true;
+            }
+        }
+        /* fewer than k records under the guessed threshold: run it without */
+        if (!finished) count = exact_total = 0;
+    }
+    if (!finished) {
+        HIP_TRY(init_state(INFINITY));
+        HIP_TRY(hipStreamSynchronize(p->stream));
+        if (!prepare_read) read_prepare();
+    } else {
+        t0 = n_tiles;
+    }
+    /* the second candidate list, where the multi-launch selection compacts
+     * from one into the other: allocated when it first runs */
+    auto second_list = [&]() -> int {
+        if (b.cand[1]) return GEPI_OK;
+        if (cap > p->buf2_cap) {
+            hipFree(p->d_cand[1]);
+            p->d_cand[1] = nullptr;
+            p->buf2_cap = 0;
+            HIP_TRY(hipMalloc(&p->d_cand[1], sizeof(Cand) * cap));
+            p->buf2_cap = cap;
+            st_local.bytes_allocated += (int64_t)(sizeof(Cand) * cap);
+        }
+        b.cand[1] = p->d_cand[1];
+        return GEPI_OK;
+    };
+    while (t0 < n_tiles) {
+        const int64_t t1 = std::min<int64_t>(n_tiles, t0 + band);
+        ea.cand = b.cand[cur];
+        k_reset_pending<<<1, 1, 0, p->stream>>>(b.state);
+        launch_count(t0, t1, p->ev0, p->ev1);
+        HIP_TRY(hipGetLastError());
+        auto ts = std::chrono::steady_clock::now();
+        launch_exact();
         HIP_TRY(hipGetLastError());
         ScanState hs;
         if ((rc = read_state(p, b, &hs)) != GEPI_OK) return rc;
@@ -749,6 +961,7 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
                 hs.count = kept;
                 hs.overflow = 0;
                 HIP_TRY(hipMemcpyAsync(b.state, &hs, sizeof hs, hipMemcpyHostToDevice, p->stream));
+                if ((rc = second_list()) != GEPI_OK) return rc;
                 launch_select(p, b, b.cand[cur], (uint32_t)k, kept);
                 k_compact<<<4096, 256, 0, p->stream>>>(b.cand[cur], b.state, b.cand[cur ^ 1],
                                                        t0, t1, tv, fp4 ? (int32_t)n_a4 : 0);
@@ -768,6 +981,7 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
             if (wg_select(path, hs.count)) {
                 k_topk_one<<<1, TOPK_THREADS, 0, p->stream>>>(topk_desc(b, cur, cap, k, par, 0, 0, n_a4));
             } else {
+                if ((rc = second_list()) != GEPI_OK) return rc;
                 launch_select(p, b, b.cand[cur], (uint32_t)k, hs.count);
                 k_compact<<<4096, 256, 0, p->stream>>>(b.cand[cur], b.state, b.cand[cur ^ 1],
                                                        0, 0, tv, fp4 ? (int32_t)n_a4 : 0);
@@ -810,15 +1024,19 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
     }
     /* final extraction: exactly k records, sorted by key on the host */
     auto ts = std::chrono::steady_clock::now();
-    std::vector<Cand> host((size_t)count);
-    if (count > 0)
-        HIP_TRY(hipMemcpyAsync(host.data(), b.cand[cur], sizeof(Cand) * count,
-                               hipMemcpyDeviceToHost, p->stream));
-    HIP_TRY(hipStreamSynchronize(p->stream));
+    if (!finished) {
+        host.resize((size_t)count);
+        if (count > 0)
+            HIP_TRY(hipMemcpyAsync(host.data(), b.cand[cur], sizeof(Cand) * count,
+                                   hipMemcpyDeviceToHost, p->stream));
+        HIP_TRY(hipStreamSynchronize(p->stream));
+    }
     const int64_t n = candidates_to_results(host, k, tops);
     *n_tops = n;
     ms_top += ms_since(ts);
     st_local.ms_count_kernels = ms_count;
+    if (finished) /* enqueued together with the rest: what is not the others' */
+        ms_top = ms_since(t_start) - ms_count - st_local.ms_prepare;
     st_local.ms_select = ms_top;
     st_local.exact_evals = (int64_t)exact_total;
     st_local.bands = bands;

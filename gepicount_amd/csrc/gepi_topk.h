@@ -217,26 +217,30 @@ static __global__ void __launch_bounds__(256) k_compact(const Cand *__restrict__
     }
 }
 
-/* Threshold score and filter coefficient of a selected key. */
+/* Filter coefficients of an admission threshold (entropy; 0 for Fisher,
+ * whose bound is made per variant pair): expm1(T) and T in nats, T = -thr ln
+ * 2, both rounded down.                                                   */
+__host__ __device__ inline void threshold_coeffs(double thr, int32_t ffun, float &kf, float &kt) {
+    kf = kt = 0.0f;
+    if (ffun != GEPI_FFUNC_ENTROPY) return;
+    const double it = -thr - 1e-12;
+    if (it > 0.0) {
+        const double k = expm1(it * 0.6931471805599453) * (1.0 - 1e-6);
+        kf = (float)k;
+        if ((double)kf > k) kf = nextafterf(kf, 0.0f);
+        const double t = it * 0.6931471805599453 * (1.0 - 1e-6);
+        kt = (float)t;
+        if ((double)kt > t) kt = nextafterf(kt, 0.0f);
+    }
+}
+
+/* Threshold score and filter coefficients of a selected key. */
 __device__ __forceinline__ void adopt_threshold(ScanState *st, uint64_t key_hi, uint64_t key_lo,
                                                 int32_t ffun) {
     const double thr = from_order_bits(key_hi);
     st->thr_score = thr;
     st->thr_idx = key_lo;
-    float kf = 0.0f, kt = 0.0f;
-    if (ffun == GEPI_FFUNC_ENTROPY) {
-        double it = -thr - 1e-12;
-        if (it > 0.0) {
-            double k = expm1(it * 0.6931471805599453) * (1.0 - 1e-6);
-            kf = (float)k;
-            if ((double)kf > k) kf = nextafterf(kf, 0.0f);
-            const double t = it * 0.6931471805599453 * (1.0 - 1e-6);
-            kt = (float)t;
-            if ((double)kt > t) kt = nextafterf(kt, 0.0f);
-        }
-    }
-    st->filt_k = kf;
-    st->filt_t = kt;
+    threshold_coeffs(thr, ffun, st->filt_k, st->filt_t);
 }
 
 /* After a compaction: adopt the compacted buffer and the new threshold. */
@@ -259,6 +263,21 @@ static __global__ void k_sel_reset(ScanState *st, uint32_t rank) {
     st->done = 0;
     st->gather_n = 0;
     for (int i = 0; i < 256; i++) st->hist[i] = 0;
+}
+
+/* A scan's state before its first band: nothing pending, no candidates, an
+ * admission threshold (+infinity admits everything) and its coefficients.
+ * As a kernel, so that no host copy stands before the first launch.        */
+static __global__ void k_state_init(ScanState *st, double thr, float kf, float kt) {
+    uint32_t *w = reinterpret_cast<uint32_t *>(st);
+    for (uint32_t i = threadIdx.x; i < sizeof(ScanState) / 4; i += blockDim.x) w[i] = 0;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        st->thr_score = thr;
+        st->thr_idx = ~0ull;
+        st->filt_k = kf;
+        st->filt_t = kt;
+    }
 }
 
 struct ItemReport {
@@ -287,39 +306,38 @@ __device__ __forceinline__ bool key_le(uint64_t ah, uint64_t al, uint64_t bh, ui
     return ah < bh || (ah == bh && al <= bl);
 }
 
-/* Block-wide exclusive prefix of one flag per thread (1024 threads). */
-__device__ __forceinline__ uint32_t block_prefix(bool flag, uint32_t *wsum, uint32_t &total) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const uint64_t b = __ballot(flag);
-    const uint32_t below = (uint32_t)__popcll(b & ((1ull << lane) - 1ull));
-    if (lane == 0) wsum[wave] = (uint32_t)__popcll(b);
-    __syncthreads();
-    uint32_t before = 0, all = 0;
-    for (int w = 0; w < TOPK_THREADS / 64; w++) {
-        const uint32_t c = wsum[w];
-        before += w < wave ? c : 0u;
-        all += c;
-    }
-    total = all;
-    return before + below;
+/* The radix select of one workgroup takes 12-bit digits: five of the key's
+ * high word and its last 4 bits, then the same of the low word.  The first
+ * digit is the score's sign and exponent, the second splits what shares it
+ * 4,096 ways, so two passes over the candidates usually leave a few keys. */
+constexpr int TOPK_BINS = 4096;
+__device__ __forceinline__ uint32_t digit_bits(uint32_t b) { return b % 64 == 60 ? 4u : 12u; }
+__device__ __forceinline__ uint32_t wide_digit(uint64_t hi, uint64_t lo, uint32_t b) {
+    const uint64_t w = b < 64 ? hi : lo;
+    return (uint32_t)(w >> (64 - b % 64 - digit_bits(b))) & ((1u << digit_bits(b)) - 1u);
 }
 
 /* Top-k maintenance of one scan by one 1024-thread workgroup: after a
  * candidate overflow, the k-th key among the records kept becomes the
  * threshold and the band's records (fp4 tile numbering) are dropped (the
  * band is redone); otherwise, with more than k candidates, exactly the k
- * smallest keys are kept, compacted in place.  Resets the pending list for
- * the next round; writes a report when d.report is set.                    */
+ * smallest keys are kept, compacted in place (in no order).  Resets the
+ * pending list for the next round; writes a report when d.report is set.
+ *
+ * One CU, so its latencies are what it costs: per pass the bins are summed
+ * by all threads (one thread reading 256 bins in turn took 7 us), the last
+ * few keys are ranked by counting instead of a 55-step sort, and the
+ * compaction moves 4,096 records between two barriers.                     */
 __device__ __forceinline__ void topk_wg_body(const TopkDesc &d) {
     ScanState *st = d.st;
     if (st == nullptr) return; /* empty descriptor slot (the whole workgroup) */
-    __shared__ uint32_t hist[256];
+    __shared__ uint32_t hist[TOPK_BINS];
     __shared__ uint64_t kh[SEL_SMALL], kl[SEL_SMALL];
     __shared__ uint32_t wsum[TOPK_THREADS / 64];
     __shared__ uint64_t s_hi, s_lo;
-    __shared__ uint32_t s_bits, s_rank, s_done, s_gather;
-    __shared__ unsigned long long s_wptr;
+    __shared__ uint32_t s_bits, s_rank, s_done, s_gather, s_wptr;
     const int t = threadIdx.x;
+    const int lane = t & 63, wave = t >> 6;
 
     const unsigned long long raw = st->count;
     const uint32_t pend_ovf = st->pend_overflow, cand_ovf = st->overflow;
@@ -335,44 +353,69 @@ __device__ __forceinline__ void topk_wg_body(const TopkDesc &d) {
             s_rank = d.k;
             s_done = 0;
         }
-        /* radix select of the k-th smallest key, 8-bit digits MSB first */
+        /* radix select of the k-th smallest key, digits MSB first */
         while (true) {
-            if (t < 256) hist[t] = 0;
+            for (int i = t; i < TOPK_BINS; i += TOPK_THREADS) hist[i] = 0;
             __syncthreads();
             SelPrefix pre;
             pre.key_hi = s_hi;
             pre.key_lo = s_lo;
             pre.bits_done = s_bits;
+            const uint32_t rank = s_rank;
+#pragma unroll 4
             for (unsigned long long i = t; i < n; i += TOPK_THREADS) {
                 const uint64_t h = order_bits(d.cand[i].score), l = d.cand[i].idx;
-                if (key_match(h, l, pre)) atomicAdd(&hist[key_digit(h, l, pre.bits_done)], 1u);
+                if (key_match(h, l, pre)) atomicAdd(&hist[wide_digit(h, l, pre.bits_done)], 1u);
             }
             __syncthreads();
-            if (t == 0) {
-                uint32_t cum = 0, dg = 0;
-                for (dg = 0; dg < 255; dg++) {
-                    if (cum + hist[dg] >= s_rank) break;
-                    cum += hist[dg];
-                }
-                const uint32_t b = s_bits;
+            /* thread t sums bins 4t .. 4t + 3; the one whose range holds the
+             * rank picks the digit */
+            uint32_t b4[4], own = 0;
+#pragma unroll
+            for (int i = 0; i < 4; i++) own += b4[i] = hist[4 * t + i];
+            uint32_t inc = own; /* inclusive sum over the wave's lanes */
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) {
+                const uint32_t v = __shfl_up(inc, off);
+                inc += lane >= off ? v : 0u;
+            }
+            if (lane == 63) wsum[wave] = inc;
+            __syncthreads();
+            uint32_t before = inc - own;
+#pragma unroll
+            for (int w = 0; w < TOPK_THREADS / 64; w++) before += w < wave ? wsum[w] : 0u;
+            if (before < rank && before + own >= rank) {
+                uint32_t cum = before, dg = 0, c = b4[0];
+#pragma unroll
+                for (int i = 0; i < 3; i++)
+                    if (dg == (uint32_t)i && cum + c < rank) {
+                        cum += c;
+                        dg = i + 1;
+                        c = b4[i + 1];
+                    }
+                const uint32_t b = pre.bits_done, nb = digit_bits(b);
+                const uint64_t v = (uint64_t)(4 * t + dg) << (64 - b % 64 - nb);
                 if (b < 64)
-                    s_hi |= (uint64_t)dg << (56 - b);
+                    s_hi |= v;
                 else
-                    s_lo |= (uint64_t)dg << (120 - b);
-                s_rank -= cum;
-                s_bits = b + 8;
-                s_done = s_bits == 128 ? 1u : (hist[dg] <= (uint32_t)SEL_SMALL ? 2u : 0u);
+                    s_lo |= v;
+                s_rank = rank - cum;
+                s_bits = b + nb;
+                s_done = b + nb == 128 ? 1u : (c <= (uint32_t)SEL_SMALL ? 2u : 0u);
                 s_gather = 0;
             }
             __syncthreads();
             if (s_done) break;
         }
         if (s_done == 2) {
-            /* the remaining matching keys fit in LDS: gather and sort them */
+            /* the remaining matching keys fit in LDS: each is ranked by
+             * counting the smaller ones (keys are distinct) */
             SelPrefix pre;
             pre.key_hi = s_hi;
             pre.key_lo = s_lo;
             pre.bits_done = s_bits;
+            const uint32_t rank = s_rank;
+#pragma unroll 4
             for (unsigned long long i = t; i < n; i += TOPK_THREADS) {
                 const uint64_t h = order_bits(d.cand[i].score), l = d.cand[i].idx;
                 if (key_match(h, l, pre)) {
@@ -385,31 +428,15 @@ __device__ __forceinline__ void topk_wg_body(const TopkDesc &d) {
             }
             __syncthreads();
             const uint32_t g = s_gather < (uint32_t)SEL_SMALL ? s_gather : (uint32_t)SEL_SMALL;
-            if (t >= (int)g) {
-                kh[t] = ~0ull;
-                kl[t] = ~0ull;
-            }
-            __syncthreads();
-            for (int size = 2; size <= SEL_SMALL; size <<= 1) {
-                for (int stride = size >> 1; stride > 0; stride >>= 1) {
-                    const int partner = t ^ stride;
-                    if (partner > t) {
-                        const bool up = (t & size) == 0;
-                        const bool gt = kh[t] > kh[partner] || (kh[t] == kh[partner] && kl[t] > kl[partner]);
-                        if (gt == up) {
-                            const uint64_t a = kh[t], b = kl[t];
-                            kh[t] = kh[partner];
-                            kl[t] = kl[partner];
-                            kh[partner] = a;
-                            kl[partner] = b;
-                        }
-                    }
-                    __syncthreads();
+            if ((uint32_t)t < g) {
+                const uint64_t h = kh[t], l = kl[t];
+                uint32_t less = 0;
+                for (uint32_t i = 0; i < g; i++)
+                    less += kh[i] < h || (kh[i] == h && kl[i] < l) ? 1u : 0u;
+                if (less == rank - 1) { /* exactly one thread */
+                    s_hi = h;
+                    s_lo = l;
                 }
-            }
-            if (t == 0) {
-                s_hi = kh[s_rank - 1];
-                s_lo = kl[s_rank - 1];
             }
             __syncthreads();
         }
@@ -417,29 +444,39 @@ __device__ __forceinline__ void topk_wg_body(const TopkDesc &d) {
          * and writes never pass the read position */
         const uint64_t khi = s_hi, klo = s_lo;
         if (t == 0) s_wptr = 0;
-        __syncthreads();
-        for (unsigned long long base = 0; base < n; base += TOPK_THREADS) {
-            const unsigned long long i = base + t;
-            Cand c;
-            bool keep = false;
-            if (i < n) {
-                c = d.cand[i];
-                keep = key_le(order_bits(c.score), c.idx, khi, klo);
-                if (keep && cand_ovf) {
-                    const int64_t a = (int64_t)(c.idx >> 32) >> 1;
-                    const int64_t b = (int64_t)((c.idx >> 3) & 0x1FFFFFFFull) >> 1;
-                    const int64_t tl = tile_index(a, b, TM, d.n_a4);
-                    keep = tl < d.drop_t0 || tl >= d.drop_t1;
-                }
+        constexpr int PER = 4;
+        for (unsigned long long base = 0; base < n; base += PER * TOPK_THREADS) {
+            Cand c[PER];
+            uint32_t keep = 0;
+#pragma unroll
+            for (int j = 0; j < PER; j++) {
+                const unsigned long long i = base + (unsigned)(j * TOPK_THREADS + t);
+                if (i < n) c[j] = d.cand[i];
             }
-            uint32_t total;
-            const uint32_t off = block_prefix(keep, wsum, total);
-            const unsigned long long w0 = s_wptr;
-            __syncthreads();
-            if (keep) d.cand[w0 + off] = c;
-            if (t == 0) s_wptr = w0 + total;
-            __syncthreads();
+#pragma unroll
+            for (int j = 0; j < PER; j++) {
+                const unsigned long long i = base + (unsigned)(j * TOPK_THREADS + t);
+                bool kp = i < n && key_le(order_bits(c[j].score), c[j].idx, khi, klo);
+                if (kp && cand_ovf) {
+                    const int64_t a = (int64_t)(c[j].idx >> 32) >> 1;
+                    const int64_t b = (int64_t)((c[j].idx >> 3) & 0x1FFFFFFFull) >> 1;
+                    const int64_t tl = tile_index(a, b, TM, d.n_a4);
+                    kp = tl < d.drop_t0 || tl >= d.drop_t1;
+                }
+                keep |= kp ? 1u << j : 0u;
+            }
+            __syncthreads(); /* the chunk is read (and s_wptr set) */
+#pragma unroll
+            for (int j = 0; j < PER; j++) {
+                const bool kp = (keep >> j) & 1u;
+                const uint64_t m = __ballot(kp);
+                uint32_t w0 = 0;
+                if (lane == 0 && m) w0 = atomicAdd(&s_wptr, (uint32_t)__popcll(m));
+                w0 = __shfl(w0, 0);
+                if (kp) d.cand[w0 + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = c[j];
+            }
         }
+        __syncthreads();
         if (t == 0) {
             st->count = s_wptr;
             st->count2 = 0;
