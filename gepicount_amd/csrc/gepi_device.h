@@ -274,8 +274,8 @@ struct FilterConsts {
     float kf;     /* entropy: chi-square coefficient, 0 = admit everything      */
     float k0, k1; /* entropy: another, k0 + k1 min(y, z); the larger one counts */
     float h0, h1; /* Fisher: the same per nat                                   */
-    float a_s;    /* Fisher: -(thr + 1e-6) ln 10 - ln(4 n0 n1) / 2 + 0.9189,
-                   * less a float error margin                                 */
+    float a_s;    /* Fisher: -(thr + 1e-6) ln 10 - ln(2.55 n) / 2, less a
+                   * float error margin                                        */
 };
 
 /* The thresholds through the constant address space: scalar loads from the
@@ -295,8 +295,7 @@ __device__ __forceinline__ FilterConsts filter_consts(const ScanState *st, const
     fc.k1 = c->filt_t * g.h1;
     const int32_t n0 = g.n0, n1 = g.n1;
     const double a = -(fc.thr_s + 1e-6) * 2.302585092994046;
-    const double A = a - 0.5 * log(4.0 * (double)(n0 > 1 ? n0 : 1) * (double)(n1 > 1 ? n1 : 1)) +
-                     0.9189;
+    const double A = a - 0.5 * log(2.55 * (double)(n0 + n1 > 1 ? n0 + n1 : 1));
     /* the float roundings of A and of the per-pair arithmetic stay far
      * under this margin, which keeps the derived bound conservative        */
     fc.a_s = fc.thr_s < 0.0 ? (float)(A - (fabs(A) + fabs(a) + 10.0) * 1e-6) : 0.0f;
@@ -378,12 +377,19 @@ __device__ __forceinline__ void push_mask(const CountArgs &g, PendStage &ps, con
  * ms, Fisher 7.47 -> 5.99; large scan 120.4 -> 116.6).
  * Entropy: -I_bits <= thr needs T = -thr * ln 2 (kf = 2^-thr - 1 and T made
  * where the threshold is updated, rounded down).
- * Fisher: p >= P(obs) = C(y,w) C(z,x) / C(m,xx); e^{nH(k/n)} / sqrt(2n) <=
- * C(n,k) for the numerator and C(m,xx) <= e^{mH} sqrt(m / (2 pi xx (m-xx)))
- * (1 <= xx <= m-1; H in nats) give P(obs) >= e^{-mI} sqrt(2 pi (m-1) / m) /
- * (2 sqrt(yz)), so log10 P(obs) - 1e-6 <= thr needs
- *     T = (-(thr + 1e-6) ln 10 - ln(4yz) / 2 + 0.9189 - 1/m) / m
- * (y, z clamped to >= 1; ln(2 pi (m-1)/m) / 2 >= 0.9189 - 1/m);
+ * Fisher: p >= P(obs) = C(y,w) C(z,x) / C(m,xx).  For 1 <= k <= n-1
+ *     sqrt(n / (8 k (n-k))) <= C(n,k) e^{-nH(k/n)} <= sqrt(n / (2 pi k (n-k)))
+ * (H in nats), and C(n,0) = C(n,n) = 1 meets the left side as 1.  With X =
+ * min(xx, m-xx) <= m/2 (a table and its complement have the same P and I):
+ * w(y-w)/y <= w, x(z-x)/z <= x, w x <= X^2/4 and X(m-X)/m >= X/2, so
+ * P(obs) >= e^{-mI} sqrt(2 pi (X/2) / (64 X^2/4)) = e^{-mI} / sqrt(5.1 X) >=
+ * e^{-mI} / sqrt(2.55 m); with w or x at an end of its range P(obs) >=
+ * e^{-mI} sqrt(pi/8), which is no less for m >= 1.  So log10 P(obs) - 1e-6 <=
+ * thr needs
+ *     T = (-(thr + 1e-6) ln 10 - ln(2.55 m) / 2) / m
+ * (taken at ln(2.55 n) >= ln(2.55 m), one log per workgroup; bounding the
+ * numerator and the denominator each by its own worst case cost ln(4yz)/2 -
+ * 0.92, 2.4 nats more at 2,048 samples and 3 at 8,192);
  * its survivors are then checked exactly against the log-factorial table.
  * The test is s = fd^2 - RN(K*y*z*(1 - 2^-16) * q) > bias with fd = float(D)
  * squared exactly inside one fma.  fd is D exactly when |D| <= 2^24 (always
@@ -521,13 +527,10 @@ __device__ __forceinline__ void filter_pair(const CountArgs &g, PendStage &ps, c
     if (FFUN == GEPI_FFUNC_FISHERPV) {
         K = 0.0f;
         if (fc.thr_s < 0.0) {
-            /* T = (a - ln(4yz)/2 + 0.9189 - 1/m) / m at ln(4yz) <= ln(4 n0 n1)
-             * (a_s; y <= n0, z <= n1), and K = T (1 + T/2) <= expm1(T) or
-             * T (h0 + h1 min(y, z)) <= T/g(p): both only lower K; 0.9189 - 1/m <= ln(2 pi (m-1)/m) / 2 comes from
-             * C(m, xx) <= e^{m H} sqrt(m / (2 pi xx (m - xx))), 1 <= xx <= m-1
-             * (the other tables have P(obs) = 1 and D = 0) */
+            /* T = a_s / m, and K = T (1 + T/2) <= expm1(T) or T (h0 + h1
+             * min(y, z)) <= T/g(p): both only lower K                      */
             const float r = __builtin_amdgcn_rcpf(m > 1 ? mf : 1.0f);
-            const float T = (fc.a_s - r) * r;
+            const float T = fc.a_s * r;
             if (T > 0.0f)
                 K = T * fmaxf(1.0f + 0.5f * T, __builtin_fmaf(fc.h1, mn, fc.h0)) * (1.0f - 2e-5f);
         }

@@ -10,7 +10,7 @@ import math
 import numpy as np
 import pytest
 
-from test_filter_bounds import all_small_tables, chi2_over_m, mi_nats, tables
+from test_filter_bounds import H, all_small_tables, chi2_over_m, lchoose, mi_nats, tables
 
 
 def g(p):
@@ -47,3 +47,21 @@ def test_tangent_below_inverse(n0, n1):
                 continue
             k = np.float32(h0 + np.float32(h1 * np.float32(min(y, z))))
             assert float(k) <= 1.0 / g(min(y, z) / (y + z)), (n0, n1, y, z)
+
+
+def ln_p_obs(w, x, y, z):
+    return lchoose(y, w) + lchoose(z, x) - lchoose(y + z, w + x)
+
+
+def test_fisher_probability_above_bound():
+    """ln P(obs) >= -m I - ln(2.55 m) / 2, and its binomial lower bound."""
+    rng = np.random.default_rng(12)
+    for w, x, y, z in list(all_small_tables(14)) + list(tables(rng, 20000, 5000)):
+        m = y + z
+        lp = ln_p_obs(w, x, y, z)
+        assert lp >= -m * mi_nats(w, x, y, z) - 0.5 * math.log(2.55 * m) - 1e-9 * max(1.0, -lp), (w, x, y, z)
+    for n in list(range(2, 200)) + [1000, 4097, 46340]:
+        for k in range(1, n) if n < 200 else np.linspace(1, n - 1, 97).astype(int):
+            k = int(k)
+            lb = n * H(k / n) + 0.5 * math.log(n / (8.0 * k * (n - k)))
+            assert lchoose(n, k) >= lb - 1e-9 * max(1.0, lb), (n, k)
