@@ -934,6 +934,12 @@ constexpr uint32_t F4W_PAIR_CAP = 1024;
  * at 20,000 variants, 0.99-1.09x its time up to 1,024 samples, 0.88-0.96x
  * from 1,536 on. */
 constexpr int32_t F4W_MIN_KSTEPS = 10;
+/* ... and, on genotype planes, for scans of at least this many 64 x 32 tiles
+ * (about 2,900 variants) whatever their samples: against the LDS-staged
+ * kernel, whole scans of 64-1,100 samples took 0.71-0.84x the time on 20,000
+ * variants (Fisher 0.72-0.80x), 0.81-0.95x (0.91-0.98x) on 4,000 and 0.95-1.09x
+ * (1.20-1.33x) on 1,000, where one wave of workgroups is all there is.     */
+constexpr int64_t F4G_MIN_TILES = 2048;
 /* Entropy scans on wave tiles park flagged pairs from this many K steps of
  * 128 samples (Fisher scans always do).  Measured, entropy top-100 at 20,000
  * variants and top-1,000 at 40,000: parking took 1.13-1.38x the time at 24-40
@@ -998,27 +1004,19 @@ struct F4WShared {
     uint32_t n_park, park_slot;
 };
 
-template <int FFUN, bool F32, bool PARK>
-__device__ __forceinline__ void count_f4w_unit(const CountArgs &g, int64_t unit, F4WShared &sh) {
-    PendStage &stage = sh.stage;
-    stage_init(stage);
-    if (PARK && threadIdx.x == 0) {
-        sh.n_park = 0;
-        sh.park_slot = g.park ? park_claim(g.park_busy, g.park_slots) : PARK_NONE;
-    }
+/* The nine products of a 32 x 32-variant wave tile (groups gA, gB of the
+ * grouped layout) over both classes: acc[p][q] ends at start plus the totals,
+ * and the class-0 counts (below 2^16) of elements e and e + 1 go to dword
+ * (e / 2 * 9 + 3p + q) * 64 of the lane's LDS column P.  start: 0, or a
+ * fraction that no count rounds away (see count_f4g_unit).                */
+__device__ __forceinline__ void f4w_products(const CountArgs &g, int32_t gA, int32_t gB, bool live,
+                                             float start, uint32_t *P, v16f (&acc)[3][3]) {
     const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int64_t tile = g.tile_begin + 2 * unit + (wave >> 1);
-    const bool live = tile < g.tile_begin + g.n_tiles;
-    int32_t ta = 0, tb = 0;
-    if (live) tile_of_f4(tile, g.n_var_pad / TM, ta, tb);
-    const int32_t gA = 2 * ta + (wave & 1), gB = tb;
     const int32_t u1 = f4_super3(g.ks0), n_u = u1 + f4_super3(g.n_ks - g.ks0);
     const int32_t last = n_u > 0 ? n_u - 1 : 0; /* n_u == 0: super-step 0 exists */
     const char *lay = reinterpret_cast<const char *>(g.planes_k);
     const int64_t ustride = (int64_t)g.n_var_pad * 192; /* bytes per super-step */
     const int loff = (lane >> 5) * 512 + (lane & 31) * 16;
-    uint32_t *P = sh.c0lds[wave] + lane; /* dword d of this lane at P[64 d] */
 
     /* c[cp][p]: A plane p, column h + 2cp; c[cp][3 + q]: B plane q */
     uint4 c[2][6];
@@ -1035,13 +1033,12 @@ __device__ __forceinline__ void count_f4w_unit(const CountArgs &g, int64_t unit,
                 as_u4(__builtin_amdgcn_raw_buffer_load_b128(rb, loff + p * 2048 + cp * 1024, 0, 0));
         }
     };
-    v16f acc[3][3];
 #pragma unroll
     for (int p = 0; p < 3; p++)
 #pragma unroll
         for (int q = 0; q < 3; q++)
 #pragma unroll
-            for (int e = 0; e < 16; e++) acc[p][q][e] = 0.0f;
+            for (int e = 0; e < 16; e++) acc[p][q][e] = start;
     /* One super-step: per column pair three chunks of 9 MFMAs; the pair's six
      * registers are reloaded as soon as the last chunk's fragments are made,
      * so a load has that chunk and the other pair's three, 36 MFMAs (about
@@ -1102,12 +1099,32 @@ __device__ __forceinline__ void count_f4w_unit(const CountArgs &g, int64_t unit,
                 for (int q = 0; q < 3; q++)
 #pragma unroll
                     for (int e = 0; e < 16; e += 2)
-                        P[((p * 3 + q) * 8 + e / 2) * 64] =
+                        P[(e / 2 * 9 + p * 3 + q) * 64] =
                             (uint32_t)acc[p][q][e] | ((uint32_t)acc[p][q][e + 1] << 16);
         }
         u_end = nu_live;
     }
+}
 
+template <int FFUN, bool F32, bool PARK>
+__device__ __forceinline__ void count_f4w_unit(const CountArgs &g, int64_t unit, F4WShared &sh) {
+    PendStage &stage = sh.stage;
+    stage_init(stage);
+    if (PARK && threadIdx.x == 0) {
+        sh.n_park = 0;
+        sh.park_slot = g.park ? park_claim(g.park_busy, g.park_slots) : PARK_NONE;
+    }
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int64_t tile = g.tile_begin + 2 * unit + (wave >> 1);
+    const bool live = tile < g.tile_begin + g.n_tiles;
+    int32_t ta = 0, tb = 0;
+    if (live) tile_of_f4(tile, g.n_var_pad / TM, ta, tb);
+    const int32_t gA = 2 * ta + (wave & 1), gB = tb;
+    uint32_t *P = sh.c0lds[wave] + lane; /* dword d of this lane at P[64 d] */
+
+    v16f acc[3][3];
+    f4w_products(g, gA, gB, live, 0.0f, P, acc);
     const FilterConsts fc = filter_consts(g.st, g);
     __syncthreads(); /* the stage counter is cleared, the park region claimed */
     const bool parks = PARK && sh.park_slot != PARK_NONE;
@@ -1125,7 +1142,7 @@ __device__ __forceinline__ void count_f4w_unit(const CountArgs &g, int64_t unit,
             for (int p = 0; p < 3; p++)
 #pragma unroll
                 for (int q = 0; q < 3; q++) {
-                    const uint32_t w = P[((p * 3 + q) * 8 + e / 2) * 64];
+                    const uint32_t w = P[(e / 2 * 9 + p * 3 + q) * 64];
                     cn[0][p][q] = (float)((e & 1) ? (w >> 16) : (w & 0xFFFFu));
                     cn[1][p][q] = acc[p][q][e] - cn[0][p][q];
                     tot[p][q] = acc[p][q][e];
@@ -1137,7 +1154,7 @@ __device__ __forceinline__ void count_f4w_unit(const CountArgs &g, int64_t unit,
             for (int p = 0; p < 3; p++)
 #pragma unroll
                 for (int q = 0; q < 3; q++) {
-                    const uint32_t w = P[((p * 3 + q) * 8 + e / 2) * 64];
+                    const uint32_t w = P[(e / 2 * 9 + p * 3 + q) * 64];
                     cn[0][p][q] = (int32_t)((e & 1) ? (w >> 16) : (w & 0xFFFFu));
                     cn[1][p][q] = (int32_t)acc[p][q][e] - cn[0][p][q];
                 }
@@ -1158,6 +1175,219 @@ __device__ __forceinline__ void count_f4w_unit(const CountArgs &g, int64_t unit,
         if (threadIdx.x == 0 && parks) atomicExch(&g.park_busy[sh.park_slot], 0u);
     }
     stage_flush(g, stage);
+}
+
+/* ---- wave tiles on genotype planes --------------------------------------
+ * The same wave tiles with a variant's planes as its three genotypes
+ * (homozygous 1, heterozygous, homozygous 2: disjoint, their union the valid
+ * calls), so that the nine products are the cells of the pair's genotype
+ * table.  Every function of the pair is a union of cells, so no evaluation
+ * has more information than the whole table, and one test of the table (the
+ * screen) stands before the tests of its 20 evaluations.  With c and T a
+ * cell's class-0 and total count, p = n0/n, u = c/T - p:
+ *
+ *   m I9 = sum T KL(c/T || y/m) <= sum T KL(c/T || p)     (y/m minimises it)
+ *   KL(p + u || p) <= u^2 / (2 p (1-p)) (1 + k |u|),  k = (2 g(s) - 1) / s,
+ *       s = min(p, 1-p), g as in the filter (the largest ratio, at the end
+ *       farther in KL)
+ *
+ * so a pair with an evaluation of at least t nats has
+ *   Q = sum T u^2 (1 + k |u|) >= 2 p (1-p) t m.
+ * Entropy: m >= n (1 - a), a = the two variants' shares of missing calls
+ * (g.miss).  Fisher: t m = a_s (filter_consts).  Near its threshold a table
+ * has small u, where the bound is the information itself, about twice as
+ * near as the single evaluations' chi-square.
+ *
+ * The screen costs about 95 VALU instructions per pair against 200 for the
+ * 20 tests, and passes one pair in 100 to 1,000 once the threshold has
+ * settled (per workgroup at 20,000 x 2,048: products 25.0 ns, screen 7.2, the
+ * collected pairs 6.7; the kernel with the tests in the lanes 42.8).  Those are collected in LDS (their totals; the class-0 counts are
+ * there already) and tested one per thread of the workgroup by the int32
+ * filter, so the expensive code runs on full waves and exists once.
+ * Accumulators start at g.sc_start, the largest fraction no count rounds
+ * away, so that an empty cell divides 0 by it; g.sc_sub takes its effect off
+ * the right side (a cell loses at most 2 (1 + 2k) times it).               */
+constexpr int F4G_LIST = 256;  /* pairs collected per workgroup               */
+constexpr int F4G_STAGE = 112; /* survivors staged per workgroup              */
+struct F4GShared {
+    uint32_t c0lds[4][F4W_PARK * 64];
+    uint32_t list[F4G_LIST * 5]; /* 9 totals of 16 bits, then wave, lane, e   */
+    PendStageN<F4G_STAGE> stage;
+    uint32_t n;
+};
+static_assert(sizeof(F4GShared) <= 81920, "two workgroups per CU");
+
+/* (float) of the low (H = 0) or high half of w in one instruction. */
+template <int H>
+__device__ __forceinline__ float half_to_float(uint32_t w) {
+    float f;
+    if (H == 0)
+        asm("v_cvt_f32_u32_sdwa %0, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:WORD_0"
+            : "=v"(f) : "v"(w));
+    else
+        asm("v_cvt_f32_u32_sdwa %0, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:WORD_1"
+            : "=v"(f) : "v"(w));
+    return f;
+}
+
+/* q + T u^2 (1 + k |u|), T u = c - p T = e. */
+__device__ __forceinline__ float screen_cell(float T, float c, float np, float k, float q) {
+    const float e = __builtin_fmaf(np, T, c);
+    const float u = e * __builtin_amdgcn_rcpf(T);
+    return __builtin_fmaf(e * u, __builtin_fmaf(k, __builtin_fabsf(u), 1.0f), q);
+}
+
+/* A pair's record: its totals and where its class-0 counts are. */
+__device__ __forceinline__ void f4g_append(uint32_t *L, const float (&T)[9], uint32_t id) {
+    uint32_t u[9];
+#pragma unroll
+    for (int i = 0; i < 9; i++) u[i] = (uint32_t)T[i];
+#pragma unroll
+    for (int i = 0; i < 4; i++) L[i] = u[2 * i] | (u[2 * i + 1] << 16);
+    L[4] = u[8] | (id << 16);
+}
+
+/* Tests a collected pair with the int32 filter.  unit: the workgroup's. */
+template <int FFUN>
+__device__ __forceinline__ void f4g_test(const CountArgs &g, F4GShared &sh, const FilterConsts &fc,
+                                         const uint32_t *L, int64_t unit) {
+    uint32_t r[5];
+#pragma unroll
+    for (int i = 0; i < 5; i++) r[i] = L[i];
+    const uint32_t id = r[4] >> 16, e = id & 15u, src = (id >> 4) & 63u, wv = id >> 10;
+    const uint16_t *c0 = reinterpret_cast<const uint16_t *>(sh.c0lds[wv]) + (e >> 1) * (9 * 128) +
+                         src * 2 + (e & 1);
+    int32_t x[2][3][3]; /* cells by class */
+#pragma unroll
+    for (int i = 0; i < 9; i++) {
+        const int32_t t = (int32_t)((r[i >> 1] >> (16 * (i & 1))) & 0xFFFFu);
+        x[0][i / 3][i % 3] = c0[i * 128];
+        x[1][i / 3][i % 3] = t - x[0][i / 3][i % 3];
+    }
+    int32_t c[2][3][3]; /* products of the allele and valid planes */
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        int32_t u[3][3];
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            u[i][0] = x[k][i][0] + x[k][i][1];
+            u[i][1] = x[k][i][1] + x[k][i][2];
+            u[i][2] = u[i][0] + x[k][i][2];
+        }
+#pragma unroll
+        for (int q = 0; q < 3; q++) {
+            c[k][0][q] = u[0][q] + u[1][q];
+            c[k][1][q] = u[1][q] + u[2][q];
+            c[k][2][q] = c[k][0][q] + u[2][q];
+        }
+    }
+    int32_t ta, tb;
+    tile_of_f4(g.tile_begin + 2 * unit + (wv >> 1), g.n_var_pad / TM, ta, tb);
+    const int32_t A = (2 * ta + (int32_t)(wv & 1u)) * 32 + 4 * (int32_t)(src >> 5) +
+                      8 * (int32_t)(e >> 2) + (int32_t)(e & 3u);
+    const int32_t B = tb * 32 + (int32_t)(src & 31u);
+    filter_pair<FFUN, true>(g, sh.stage, fc, A, B, c);
+}
+
+template <int FFUN>
+__device__ __forceinline__ void count_f4g_unit(const CountArgs &g, int64_t unit, F4GShared &sh) {
+    stage_init(sh.stage);
+    if (threadIdx.x == 0) sh.n = 0;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int64_t tile = g.tile_begin + 2 * unit + (wave >> 1);
+    const bool live = tile < g.tile_begin + g.n_tiles;
+    int32_t ta = 0, tb = 0;
+    if (live) tile_of_f4(tile, g.n_var_pad / TM, ta, tb);
+    const int32_t gA = 2 * ta + (wave & 1), gB = tb;
+    uint32_t *P = sh.c0lds[wave] + lane;
+    v16f acc[3][3];
+    f4w_products(g, gA, gB, live, g.sc_start, P, acc);
+
+    const FilterConsts fc = filter_consts(g.st, g);
+    /* the right side is R (1 - a) - sc_sub, or negative: every pair passes */
+    float R;
+    if (FFUN == GEPI_FFUNC_ENTROPY)
+        R = fc.kt * g.sc_m;
+    else
+        R = fc.thr_s < 0.0 && fc.a_s > 0.0f ? fc.a_s * g.sc_q : 0.0f;
+    const int32_t B = gB * 32 + (lane & 31);
+    const int32_t Ab = gA * 32 + 4 * (lane >> 5);
+    const float RA = FFUN == GEPI_FFUNC_ENTROPY ? R : 0.0f;
+    const float rB = __builtin_fmaf(-RA, g.miss[B], R - g.sc_sub), np = -g.sc_p, kk = g.sc_k;
+    __syncthreads(); /* the counters are cleared */
+    uint32_t pend = 0; /* elements that found the list full */
+    auto in_scan = [&](int e) {
+        const int32_t A = Ab + 8 * (e >> 2) + (e & 3);
+        return live && A < g.n_var && B <= A;
+    };
+    /* the lanes of fl append their element e; true for those without room.
+     * Every lane of the wave calls it: lane 0 reserves the places            */
+    auto collect = [&](bool fl, const float (&T)[9], int e) {
+        const uint64_t m = __ballot(fl);
+        uint32_t at = 0;
+        if (lane == 0) at = atomicAdd(&sh.n, (uint32_t)__popcll(m));
+        at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at) +
+             __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+        const bool room = at < (uint32_t)F4G_LIST;
+        if (fl && room) f4g_append(sh.list + at * 5, T, (uint32_t)(wave << 10 | lane << 4 | e));
+        return fl && !room;
+    };
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        uint32_t w[9];
+#pragma unroll
+        for (int i = 0; i < 9; i++) w[i] = P[(j * 9 + i) * 64];
+        float4 mA = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (FFUN == GEPI_FFUNC_ENTROPY) mA = *reinterpret_cast<const float4 *>(g.miss + Ab + 8 * (j >> 1));
+#pragma unroll
+        for (int hf = 0; hf < 2; hf++) {
+            const int e = 2 * j + hf;
+            float T[9], q = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 9; i++) {
+                T[i] = acc[i / 3][i % 3][e];
+                q = screen_cell(T[i], hf == 0 ? half_to_float<0>(w[i]) : half_to_float<1>(w[i]), np, kk, q);
+            }
+            const float mAe = (e & 3) == 0 ? mA.x : (e & 3) == 1 ? mA.y : (e & 3) == 2 ? mA.z : mA.w;
+            bool fl = q > __builtin_fmaf(-RA, mAe, rB);
+            if (__ballot(fl)) {
+                fl = fl && in_scan(e);
+                if (__ballot(fl)) pend |= collect(fl, T, e) ? 1u << e : 0u;
+            }
+        }
+    }
+    __syncthreads(); /* the list and every wave's class-0 counts are written */
+    while (true) {
+        const uint32_t n = sh.n < (uint32_t)F4G_LIST ? sh.n : (uint32_t)F4G_LIST;
+        for (uint32_t i = threadIdx.x; i < n; i += F4W_THREADS)
+            f4g_test<FFUN>(g, sh, fc, sh.list + i * 5, unit);
+        if (!__syncthreads_or(pend != 0)) break;
+        /* the list was full (loose thresholds): the next of the elements left
+         * over.  e is uniform here, so the accumulators are read by register
+         * index                                                           */
+        if (threadIdx.x == 0) sh.n = 0;
+        __syncthreads();
+#pragma unroll 1
+        for (int e = 0; e < 16; e++) {
+            const bool fl = (pend >> e) & 1u;
+            if (!__ballot(fl)) continue;
+            float T[9];
+#pragma unroll
+            for (int i = 0; i < 9; i++) T[i] = acc[i / 3][i % 3][e];
+            const bool left = collect(fl, T, e); /* by every lane: lane 0 reserves */
+            if (!left) pend &= ~(1u << e);
+        }
+        __syncthreads();
+    }
+    stage_flush_after_barrier(g, sh.stage);
+}
+
+template <int FFUN>
+__global__ void __launch_bounds__(F4W_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
+k_count_f4g(CountArgs g) {
+    __shared__ F4GShared sh;
+    count_f4g_unit<FFUN>(g, band_unit((g.n_tiles + 1) >> 1), sh);
 }
 
 template <int FFUN, bool F32, bool PARK>

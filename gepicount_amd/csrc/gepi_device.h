@@ -81,6 +81,11 @@ struct CountArgs {
     int32_t f32;              /* fp4: class sizes for which the filter may work on
                                * the fp32 counts (f32_counts)                    */
     int32_t n0, n1;           /* class sizes (bounds of y and z: Fisher filter)   */
+    /* wave tiles on genotype planes (count_f4g_unit): per variant the share
+     * of missing calls [n_var_pad]; p = n0/n, k, 2 p (1-p), 2 p (1-p) n; the
+     * accumulators' start and what it takes off the screen's right side    */
+    const float *miss;
+    float sc_p, sc_k, sc_q, sc_m, sc_start, sc_sub;
     float h0, h1;             /* chi-square coefficient per nat: h0 + h1 min(y, z)
                                * (chi2_slope)                                     */
     ScanState *st;
@@ -195,12 +200,15 @@ __device__ __forceinline__ int64_t band_tile(int64_t tile_begin, int32_t n_tiles
  * the pending list with one global reservation per workgroup; past
  * PEND_LDS they go to the pending list directly.                          */
 constexpr int PEND_LDS = 256;
-struct PendStage {
-    Pend rec[PEND_LDS];
+template <int N>
+struct PendStageN {
+    static constexpr uint32_t cap = N;
+    Pend rec[N];
     uint32_t n;
     uint32_t pad;
     unsigned long long base;
 };
+typedef PendStageN<PEND_LDS> PendStage;
 
 /* Atomics on the scan state through global-address-space pointers: the
  * state pointer may come from a descriptor in memory, where the compiler
@@ -223,7 +231,8 @@ __device__ __forceinline__ void push_global(const CountArgs &g, const Pend &p) {
         st_or(&g.st->pend_overflow, 1u);
 }
 
-__device__ __forceinline__ void push_pending(const CountArgs &g, PendStage &ps, int32_t w,
+template <class PS>
+__device__ __forceinline__ void push_pending(const CountArgs &g, PS &ps, int32_t w,
                                              int32_t x, int32_t y, int32_t z, uint64_t idx) {
     Pend p;
     p.w = (uint16_t)w;
@@ -232,7 +241,7 @@ __device__ __forceinline__ void push_pending(const CountArgs &g, PendStage &ps, 
     p.z = (uint16_t)z;
     p.idx = idx;
     const uint32_t pos = atomicAdd(&ps.n, 1u);
-    if (pos < (uint32_t)PEND_LDS)
+    if (pos < PS::cap)
         ps.rec[pos] = p;
     else
         push_global(g, p);
@@ -240,15 +249,17 @@ __device__ __forceinline__ void push_pending(const CountArgs &g, PendStage &ps, 
 
 /* Called by every thread of the workgroup at kernel start (before the first
  * barrier) and after the last push, respectively.                          */
-__device__ __forceinline__ void stage_init(PendStage &ps) {
+template <class PS>
+__device__ __forceinline__ void stage_init(PS &ps) {
     if (threadIdx.x == 0) ps.n = 0;
 }
 
 /* The flush proper: every push is complete (the caller has passed a
  * barrier after the last push).                                           */
-__device__ __forceinline__ void stage_flush_after_barrier(const CountArgs &g, PendStage &ps) {
+template <class PS>
+__device__ __forceinline__ void stage_flush_after_barrier(const CountArgs &g, PS &ps) {
     if (threadIdx.x == 0) {
-        const uint32_t n = ps.n < (uint32_t)PEND_LDS ? ps.n : (uint32_t)PEND_LDS;
+        const uint32_t n = ps.n < PS::cap ? ps.n : PS::cap;
         ps.n = n;
         ps.base = n ? st_add(&g.st->pend_count, (unsigned long long)n) : 0ull;
     }
@@ -263,7 +274,8 @@ __device__ __forceinline__ void stage_flush_after_barrier(const CountArgs &g, Pe
     }
 }
 
-__device__ __forceinline__ void stage_flush(const CountArgs &g, PendStage &ps) {
+template <class PS>
+__device__ __forceinline__ void stage_flush(const CountArgs &g, PS &ps) {
     __syncthreads();
     stage_flush_after_barrier(g, ps);
 }
@@ -272,6 +284,7 @@ __device__ __forceinline__ void stage_flush(const CountArgs &g, PendStage &ps) {
 struct FilterConsts {
     double thr_s; /* admission score threshold                                 */
     float kf;     /* entropy: chi-square coefficient, 0 = admit everything      */
+    float kt;     /* entropy: threshold in nats                                */
     float k0, k1; /* entropy: another, k0 + k1 min(y, z); the larger one counts */
     float h0, h1; /* Fisher: the same per nat                                   */
     float a_s;    /* Fisher: -(thr + 1e-6) ln 10 - ln(2.55 n) / 2, less a
@@ -291,6 +304,7 @@ __device__ __forceinline__ FilterConsts filter_consts(const ScanState *st, const
     fc.kf = c->filt_k;
     fc.h0 = g.h0;
     fc.h1 = g.h1;
+    fc.kt = c->filt_t;
     fc.k0 = c->filt_t * g.h0;
     fc.k1 = c->filt_t * g.h1;
     const int32_t n0 = g.n0, n1 = g.n1;
@@ -327,8 +341,8 @@ __device__ __forceinline__ bool fisher_admits(const CountArgs &g, const FilterCo
  * runtime index would place them in scratch memory.  Fisher: the survivors
  * of the chi-square bound are checked against log10 P(obs) <= thr (p >=
  * P(observed table)) with the log-factorial table first.                 */
-template <int FFUN>
-__device__ __forceinline__ void push_mask(const CountArgs &g, PendStage &ps, const FilterConsts &fc,
+template <int FFUN, class PS>
+__device__ __forceinline__ void push_mask(const CountArgs &g, PS &ps, const FilterConsts &fc,
                                           int32_t A, int32_t B, const int32_t (&c)[2][3][3],
                                           uint32_t mask) {
     const int32_t y = c[0][2][2], z = c[1][2][2];
@@ -475,8 +489,8 @@ __device__ __forceinline__ float yz_of(int32_t y, int32_t z) { return (float)__m
 __device__ __forceinline__ float yz_of(float y, float z) { return y * z; }
 
 struct PairList;
-template <int FFUN, bool ROLLED, bool DEFER = false, typename CT, typename PL = PairList>
-__device__ __forceinline__ void filter_pair(const CountArgs &g, PendStage &ps, const FilterConsts &fc,
+template <int FFUN, bool ROLLED, bool DEFER = false, typename CT, typename PL = PairList, class PS>
+__device__ __forceinline__ void filter_pair(const CountArgs &g, PS &ps, const FilterConsts &fc,
                                             int32_t A, int32_t B, const CT (&c)[2][3][3],
                                             PL *pl = nullptr, const CT (*tot)[3] = nullptr,
                                             uint32_t rows_known = 0);
@@ -513,8 +527,8 @@ struct PairListG {
 __device__ __forceinline__ uint32_t park_reserve(PairList *pl) { return atomicAdd(&pl->n, 1u); }
 __device__ __forceinline__ uint32_t park_reserve(PairListG *pl) { return atomicAdd(pl->n, 1u); }
 
-template <int FFUN, bool ROLLED, bool DEFER, typename CT, typename PL>
-__device__ __forceinline__ void filter_pair(const CountArgs &g, PendStage &ps, const FilterConsts &fc,
+template <int FFUN, bool ROLLED, bool DEFER, typename CT, typename PL, class PS>
+__device__ __forceinline__ void filter_pair(const CountArgs &g, PS &ps, const FilterConsts &fc,
                                             int32_t A, int32_t B, const CT (&c)[2][3][3],
                                             PL *pl, const CT (*tot)[3], uint32_t rows_known) {
     /* tot: the products' totals over both classes, c[0] + c[1], when the

@@ -49,6 +49,9 @@ struct gepi_panel {
     int64_t n_var = 0;
     int32_t n_samples = 0;
     int32_t w64 = 0;
+    /* every valid call carries an allele (always so for .bed genotypes), so
+     * that three genotypes describe it (count_f4g_unit)                    */
+    bool three_genotypes = true;
     uint64_t *d_nat = nullptr;
     hipStream_t stream = nullptr;
     /* per-scan workspace, grown on demand and reused */
@@ -121,6 +124,51 @@ inline void chi2_slope(int32_t n0, int32_t n1, float *h0, float *h1) {
     }
     *h0 = (float)(h - d * p - 1e-6);
     *h1 = n > 0 ? (float)(d / n * (1.0 - 1e-6)) : 0.0f;
+}
+
+/* The super-steps of a scan (384 samples of a class each, class 0 first)
+ * in the panel's file order, for k_class_geno.                            */
+inline void build_super_src(const std::vector<gepi::CompressWord> &cw, int32_t w64, int32_t n0,
+                            int32_t n1, std::vector<gepi::SuperSrc> &src) {
+    src.clear();
+    const int32_t nw32 = 2 * w64;
+    for (int c = 0; c < 2; c++) {
+        const int32_t n = c == 0 ? n0 : n1;
+        int32_t j = 0, seen = 0; /* class samples before word j */
+        auto upto = [&](int32_t s) { /* word j holds class sample s */
+            while (j < nw32 && seen + (int32_t)cw[(size_t)c * nw32 + j].cnt <= s)
+                seen += (int32_t)cw[(size_t)c * nw32 + j++].cnt;
+        };
+        for (int32_t s = 0; s < n; s += 384) {
+            gepi::SuperSrc r;
+            r.cls = c;
+            upto(s);
+            r.j0 = j;
+            r.skip = s - seen;
+            upto(std::min(n, s + 384) - 1);
+            r.j1 = j + 1;
+            src.push_back(r);
+        }
+    }
+}
+
+/* The screen's constants of a scan (count_f4g_unit); g.miss is the caller's. */
+inline void screen_consts(int32_t n0, int32_t n1, gepi::CountArgs &g) {
+    const double n = (double)n0 + n1, p = n > 0 ? n0 / n : 0.5, s = std::min(p, 1.0 - p);
+    /* k = (2 g(s) - 1) / s; a class without samples has no information (every
+     * pair passes or none: both are right)                                 */
+    const double k = s > 0.0 ? (2.0 * -std::log1p(-s) * (1.0 - s) / s - 1.0) / s * (1.0 + 1e-6) : 0.0;
+    g.sc_p = (float)p;
+    g.sc_k = (float)k;
+    g.sc_q = (float)(2.0 * p * (1.0 - p) * (1.0 - 1e-4)); /* 1e-4: the roundings */
+    g.sc_m = (float)(2.0 * p * (1.0 - p) * (1.0 - 1e-4) * n);
+    /* counts up to n leave 24 - bits(n) bits for the fraction; at least 2^-12,
+     * below which it no longer matters                                     */
+    int bits = 0;
+    while (bits < 16 && n >= (double)(1 << bits)) bits++;
+    const double start = std::ldexp(1.0, -std::min(24 - bits, 12));
+    g.sc_start = (float)start;
+    g.sc_sub = (float)(18.0 * start * (1.0 + 2.0 * k) + 1e-3);
 }
 
 /* Sorts candidate records by the canonical key and writes the first

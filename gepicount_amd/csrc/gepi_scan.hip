@@ -164,7 +164,6 @@ int panel_alloc(gepi_panel *p, int device, int64_t n_var, int32_t n_samples) {
     HIP_TRY(hipMalloc(&p->d_small, sizeof(uint64_t) * 2 * SEL_SMALL));
     HIP_TRY(hipEventCreate(&p->ev0));
     HIP_TRY(hipEventCreate(&p->ev1));
-    HIP_TRY(hipHostMalloc(&p->mail, sizeof(HostMail), hipHostMallocDefault));
     return GEPI_OK;
 }
 
@@ -380,10 +379,14 @@ double ms_since(std::chrono::steady_clock::time_point t) {
  *
  * Without association 2 m I (I in nats) of a table is close to chi-square
  * with one degree of freedom, and P(p <= a) of a Fisher test is at most a.
- * So the first band admits the quantile where GUESS times k of its
+ * So the first band, a pilot, admits the quantile where GUESS times k of its
  * evaluations are expected: few enough to be cheap, and if the k best are
- * among them (nearly always: the count says so) the threshold was valid.  A
- * scan that ends with fewer than k records is run again without it.
+ * among them (nearly always: the count says so) the threshold was valid.
+ * The others run under the k-th key so far.  A scan that ends with fewer than
+ * k records is run again without the guess.  (Guessing the whole scan's
+ * threshold after the pilot saved 10-15% where it held, but the tail hangs
+ * on the few variants with the largest effects of their own: over seeds the
+ * k-th key had 0.17 to 2 times the expected evaluations beyond it.)
  * Against bands that began with one tile admitting everything and grew
  * fourfold, a host round trip (40 us) and a selection between two: 1,024 x
  * 256 0.73 -> 0.13 ms (5 bands -> 1), 3,001 x 777 Fisher 1.44 -> 0.29, 20,000
@@ -421,11 +424,14 @@ struct BandPlan {
     }
     /* Tiles of the band that follows `done` tiles.  About 250,000 survivors
      * cost what a band's fixed part does (100 us); at least three times what
-     * is done while the list holds them.                                    */
+     * is done while the list holds them, at most that for Fisher and eight
+     * times for entropy (the pairs that pass the screen cost more under an
+     * older threshold).                                                     */
     int64_t next(int64_t done, int64_t left) const {
         const double q = 1.3 * k / ((double)done * evals_tile);
         const double per = factor * evals_tile * pass(q);
-        const double cheap = std::max(250000.0 / per, 3.0 * (double)done);
+        const double cheap = std::min(std::max(250000.0 / per, 3.0 * (double)done),
+                                      (entropy ? 8.0 : 3.0) * (double)done);
         const double tiles = std::min({cheap, most / per, 1048576.0, (double)left});
         /* a remainder below a fifth of the band goes with it */
         if ((double)left < 1.2 * tiles && (double)left * per < most) return left;
@@ -479,14 +485,17 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
     int path = par->count_path;
     /* fp4: wave tiles from F4W_MIN_KSTEPS K steps on (below, a class's
      * padding K steps, multiplied on the 3-step layout, cost more than the
-     * wave tiles save).  Fisher flags about one variant pair in 8; the wave
-     * tiles park those in a global list per workgroup, which the
-     * allocation-free scan has no room for, so there the LDS-staged kernel
-     * (parking in LDS) runs Fisher. */
+     * wave tiles save), and on genotype planes, whose screen spares most of
+     * the filter, for any number of samples from F4G_MIN_TILES tiles on.
+     * Without genotype planes Fisher parks the one pair in 8 that it flags
+     * in a global list per workgroup, which the allocation-free scan has no
+     * room for, so there the LDS-staged kernel (parking in LDS) runs Fisher. */
     if (path == 0) {
         const int32_t ks = (n0 + 127) / 128 + (n1 + 127) / 128;
         const bool fisher = par->ffun != GEPI_FFUNC_ENTROPY;
-        path = ks >= F4W_MIN_KSTEPS && !(fisher && noalloc) ? 3 : 4;
+        const int64_t a4 = (n_var + TM - 1) / TM;
+        const bool wide = p->three_genotypes && !noalloc && a4 * (a4 + 1) >= F4G_MIN_TILES;
+        path = wide || (ks >= F4W_MIN_KSTEPS && !(fisher && noalloc)) ? 3 : 4;
     }
     /* Wave tiles: Fisher scans park flagged variant pairs (its bound flags
      * about one pair in eight), entropy scans from F4W_PARK_MIN_KSTEPS K
@@ -500,8 +509,10 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
      * than 0.02 evaluations per variant pair through); the large scan
      * (65 K steps) 126.0 ms parking and 129.2 ms not.                     */
     const uint32_t park_slots = (uint32_t)(((4 * device_cus(p->device)) + 7) / 8 * 8);
+    /* wave tiles on genotype planes, unless a valid call has no allele */
+    const bool geno = path == 3 && p->three_genotypes;
     const bool f4w_park =
-        path == 3 && !noalloc &&
+        path == 3 && !geno && !noalloc &&
         (par->ffun != GEPI_FFUNC_ENTROPY || (n0 + 127) / 128 + (n1 + 127) / 128 >= F4W_PARK_MIN_KSTEPS);
     const size_t park_rec_bytes = (size_t)park_slots * F4W_PAIR_CAP * sizeof(PairRec);
     const bool fp4 = path == 3 || path == 4;
@@ -553,18 +564,26 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
         int32_t c0n, c1n;
         build_compress_words(mask_ctrl, mask_case, p->n_samples, p->w64, cw, c0n, c1n);
     }
+    /* genotype planes: the super-steps' places follow the words */
+    std::vector<SuperSrc> src;
+    const size_t cw_words = cw.size();
+    if (geno) {
+        build_super_src(cw, p->w64, n0, n1, src);
+        cw.resize(cw_words + (src.size() * sizeof(SuperSrc) + sizeof(CompressWord) - 1) / sizeof(CompressWord));
+        if (!src.empty()) memcpy(cw.data() + cw_words, src.data(), src.size() * sizeof(SuperSrc));
+    }
     /* Candidate buffers: between bands at most k records are kept, and a
      * one-tile band admits at most TILE_EVALS_MAX, so cap >= k +
      * TILE_EVALS_MAX lets a band shrunk to one tile always complete.        */
     const unsigned long long cap_min = (unsigned long long)k + TILE_EVALS_MAX + 1024;
-    /* 4k or 2^23 records, but no more than a 64th of the evaluations: bands
-     * are sized for the lists, and a drop-in call allocates them anew (a
-     * list of 2^23 records cost 0.5 ms to allocate and free, with 80 bytes a
-     * record three fifths of a 1,020 x 89 call)                             */
+    /* 4k or 2^23 records, for k up to 16,384 no more than a 64th of the evaluations:
+     * bands are sized for the lists, and a drop-in call allocates them anew
+     * (a list of 2^23 records cost 0.5 ms to allocate and free, with 80 bytes
+     * a record three fifths of a 1,020 x 89 call)                           */
     unsigned long long cap = std::max<unsigned long long>(
         cap_min, std::min<unsigned long long>(
                      (unsigned long long)std::max<int64_t>(4 * k, 1 << 23),
-                     std::max<unsigned long long>((unsigned long long)total_evals / 64, 1u << 18)));
+                     std::max<unsigned long long>({(unsigned long long)total_evals / 64, k > 16384 ? 1ull << 23 : 1ull << 18})));
     if (const char *env = getenv("GEPI_CAND_CAP")) {
         /* capacity override for exercising the overflow recovery in tests */
         cap = std::max<unsigned long long>((unsigned long long)std::max(atoll(env), 0ll), cap_min);
@@ -650,7 +669,13 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
     if (fp4) {
         const int64_t rows = n_var_pad * 3;
         const unsigned cgrid = (unsigned)((rows + 255) / 256);
-        if (n_ks > 0 && path == 3) {
+        if (geno) {
+            k_class_geno<<<dim3((unsigned)(n_var_pad / 64), (unsigned)n_u + 1), CLSG_THREADS, 0, p->stream>>>(
+                p->d_nat, (int32_t)n_var, p->w64, b.cw,
+                reinterpret_cast<const SuperSrc *>(b.cw + cw_words), n_u, n0 + n1,
+                reinterpret_cast<uint4 *>(b.clsk), reinterpret_cast<float *>(d_pc3));
+            HIP_TRY(hipGetLastError());
+        } else if (n_ks > 0 && path == 3) {
             k_class_f4<3, true><<<cgrid, 256, 0, p->stream>>>(
                 p->d_nat, (int32_t)n_var, p->w64, b.cw, rows, f4_super3(w0 / 4),
                 reinterpret_cast<uint4 *>(b.clsk), d_pc3);
@@ -707,6 +732,8 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
     ca.n0 = n0;
     ca.n1 = n1;
     chi2_slope(n0, n1, &ca.h0, &ca.h1);
+    ca.miss = reinterpret_cast<const float *>(d_pc3);
+    screen_consts(n0, n1, ca);
     ca.st = b.state;
     ca.pend = b.pend;
     ca.pcap = pcap;
@@ -761,7 +788,12 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
         auto go = [&](auto kernel, unsigned threads) {
             hipExtLaunchKernelGGL(kernel, dim3(grid), dim3(threads), 0, p->stream, e0, e1, 0, ca);
         };
-        if (path == 3) {
+        if (geno) {
+            if (entropy)
+                go(k_count_f4g<GEPI_FFUNC_ENTROPY>, F4W_THREADS);
+            else
+                go(k_count_f4g<GEPI_FFUNC_FISHERPV>, F4W_THREADS);
+        } else if (path == 3) {
             if (entropy && f32 && park)
                 go(k_count_f4w<GEPI_FFUNC_ENTROPY, true, true>, F4W_THREADS);
             else if (entropy && f32)
@@ -814,16 +846,19 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
     const double guess = entropy ? GUESS_ENTROPY : GUESS_FISHER;
     /* the share of n tiles' evaluations that the first threshold admits */
     auto share = [&](int64_t n) { return guess * (double)k / ((double)n * evals_per_tile); };
-    /* the first band: a scan of up to about 5,000 variants whole, else one
-     * tile per workgroup the chip holds, as a pilot for the others' sizes */
-    int64_t first = n_tiles <= 6400 ? n_tiles : 1024;
-    if (first == n_tiles && n_tiles > 1024 && plan.survivors(first, share(first)) > 600000.0) first = 1024;
+    /* the first band: a scan of up to about 5,000 variants whole; else a pilot
+     * of one tile per workgroup the chip holds, or more where that would
+     * admit more than 4e-5 (the filter's expensive branch in most waves)   */
+    int64_t first = n_tiles;
+    if (n_tiles > 6400 || plan.survivors(first, share(first)) > 600000.0)
+        first = std::min<int64_t>(n_tiles, std::max<int64_t>(1024, (int64_t)(share(1) / 4e-5)));
     const bool hooks = forced_band || getenv("GEPI_CAND_CAP") || getenv("GEPI_PEND_CAP");
     const bool planned = fp4 && n_ks > 0 && !hooks && !par->intermediate && par->max_grid_area <= 0 &&
-                         share(first) <= 0.02 && 1.5 * (guess + 1.0) * (double)k <= (double)cap &&
+                         share(first) <= 0.1 && 1.5 * (guess + 1.0) * (double)k <= (double)cap &&
                          (guess + 1.0) * (double)k <= (double)WG_SELECT_MAX &&
                          plan.survivors(first, share(first)) <= plan.most;
     if (planned) {
+        if (!p->mail) HIP_TRY(hipHostMalloc(&p->mail, sizeof(HostMail), hipHostMallocDefault));
         HostMail *mail = static_cast<HostMail *>(p->mail);
         while (p->band_ev.size() < 2 * PLAN_BANDS) {
             hipEvent_t e;
@@ -1052,6 +1087,7 @@ int upload_planes(gepi_panel *p, const uint64_t *bits, const uint64_t *valid, in
                   int32_t words) {
     const int64_t n_var = n_rows / 2;
     std::vector<uint64_t> nat((size_t)(n_var > 0 ? n_var : 1) * 3 * (words > 0 ? words : 1), 0);
+    uint64_t bare = 0; /* valid calls without an allele */
     for (int64_t v = 0; v < n_var; v++) {
         const uint64_t *b1 = bits + (size_t)(2 * v) * words, *b2 = b1 + words;
         const uint64_t *v1 = valid + (size_t)(2 * v) * words;
@@ -1060,8 +1096,10 @@ int upload_planes(gepi_panel *p, const uint64_t *bits, const uint64_t *valid, in
             o[w] = b1[w] & v1[w];
             o[words + w] = b2[w] & v1[w];
             o[2 * words + w] = v1[w];
+            bare |= v1[w] & ~(b1[w] | b2[w]);
         }
     }
+    p->three_genotypes = bare == 0;
     /* on the panel's stream, after panel_alloc's zero fill of the same
      * buffer (a null-stream copy would not be ordered with that non-blocking
      * stream); nat lives until the synchronisation */
@@ -1266,6 +1304,7 @@ extern "C" int gepi_panel_filter(gepi_panel *p, float max_miss_snps, float max_m
                 keep_samples[s >> 6] |= 1ull << (s & 63);
     }
     gepi_panel *q = new gepi_panel();
+    q->three_genotypes = p->three_genotypes;
     if ((rc = panel_alloc(q, p->device, (int64_t)keep.size(), p->n_samples)) != GEPI_OK) {
         panel_free(q);
         return rc;

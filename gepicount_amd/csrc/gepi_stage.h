@@ -322,6 +322,103 @@ __global__ void __launch_bounds__(256) k_class_f4(const uint64_t *__restrict__ n
     }
 }
 
+/* Where a super-step's 384 class samples lie in the panel's file order: from
+ * bit `skip` of the class's samples in 32-bit word j0, up to word j1. */
+struct SuperSrc {
+    int32_t cls, j0, skip, j1;
+};
+
+/* Class layout of the wave tiles on genotype planes (count_f4g_unit): the
+ * grouped layout with plane 0 = homozygous for allele 1 (a1 & ~a2), 1 =
+ * heterozygous (a1 & a2), 2 = homozygous for allele 2.  blockIdx.x: 64
+ * variants, a wave per plane; blockIdx.y: the super-step, whose samples the
+ * host has located (src), so that a scan's super-steps are made in parallel
+ * (one thread for a row's whole sample range took 384 us for 8,000 x 20,001
+ * and 38 us for 20,000 x 2,048).  blockIdx.y = n_u: the variants' shares of
+ * missing calls among the class samples, rounded up.                       */
+constexpr int CLSG_THREADS = 192;
+static __global__ void __launch_bounds__(CLSG_THREADS)
+    k_class_geno(const uint64_t *__restrict__ nat, int32_t n_var, int32_t w64,
+                 const CompressWord *__restrict__ cw, const SuperSrc *__restrict__ src, int32_t n_u,
+                 int32_t n, uint4 *__restrict__ out, float *__restrict__ miss) {
+    __shared__ uint64_t row[2][64][CLS_CHUNK + 1];
+    __shared__ int32_t valid[64];
+    const int tid = threadIdx.x, p = tid >> 6, vl = tid & 63;
+    const int32_t v0 = blockIdx.x * 64, u = blockIdx.y;
+    auto stage = [&](int32_t w0) {
+        /* words w0 .. w0 + 7 of the allele planes of the 64 variants */
+        __syncthreads();
+        for (int i = tid; i < 2 * 64 * CLS_CHUNK; i += CLSG_THREADS) {
+            const int wd = i % CLS_CHUNK, v = (i / CLS_CHUNK) & 63, pl = i / (64 * CLS_CHUNK);
+            const bool in = v0 + v < n_var && w0 + wd < w64;
+            row[pl][v][wd] = in ? nat[((int64_t)(v0 + v) * 3 + pl) * w64 + w0 + wd] : 0ull;
+        }
+        __syncthreads();
+    };
+    if (u == n_u) {
+        if (tid < 64) valid[tid] = 0;
+        int32_t c0 = 0;
+        for (int32_t w0 = 0; w0 < w64; w0 += CLS_CHUNK) {
+            stage(w0);
+            const int32_t nw = w64 - w0 < CLS_CHUNK ? w64 - w0 : CLS_CHUNK;
+            for (int32_t wd = p; wd < nw; wd += 3) { /* the waves share the words */
+                const uint64_t x = row[0][vl][wd] | row[1][vl][wd];
+                const CompressWord *a = cw + 2 * (w0 + wd), *b = a + 2 * w64;
+                c0 += __popcll(x & (((uint64_t)a[1].m << 32) | a[0].m)) +
+                      __popcll(x & (((uint64_t)b[1].m << 32) | b[0].m));
+            }
+        }
+        __syncthreads();
+        atomicAdd(&valid[vl], c0);
+        __syncthreads();
+        if (p == 0 && n > 0)
+            miss[v0 + vl] = (float)(n - valid[vl]) / (float)n * (1.0f + 1e-6f);
+        if (p == 0 && n <= 0) miss[v0 + vl] = 0.0f;
+        return;
+    }
+    const SuperSrc s = src[u];
+    const CompressWord *c = cw + (int64_t)s.cls * 2 * w64;
+    uint64_t acc = 0;
+    int32_t na = 0, nq = 0, skip = s.skip;
+    uint32_t q[12]; /* the last 12 words made; the oldest first */
+#pragma unroll
+    for (int i = 0; i < 12; i++) q[i] = 0;
+    auto emit = [&](uint32_t w) {
+#pragma unroll
+        for (int i = 0; i < 11; i++) q[i] = q[i + 1];
+        q[11] = w;
+        nq++;
+    };
+    for (int32_t w0 = s.j0 >> 1; 2 * w0 < s.j1; w0 += CLS_CHUNK) {
+        stage(w0);
+        for (int32_t wd = 0; wd < CLS_CHUNK; wd++) {
+            const uint64_t a1 = row[0][vl][wd], a2 = row[1][vl][wd];
+            const uint64_t x = p == 0 ? a1 & ~a2 : p == 1 ? a1 & a2 : a2 & ~a1;
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int32_t j = 2 * (w0 + wd) + h;
+                if (j < s.j0 || j >= s.j1) continue;
+                const CompressWord m = c[j];
+                acc |= (uint64_t)(compress_word((uint32_t)(x >> (32 * h)), m) >> skip) << na;
+                na += (int32_t)m.cnt - skip;
+                skip = 0;
+                if (na >= 32 && nq < 12) {
+                    emit((uint32_t)acc);
+                    acc >>= 32;
+                    na -= 32;
+                }
+            }
+        }
+    }
+    /* a class's last super-step: zero-padded */
+    if (nq < 12) emit((uint32_t)acc);
+    while (nq < 12) emit(0u);
+    const int64_t G = blockIdx.x * 2 + (vl >> 5), NG = (int64_t)gridDim.x * 2;
+    uint4 *dst = out + (((int64_t)u * NG + G) * 3 + p) * 128 + (vl & 31);
+#pragma unroll
+    for (int g = 0; g < 4; g++) dst[32 * g] = super_group(q[g], q[4 + g], q[8 + g], 0u);
+}
+
 /* missing[v] = n_samples - popc(valid plane of variant v); 64 threads per
  * variant.  Samples beyond n_samples are never valid in a panel. */
 static __global__ void __launch_bounds__(256) k_qa_variants(const uint64_t *__restrict__ nat,
