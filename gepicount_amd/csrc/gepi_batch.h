@@ -10,6 +10,7 @@
  *   k_count_f4w_batch the same for scans on wave tiles (Fisher's, and long
  *                     entropy scans): one (scan, unit of two tiles) slot per
  *                     workgroup
+ *   k_count_f4g_batch the same on genotype planes (every .bed panel's)
  *   k_exact_batch     exact scores of each scan's filter survivors
  *                     (blockIdx.y = scan)
  *   k_topk_wg         one 1024-thread workgroup per scan: radix select of
@@ -146,6 +147,18 @@ k_count_f4w_batch(const BatchDesc *__restrict__ d, BatchMap map) {
         count_f4w_unit<FFUN, true, PARK>(g, unit, sh);
     else
         count_f4w_unit<FFUN, false, PARK>(g, unit, sh);
+}
+
+/* The same for scans on genotype planes (count_f4g_unit). */
+template <int FFUN>
+__global__ void __launch_bounds__(F4W_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
+k_count_f4g_batch(const BatchDesc *__restrict__ d, BatchMap map) {
+    __shared__ F4GShared sh;
+    const F4BatchOnceSrc src{d, map};
+    const F4Job j = uniform_job(src.grab(0));
+    if (!j.ok) return;
+    const CountArgs g = d[j.item].g;
+    count_f4g_unit<FFUN>(g, j.tile - g.tile_begin, sh);
 }
 
 /* p[0..n) = v (one workgroup of 64 threads per 64 words). */

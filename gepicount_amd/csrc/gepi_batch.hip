@@ -34,7 +34,15 @@ constexpr int EXACT_BLOCKS_X = 64; /* blocks per scan of the batched exact pass 
  * persistent launch, count launches: 1.27-1.32x the time at 1,536-2,048
  * samples, 1.10-1.14x at 3,072-4,096, 0.97x at 6,144, 0.85x at 8,192.     */
 constexpr int32_t BATCH_WAVE_MIN_KSTEPS = 48;
-int batch_shape_default(int32_t ks) { return ks >= BATCH_WAVE_MIN_KSTEPS ? 2 : 0; }
+/* On genotype planes, whose screen spares most of the filter, also from 256
+ * tiles (1,000 variants) on: 4 scans a batch, whole batches, against whole
+ * tiles 0.78x the time for 40,000 x 256, 0.73x for 28,000 x 1,024, 0.71x for
+ * 18,000 x 4,096, 0.82-0.91x for 1,000-4,000 x 1,000-2,000, 1.04x for 600 x
+ * 600 (10 x 11 tiles).                                                     */
+constexpr int64_t BATCH_GENO_MIN_TILES = 256;
+int batch_shape_default(int32_t ks, int64_t n_tiles, bool geno) {
+    return ks >= BATCH_WAVE_MIN_KSTEPS || (geno && n_tiles >= BATCH_GENO_MIN_TILES) ? 2 : 0;
+}
 
 double ms_since(std::chrono::steady_clock::time_point t) {
     return std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t).count();
@@ -88,7 +96,11 @@ void Engine::launch_count(int g, bool persist, unsigned grid, const BatchMap &m)
     const BatchDesc *d = d_bdesc_[g];
     if (g >= 4) {
         /* wave tiles: one unit per workgroup, no persistent form */
-        if (g == 4)
+        if (g == 6)
+            k_count_f4g_batch<GEPI_FFUNC_ENTROPY><<<grid, F4W_THREADS, 0, stream>>>(d, m);
+        else if (g == 7)
+            k_count_f4g_batch<GEPI_FFUNC_FISHERPV><<<grid, F4W_THREADS, 0, stream>>>(d, m);
+        else if (g == 4)
             k_count_f4w_batch<GEPI_FFUNC_ENTROPY><<<grid, F4W_THREADS, 0, stream>>>(d, m);
         else
             k_count_f4w_batch<GEPI_FFUNC_FISHERPV><<<grid, F4W_THREADS, 0, stream>>>(d, m);
@@ -292,7 +304,8 @@ int Engine::autotune(int32_t repeats) {
     /* the default schedule's shape for a class's trial scans (about half
      * cases); captured rounds run whole tiles in place of wave tiles     */
     auto dflt_tile = [&](int c) {
-        return use_graph_ ? 0 : batch_shape_default((trials[c].n / 2 + 127) / 128 * 2);
+        const int64_t a4 = (trials[c].n_var + TM - 1) / TM;
+        return use_graph_ ? 0 : batch_shape_default((trials[c].n / 2 + 127) / 128 * 2, a4 * (a4 + 1), true);
     };
     repeats = std::max(1, std::min(repeats, 16));
     std::vector<gepi_tune_class> table;
@@ -451,7 +464,7 @@ size_t Engine::estimate_footprint(const gepi_panel *p, int64_t topmost) {
     const unsigned long long cap =
         std::max<unsigned long long>((unsigned long long)k + TILE_EVALS_MAX + 1024, 4ull * k);
     const unsigned long long pcap = std::max<unsigned long long>(cap, 1ull << 20);
-    return round_block((size_t)n_u * n_var_pad * 3 * 64) + round_block(cap * sizeof(Cand)) +
+    return round_block((size_t)n_u * n_var_pad * 3 * 64 + (size_t)n_var_pad * sizeof(float)) + round_block(cap * sizeof(Cand)) +
            round_block(pcap * sizeof(Pend)) + round_block((size_t)4 * p->w64 * sizeof(CompressWord)) +
            round_block(sizeof(ScanState));
 }
@@ -505,9 +518,11 @@ int Engine::add(ScanItem *it) {
      * rounds have no wave-tile launch                                      */
     const int32_t ks = (it->n0 + 127) / 128 + (it->n1 + 127) / 128;
     const gepi_tune_class *tc = tune_of(ks);
-    it->shape = tc ? tc->tile : batch_shape_default(ks);
+    const int64_t a4 = (p->n_var + TM - 1) / TM;
+    it->shape = tc ? tc->tile : batch_shape_default(ks, a4 * (a4 + 1), p->three_genotypes);
     if (it->ffun != GEPI_FFUNC_ENTROPY && !use_graph_) it->shape = 2;
     if (it->shape == 2 && use_graph_) it->shape = 0;
+    it->geno = it->shape == 2 && p->three_genotypes;
     it->stats.count_path = it->shape == 2 ? 3 : 4;
     it->stats.n_class0 = it->n0;
     it->stats.n_class1 = it->n1;
@@ -551,7 +566,16 @@ int Engine::add(ScanItem *it) {
                                                 (unsigned long long)TILE_EVALS_MAX + 1024);
     /* three K steps per super-step (f4_super3, see count_f4_run) */
     const int32_t n_u = f4_super3(w0 / 4) + f4_super3(w1 / 4); /* 64-byte rows each */
-    const size_t lay = (size_t)std::max(n_u, 1) * it->n_var_pad * 3 * 4 * sizeof(uint4);
+    const size_t rows_bytes = (size_t)std::max(n_u, 1) * it->n_var_pad * 3 * 4 * sizeof(uint4);
+    const size_t lay = rows_bytes + (it->geno ? (size_t)it->n_var_pad * sizeof(float) : 0);
+    const size_t cw_words = it->h_cw.size();
+    if (it->geno) {
+        /* the super-steps' places follow the compression words */
+        std::vector<SuperSrc> src;
+        build_super_src(it->h_cw, p->w64, it->n0, it->n1, src);
+        it->h_cw.resize(cw_words + (src.size() * sizeof(SuperSrc) + sizeof(CompressWord) - 1) / sizeof(CompressWord));
+        if (!src.empty()) memcpy(it->h_cw.data() + cw_words, src.data(), src.size() * sizeof(SuperSrc));
+    }
     it->d_layout = (uint4 *)dalloc(lay);
     it->d_cw = (CompressWord *)dalloc(it->h_cw.size() * sizeof(CompressWord));
     it->d_pend = (Pend *)dalloc(it->pcap * sizeof(Pend));
@@ -565,14 +589,16 @@ int Engine::add(ScanItem *it) {
     it->footprint = round_block(lay) + round_block(it->h_cw.size() * sizeof(CompressWord)) +
                     round_block(it->pcap * sizeof(Pend)) + round_block(it->cap * sizeof(Cand)) +
                     round_block(sizeof(ScanState));
-    memset(&it->h_state0, 0, sizeof it->h_state0);
-    it->h_state0.thr_score = INFINITY;
-    it->h_state0.thr_idx = ~0ull;
     HIP_TRY(hipMemcpyAsync(it->d_cw, it->h_cw.data(), it->h_cw.size() * sizeof(CompressWord),
                            hipMemcpyHostToDevice, stream));
-    HIP_TRY(hipMemcpyAsync(it->d_state, &it->h_state0, sizeof(ScanState), hipMemcpyHostToDevice,
-                           stream));
-    if (it->n_k4 > 0) {
+    if (it->geno) {
+        it->d_miss = reinterpret_cast<const float *>(reinterpret_cast<char *>(it->d_layout) + rows_bytes);
+        k_class_geno<<<dim3((unsigned)(it->n_var_pad / 64), (unsigned)n_u + 1), CLSG_THREADS, 0, stream>>>(
+            p->d_nat, (int32_t)it->n_var, p->w64, it->d_cw,
+            reinterpret_cast<const SuperSrc *>(it->d_cw + cw_words), n_u, it->n0 + it->n1, it->d_layout,
+            const_cast<float *>(it->d_miss));
+        HIP_TRY(hipGetLastError());
+    } else if (it->n_k4 > 0) {
         const int64_t rows = it->n_var_pad * 3;
         const unsigned cgrid = (unsigned)((rows + 255) / 256);
         if (it->shape == 2)
@@ -587,16 +613,41 @@ int Engine::add(ScanItem *it) {
     }
     const double band_evals = tc ? tc->band_evals : 2.0e9;
     it->max_band = std::max<int64_t>(64, (int64_t)(band_evals / (double)F4_TILE_EVALS));
-    it->band = std::max<int64_t>(1, std::min<int64_t>(it->max_band, (2 * it->k) / F4_TILE_EVALS + 1));
+    const int64_t band = std::max<int64_t>(1, std::min<int64_t>(it->max_band, (2 * it->k) / F4_TILE_EVALS + 1));
     it->forced_band = 0;
-    if (const char *env = getenv("GEPI_BAND_TILES")) {
-        it->forced_band = std::max<long long>(1, atoll(env));
-        it->band = it->forced_band;
+    if (const char *env = getenv("GEPI_BAND_TILES")) it->forced_band = std::max<long long>(1, atoll(env));
+    /* the first band under a guessed threshold, as in a planned single scan */
+    CountArgs ca;
+    chi2_slope(it->n0, it->n1, &ca.h0, &ca.h1);
+    BandPlan &pl = it->plan;
+    pl = BandPlan{};
+    pl.entropy = it->ffun == GEPI_FFUNC_ENTROPY;
+    pl.evals_tile = (double)F4_TILE_EVALS;
+    pl.h = (double)ca.h0 + (double)ca.h1 * std::min(it->n0, it->n1);
+    pl.k = (double)it->k;
+    pl.most = (double)it->pcap / 4;
+    it->first = std::min(pl.first(it->n_tiles), it->max_band);
+    it->guessed = it->n_k4 > 0 && !it->forced_band && !getenv("GEPI_CAND_CAP") && !getenv("GEPI_PEND_CAP") &&
+                  pl.sound(it->first, it->cap);
+    int rs;
+    if ((rs = it->guessed ? start(it, pl.score(pl.share(it->first), it->n0 + it->n1), it->first)
+                          : start(it, INFINITY, it->forced_band ? it->forced_band : band)) != GEPI_OK) {
+        drop(it, rs);
+        return rs;
     }
+    active_.push_back(it);
+    return GEPI_OK;
+}
+
+int Engine::start(ScanItem *it, double thr, int64_t band) {
+    float kf, kt;
+    threshold_coeffs(thr, it->ffun, kf, kt);
+    k_state_init<<<1, 256, 0, stream>>>(it->d_state, thr, kf, kt);
+    HIP_TRY(hipGetLastError());
+    it->band = band;
     it->t0 = 0;
     it->count = 0;
     it->exact_total = 0;
-    active_.push_back(it);
     return GEPI_OK;
 }
 
@@ -640,7 +691,7 @@ int Engine::round(std::vector<ScanItem *> &finished) {
     std::vector<TopkDesc> td(na);
     for (size_t i = 0; i < na; i++) {
         ScanItem *it = active_[i];
-        grp[(it->ffun == GEPI_FFUNC_ENTROPY ? 0 : 1) + 2 * it->shape].push_back(it);
+        grp[(it->ffun == GEPI_FFUNC_ENTROPY ? 0 : 1) + 2 * (it->geno ? 3 : it->shape)].push_back(it);
         ExactDesc &e = ed[i];
         memset(&e, 0, sizeof e);
         e.e.st = it->d_state;
@@ -726,6 +777,8 @@ int Engine::round(std::vector<ScanItem *> &finished) {
             d.g.n0 = it->n0;
             d.g.n1 = it->n1;
             chi2_slope(it->n0, it->n1, &d.g.h0, &d.g.h1);
+            d.g.miss = it->d_miss;
+            screen_consts(it->n0, it->n1, d.g);
             d.g.st = it->d_state;
             d.g.pend = it->d_pend;
             d.g.pcap = it->pcap;
@@ -737,7 +790,7 @@ int Engine::round(std::vector<ScanItem *> &finished) {
                 d.g.park_slots = (uint32_t)park_slots_;
             }
             bd[f].push_back(d);
-            const int64_t b = shape == 2 ? (it->band_used + 1) / 2 : it->band_used * per_tile;
+            const int64_t b = shape >= 2 ? (it->band_used + 1) / 2 : it->band_used * per_tile;
             const int64_t r = dealt & 7;
             int64_t start = 0;
             for (int x = 0; x < 8; x++) {
@@ -866,10 +919,25 @@ int Engine::round(std::vector<ScanItem *> &finished) {
         if (adm_rate > 0.0)
             next = std::min<int64_t>(
                 next, (int64_t)((double)((it->cap - (unsigned long long)it->k) / 2) / adm_rate));
-        it->band = std::max<int64_t>(1, std::min<int64_t>(next, used * 4));
-        if (it->forced_band) it->band = std::min<int64_t>(it->forced_band, used * 4);
         it->t0 += used;
-        if (it->t0 >= it->n_tiles) {
+        int64_t grow = used * 4;
+        if (it->guessed && it->t0 < it->n_tiles) {
+            if (it->t0 == used) it->plan.learn(used, it->plan.share(it->first), r.pend_count);
+            grow = it->plan.next(it->t0, it->n_tiles - it->t0);
+        }
+        it->band = std::max<int64_t>(1, std::min<int64_t>(next, grow));
+        if (it->forced_band) it->band = std::min<int64_t>(it->forced_band, used * 4);
+        const bool done = it->t0 >= it->n_tiles;
+        if (it->guessed && (done || it->t0 >= it->first) &&
+            it->count < (unsigned long long)(done ? it->k : it->k / 4)) {
+            /* too few under the guessed threshold: again without it */
+            it->guessed = false;
+            if ((rc = start(it, INFINITY,
+                            std::max<int64_t>(1, std::min<int64_t>(it->max_band, (2 * it->k) / F4_TILE_EVALS + 1)))) !=
+                GEPI_OK)
+                return rc;
+            still.push_back(it);
+        } else if (done) {
             if ((rc = finish(it)) != GEPI_OK) return rc;
             finished.push_back(it);
         } else {

@@ -53,6 +53,11 @@ struct ScanItem {
     /* count job shape (its class's tile): 0 tiles, 1 half tiles, 2 wave
      * tiles on the grouped layout                                          */
     int32_t shape = 0;
+    bool geno = false;    /* wave tiles on genotype planes */
+    const float *d_miss = nullptr; /* ... and their missing shares (in d_layout) */
+    bool guessed = false; /* the first band runs under a guessed threshold    */
+    BandPlan plan{};
+    int64_t first = 0;    /* tiles of that band                               */
     unsigned long long cap = 0, pcap = 0, count = 0, exact_total = 0;
     uint4 *d_layout = nullptr;
     gepi::CompressWord *d_cw = nullptr;
@@ -61,7 +66,6 @@ struct ScanItem {
     gepi::ScanState *d_state = nullptr;
     size_t footprint = 0; /* device bytes held */
     std::vector<gepi::CompressWord> h_cw;
-    gepi::ScanState h_state0;
 };
 
 class Engine {
@@ -99,6 +103,8 @@ class Engine {
     void *dalloc(size_t bytes);
     void dfree(void *p);
     int finish(ScanItem *it);
+    /* Starts a scan (again): its state admits what scores at most thr. */
+    int start(ScanItem *it, double thr, int64_t band);
     void drop(ScanItem *it, int status);
     int grow_desc(size_t n);
     /* The class of a scan with n_k4 K steps (nullptr without a table). */
@@ -112,7 +118,7 @@ class Engine {
      * groups in bit mask part: bit g = objective (g & 1: 0 entropy, 1
      * Fisher) and job shape (g >> 1: 0 whole tiles, 1 half tiles)), part
      * NGRAPH_COUNT into gx_finish_ (exact + top-k launches).  Wave-tile
-     * groups (4, 5) have no persistent form and are never captured: with
+     * groups (4-7) have no persistent form and are never captured: with
      * graphs on, scans keep whole tiles instead.                          */
     int capture_graph(int part, int per_cu);
     /* One count launch of group g (as in capture_graph). */
@@ -124,8 +130,9 @@ class Engine {
     std::multimap<size_t, void *> free_;
     std::map<void *, size_t> live_;
     size_t in_use_ = 0;
-    /* count launch groups: objective (g & 1) x job shape (g >> 1) */
-    static constexpr int NGROUP = 6, NGRAPH_COUNT = 16;
+    /* count launch groups: objective (g & 1) x job shape (g >> 1; 3: wave
+     * tiles on genotype planes) */
+    static constexpr int NGROUP = 8, NGRAPH_COUNT = 16;
     gepi::BatchDesc *d_bdesc_[NGROUP] = {};
     int64_t *d_map_[NGROUP] = {};
     gepi::ExactDesc *d_edesc_ = nullptr;

@@ -171,6 +171,99 @@ inline void screen_consts(int32_t n0, int32_t n1, gepi::CountArgs &g) {
     g.sc_sub = (float)(18.0 * start * (1.0 + 2.0 * k) + 1e-3);
 }
 
+/* ---- planned bands --------------------------------------------------------
+ * A scan's bands need no answer from the device between them: a band's
+ * count, exact and top-k launches find the threshold, the lists and an
+ * overflow flag in device memory, so all of them can be enqueued at once and
+ * their reports read at the end (bands that overflowed are redone; the order
+ * of bands does not change the result).  What has to be chosen beforehand is
+ * the size of each band, from how many evaluations its threshold lets
+ * through, and a threshold for the first one.
+ *
+ * Without association 2 m I (I in nats) of a table is close to chi-square
+ * with one degree of freedom, and P(p <= a) of a Fisher test is at most a.
+ * So the first band, a pilot, admits the quantile where GUESS times k of its
+ * evaluations are expected: few enough to be cheap, and if the k best are
+ * among them (nearly always: the count says so) the threshold was valid.
+ * The others run under the k-th key so far.  A scan that ends with fewer than
+ * k records is run again without the guess.  (Guessing the whole scan's
+ * threshold after the pilot saved 10-15% where it held, but the tail hangs
+ * on the few variants with the largest effects of their own: over seeds the
+ * k-th key had 0.17 to 2 times the expected evaluations beyond it.)
+ * Against bands that began with one tile admitting everything and grew
+ * fourfold, a host round trip (40 us) and a selection between two: 1,024 x
+ * 256 0.73 -> 0.13 ms (5 bands -> 1), 3,001 x 777 Fisher 1.44 -> 0.29, 20,000
+ * x 2,048 3.69 -> 2.38 (10 -> 3), 8,000 x 20,001 3.84 -> 2.50.               */
+constexpr double GUESS_ENTROPY = 8.0, GUESS_FISHER = 16.0;
+
+/* P(chi2_1 > t) and its inverse */
+inline double chi2_tail(double t) { return std::erfc(std::sqrt(0.5 * std::max(t, 0.0))); }
+inline double chi2_quantile(double p) {
+    double lo = 0.0, hi = 1400.0;
+    for (int i = 0; i < 60; i++) {
+        const double mid = 0.5 * (lo + hi);
+        (chi2_tail(mid) > p ? lo : hi) = mid;
+    }
+    return lo;
+}
+
+struct BandPlan {
+    bool entropy;
+    double evals_tile;  /* evaluations per tile                              */
+    double h;           /* chi-square coefficient per nat (chi2_slope)       */
+    double k;
+    double most;        /* survivors a band may have                         */
+    double factor = 1.0; /* survivors measured over survivors expected       */
+
+    /* Expected survivors per evaluation under the threshold that admits a
+     * share q: the filter's chi-square cut is h/2 of the quantile; Fisher's
+     * exact check of log10 P(obs) admits a few times the two-sided p.      */
+    double pass(double q) const {
+        q = std::min(q, 1.0);
+        return entropy ? chi2_tail(0.5 * h * chi2_quantile(q)) : std::min(1.0, 4.0 * q);
+    }
+    double survivors(int64_t tiles, double q) const {
+        return factor * (double)tiles * evals_tile * pass(q);
+    }
+    double guess() const { return entropy ? GUESS_ENTROPY : GUESS_FISHER; }
+    /* the share of n tiles' evaluations that the first threshold admits */
+    double share(int64_t n) const { return guess() * k / ((double)n * evals_tile); }
+    /* the score that a share q of unassociated evaluations reaches */
+    double score(double q, int32_t n) const {
+        return entropy ? -chi2_quantile(q) / (2.0 * n) * 1.4426950408889634 : std::log10(q);
+    }
+    /* the first band: a scan of up to about 5,000 variants whole; else a pilot
+     * of one tile per workgroup the chip holds, or more where that would
+     * admit more than 4e-5 (the filter's expensive branch in most waves)   */
+    int64_t first(int64_t n_tiles) const {
+        if (n_tiles <= 6400 && survivors(n_tiles, share(n_tiles)) <= 600000.0) return n_tiles;
+        return std::min<int64_t>(n_tiles, std::max<int64_t>(1024, (int64_t)(share(1) / 4e-5)));
+    }
+    /* whether a guess for n tiles tells anything and the lists hold it */
+    bool sound(int64_t n, unsigned long long cap) const {
+        return share(n) <= 0.1 && 1.5 * (guess() + 1.0) * k <= (double)cap &&
+               survivors(n, share(n)) <= most;
+    }
+    void learn(int64_t n, double q, unsigned long long found) {
+        factor = std::min(64.0, std::max(0.25, (double)found / std::max(1.0, survivors(n, q))));
+    }
+    /* Tiles of the band that follows `done` tiles.  About 250,000 survivors
+     * cost what a band's fixed part does (100 us); at least three times what
+     * is done while the list holds them, at most that for Fisher and eight
+     * times for entropy (the pairs that pass the screen cost more under an
+     * older threshold).                                                     */
+    int64_t next(int64_t done, int64_t left) const {
+        const double q = 1.3 * k / ((double)done * evals_tile);
+        const double per = factor * evals_tile * pass(q);
+        const double cheap = std::min(std::max(250000.0 / per, 3.0 * (double)done),
+                                      (entropy ? 8.0 : 3.0) * (double)done);
+        const double tiles = std::min({cheap, most / per, 1048576.0, (double)left});
+        /* a remainder below a fifth of the band goes with it */
+        if ((double)left < 1.2 * tiles && (double)left * per < most) return left;
+        return std::max<int64_t>(1, (int64_t)tiles);
+    }
+};
+
 /* Sorts candidate records by the canonical key and writes the first
  * min(k, size) as results; returns how many were written.                   */
 inline int64_t candidates_to_results(std::vector<gepi::Cand> &host, int64_t k, gepi_result *tops) {

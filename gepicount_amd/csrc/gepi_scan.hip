@@ -368,77 +368,6 @@ double ms_since(std::chrono::steady_clock::time_point t) {
     return std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t).count();
 }
 
-/* ---- planned bands --------------------------------------------------------
- * A scan's bands need no answer from the device between them: a band's
- * count, exact and top-k launches find the threshold, the lists and an
- * overflow flag in device memory, so all of them can be enqueued at once and
- * their reports read at the end (bands that overflowed are redone; the order
- * of bands does not change the result).  What has to be chosen beforehand is
- * the size of each band, from how many evaluations its threshold lets
- * through, and a threshold for the first one.
- *
- * Without association 2 m I (I in nats) of a table is close to chi-square
- * with one degree of freedom, and P(p <= a) of a Fisher test is at most a.
- * So the first band, a pilot, admits the quantile where GUESS times k of its
- * evaluations are expected: few enough to be cheap, and if the k best are
- * among them (nearly always: the count says so) the threshold was valid.
- * The others run under the k-th key so far.  A scan that ends with fewer than
- * k records is run again without the guess.  (Guessing the whole scan's
- * threshold after the pilot saved 10-15% where it held, but the tail hangs
- * on the few variants with the largest effects of their own: over seeds the
- * k-th key had 0.17 to 2 times the expected evaluations beyond it.)
- * Against bands that began with one tile admitting everything and grew
- * fourfold, a host round trip (40 us) and a selection between two: 1,024 x
- * 256 0.73 -> 0.13 ms (5 bands -> 1), 3,001 x 777 Fisher 1.44 -> 0.29, 20,000
- * x 2,048 3.69 -> 2.38 (10 -> 3), 8,000 x 20,001 3.84 -> 2.50.               */
-constexpr double GUESS_ENTROPY = 8.0, GUESS_FISHER = 16.0;
-
-/* P(chi2_1 > t) and its inverse */
-inline double chi2_tail(double t) { return std::erfc(std::sqrt(0.5 * std::max(t, 0.0))); }
-double chi2_quantile(double p) {
-    double lo = 0.0, hi = 1400.0;
-    for (int i = 0; i < 60; i++) {
-        const double mid = 0.5 * (lo + hi);
-        (chi2_tail(mid) > p ? lo : hi) = mid;
-    }
-    return lo;
-}
-
-struct BandPlan {
-    bool entropy;
-    double evals_tile;  /* evaluations per tile                              */
-    double h;           /* chi-square coefficient per nat (chi2_slope)       */
-    double k;
-    double most;        /* survivors a band may have                         */
-    double factor = 1.0; /* survivors measured over survivors expected       */
-
-    /* Expected survivors per evaluation under the threshold that admits a
-     * share q: the filter's chi-square cut is h/2 of the quantile; Fisher's
-     * exact check of log10 P(obs) admits a few times the two-sided p.      */
-    double pass(double q) const {
-        q = std::min(q, 1.0);
-        return entropy ? chi2_tail(0.5 * h * chi2_quantile(q)) : std::min(1.0, 4.0 * q);
-    }
-    double survivors(int64_t tiles, double q) const {
-        return factor * (double)tiles * evals_tile * pass(q);
-    }
-    /* Tiles of the band that follows `done` tiles.  About 250,000 survivors
-     * cost what a band's fixed part does (100 us); at least three times what
-     * is done while the list holds them, at most that for Fisher and eight
-     * times for entropy (the pairs that pass the screen cost more under an
-     * older threshold).                                                     */
-    int64_t next(int64_t done, int64_t left) const {
-        const double q = 1.3 * k / ((double)done * evals_tile);
-        const double per = factor * evals_tile * pass(q);
-        const double cheap = std::min(std::max(250000.0 / per, 3.0 * (double)done),
-                                      (entropy ? 8.0 : 3.0) * (double)done);
-        const double tiles = std::min({cheap, most / per, 1048576.0, (double)left});
-        /* a remainder below a fifth of the band goes with it */
-        if ((double)left < 1.2 * tiles && (double)left * per < most) return left;
-        return std::max<int64_t>(1, (int64_t)tiles);
-    }
-};
-
 int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case,
              const gepi_params *par, gepi_result *tops, int64_t *n_tops,
              gepi_scan_stats *stats, bool noalloc) {
@@ -843,20 +772,11 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
     plan.h = (double)ca.h0 + (double)ca.h1 * std::min(n0, n1);
     plan.k = (double)k;
     plan.most = (double)pcap / 4;
-    const double guess = entropy ? GUESS_ENTROPY : GUESS_FISHER;
-    /* the share of n tiles' evaluations that the first threshold admits */
-    auto share = [&](int64_t n) { return guess * (double)k / ((double)n * evals_per_tile); };
-    /* the first band: a scan of up to about 5,000 variants whole; else a pilot
-     * of one tile per workgroup the chip holds, or more where that would
-     * admit more than 4e-5 (the filter's expensive branch in most waves)   */
-    int64_t first = n_tiles;
-    if (n_tiles > 6400 || plan.survivors(first, share(first)) > 600000.0)
-        first = std::min<int64_t>(n_tiles, std::max<int64_t>(1024, (int64_t)(share(1) / 4e-5)));
+    const int64_t first = plan.first(n_tiles);
     const bool hooks = forced_band || getenv("GEPI_CAND_CAP") || getenv("GEPI_PEND_CAP");
     const bool planned = fp4 && n_ks > 0 && !hooks && !par->intermediate && par->max_grid_area <= 0 &&
-                         share(first) <= 0.1 && 1.5 * (guess + 1.0) * (double)k <= (double)cap &&
-                         (guess + 1.0) * (double)k <= (double)WG_SELECT_MAX &&
-                         plan.survivors(first, share(first)) <= plan.most;
+                         plan.sound(first, cap) &&
+                         (plan.guess() + 1.0) * (double)k <= (double)WG_SELECT_MAX;
     if (planned) {
         if (!p->mail) HIP_TRY(hipHostMalloc(&p->mail, sizeof(HostMail), hipHostMallocDefault));
         HostMail *mail = static_cast<HostMail *>(p->mail);
@@ -865,9 +785,8 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
             HIP_TRY(hipEventCreate(&e));
             p->band_ev.push_back(e);
         }
-        const double q = share(first);
-        HIP_TRY(init_state(entropy ? -chi2_quantile(q) / (2.0 * (n0 + n1)) * 1.4426950408889634
-                                   : std::log10(q)));
+        const double q = plan.share(first);
+        HIP_TRY(init_state(plan.score(q, n0 + n1)));
         ea.cand = b.cand[0];
         struct Job {
             int64_t t0, t1;
@@ -915,8 +834,7 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
                 /* after the pilot: was its threshold sound, how many
                  * survivors did it have, and the other bands             */
                 if (redo.empty() && count < (unsigned long long)k / 4) break;
-                plan.factor = std::min(64.0, std::max(0.25, (double)mail->report[0].pend_count /
-                                                                std::max(1.0, plan.survivors(first, q))));
+                plan.learn(first, q, mail->report[0].pend_count);
                 for (; upto < n_tiles; upto = redo.back().t1)
                     redo.push_back(Job{upto, upto + plan.next(upto, n_tiles - upto)});
             }

@@ -263,8 +263,8 @@ typedef struct gepi_tune_class {
  * CU, or wave tiles; x 5e8, 2e9 or 8e9 evaluations per band), repeats times
  * each, and keeps the fastest (the default unless another is more than 3%
  * faster).  The default schedule: 2 persistent workgroups per CU, 2e9
- * evaluations per band, entropy scans of at least 48 K steps on wave tiles
- * and smaller ones on 64 x 32 tiles.  The engine uses the table from then
+ * evaluations per band, entropy scans of at least 48 K steps or about 1,000
+ * variants on wave tiles and smaller ones on 64 x 32 tiles.  The engine uses the table from then
  * on: a scan's job shape and band size by its class, a round's launch form
  * by the class with the most count work in it.  A table that differs from
  * the default is kept only if it is also 1% faster on all 16 trial scans
