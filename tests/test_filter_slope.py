@@ -65,3 +65,20 @@ def test_fisher_probability_above_bound():
             k = int(k)
             lb = n * H(k / n) + 0.5 * math.log(n / (8.0 * k * (n - k)))
             assert lchoose(n, k) >= lb - 1e-9 * max(1.0, lb), (n, k)
+
+
+def test_float_information_within_margin():
+    """entropy_admits: float32 sums of t log2 t within 8e-6 m log2 m (+ 1e-6)
+    of the exact -I m."""
+    f = np.float32
+    rng = np.random.default_rng(13)
+
+    def t(v):
+        return f(0) if v == 0 else f(f(v) * np.log2(f(v)))
+
+    for w, x, y, z in list(all_small_tables(9)) + list(tables(rng, 20000, 20000)):
+        m = y + z
+        s = f(f(f(t(y) + t(z)) - t(m)) + f(t(w + x) + t(m - w - x))) - \
+            f(f(t(w) + t(y - w)) + f(t(x) + t(z - x)))
+        exact = -m * mi_nats(w, x, y, z) / math.log(2.0)
+        assert abs(float(s) - exact) <= 8e-6 * m * math.log2(max(m, 1)) + 1e-6, (w, x, y, z)
