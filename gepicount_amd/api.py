@@ -239,7 +239,12 @@ def score_table(w, x, y, z, ffun=GEPI_FFUNC_ENTROPY):
 
 def _result_buffer(topmost, n_rows):
     total = 5 * (n_rows * (n_rows + 1) // 2)
-    return np.zeros(max(1, min(int(topmost), total)), dtype=RESULT_DTYPE)
+    return np.empty(max(1, min(int(topmost), total)), dtype=RESULT_DTYPE)
+
+
+def _filled(out, n):
+    """The first n records of a result buffer: itself when it is full."""
+    return out if n == len(out) else out[:n].copy()
 
 
 def _masks(mask_ctrl, mask_case, words):
@@ -267,7 +272,7 @@ def process_gpu_1(bit_data, valid_data, mask_ctrl, mask_case, n_samples, topmost
     _check(lib().gepi_process_gpu_1(_u64p(b), _u64p(v), _u64p(m0), _u64p(m1), R, int(n_samples),
                                     ctypes.byref(par), out.ctypes.data, ctypes.byref(n),
                                     ctypes.byref(st)))
-    return out[:n.value].copy(), st.as_dict()
+    return _filled(out, n.value), st.as_dict()
 
 
 class Panel:
@@ -308,7 +313,7 @@ class Panel:
         st = ScanStats()
         _check(lib().gepi_scan(self._h, _u64p(m0), _u64p(m1), ctypes.byref(par),
                                out.ctypes.data, ctypes.byref(n), ctypes.byref(st)))
-        return out[:n.value].copy(), st.as_dict()
+        return _filled(out, n.value), st.as_dict()
 
     def scan_noalloc(self, mask_ctrl, mask_case, topmost=1000000, ffun=GEPI_FFUNC_ENTROPY,
                      count_path=0):
@@ -321,7 +326,7 @@ class Panel:
         st = ScanStats()
         _check(lib().gepi_scan_noalloc(self._h, _u64p(m0), _u64p(m1), ctypes.byref(par),
                                        out.ctypes.data, ctypes.byref(n), ctypes.byref(st)))
-        return out[:n.value].copy(), st.as_dict()
+        return _filled(out, n.value), st.as_dict()
 
     def qa(self, max_miss_snps=0.05, max_miss_samples=0.05):
         """Missing calls per variant and per sample, and how many exceed the
@@ -406,7 +411,7 @@ class Engine:
         res = []
         for i in range(n):
             out = keep[i][2]
-            res.append((out[:arr[i].n_tops].copy(), arr[i].stats.as_dict(), int(arr[i].status)))
+            res.append((_filled(out, arr[i].n_tops), arr[i].stats.as_dict(), int(arr[i].status)))
         return res, bs.as_dict()
 
     def autotune(self, repeats=2):
@@ -499,7 +504,7 @@ class Server:
         st = ScanStats()
         rc = lib().gepi_server_wait(self._h, ctypes.c_uint64(t), out.ctypes.data, len(out),
                                     ctypes.byref(n), ctypes.byref(st))
-        return out[:n.value].copy(), st.as_dict(), int(rc)
+        return _filled(out, n.value), st.as_dict(), int(rc)
 
     def stats(self):
         st = ServerStats()

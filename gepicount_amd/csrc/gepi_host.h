@@ -195,6 +195,7 @@ inline void screen_consts(int32_t n0, int32_t n1, gepi::CountArgs &g) {
  * 256 0.73 -> 0.13 ms (5 bands -> 1), 3,001 x 777 Fisher 1.44 -> 0.29, 20,000
  * x 2,048 3.69 -> 2.38 (10 -> 3), 8,000 x 20,001 3.84 -> 2.50.               */
 constexpr double GUESS_ENTROPY = 8.0, GUESS_FISHER = 16.0;
+constexpr double LOOP_GUESS_ENTROPY = 2.0, LOOP_GUESS_FISHER = 4.0; /* long rankings */
 
 /* P(chi2_1 > t) and its inverse */
 inline double chi2_tail(double t) { return std::erfc(std::sqrt(0.5 * std::max(t, 0.0))); }
@@ -213,11 +214,13 @@ struct BandPlan {
     double h;           /* chi-square coefficient per nat (chi2_slope)       */
     double k;
     double most;        /* survivors a band may have                         */
+    double c;           /* GUESS or LOOP_GUESS of the objective              */
     double factor = 1.0; /* survivors measured over survivors expected       */
 
-    /* Expected survivors per evaluation under the threshold that admits a
-     * share q: the filter's chi-square cut is h/2 of the quantile; Fisher's
-     * exact check of log10 P(obs) admits a few times the two-sided p.      */
+    /* Expected survivors of the chi-square bound per evaluation under the
+     * threshold that admits a share q: its cut is h/2 of the quantile (a few
+     * times fewer become records); Fisher's exact check of log10 P(obs)
+     * admits a few times the two-sided p.                                   */
     double pass(double q) const {
         q = std::min(q, 1.0);
         return entropy ? chi2_tail(0.5 * h * chi2_quantile(q)) : std::min(1.0, 4.0 * q);
@@ -225,9 +228,8 @@ struct BandPlan {
     double survivors(int64_t tiles, double q) const {
         return factor * (double)tiles * evals_tile * pass(q);
     }
-    double guess() const { return entropy ? GUESS_ENTROPY : GUESS_FISHER; }
     /* the share of n tiles' evaluations that the first threshold admits */
-    double share(int64_t n) const { return guess() * k / ((double)n * evals_tile); }
+    double share(int64_t n) const { return c * k / ((double)n * evals_tile); }
     /* the score that a share q of unassociated evaluations reaches */
     double score(double q, int32_t n) const {
         return entropy ? -chi2_quantile(q) / (2.0 * n) * 1.4426950408889634 : std::log10(q);
@@ -241,7 +243,7 @@ struct BandPlan {
     }
     /* whether a guess for n tiles tells anything and the lists hold it */
     bool sound(int64_t n, unsigned long long cap) const {
-        return share(n) <= 0.1 && 1.5 * (guess() + 1.0) * k <= (double)cap &&
+        return share(n) <= 0.1 && 1.5 * (c + 1.0) * k <= (double)cap &&
                survivors(n, share(n)) <= most;
     }
     void learn(int64_t n, double q, unsigned long long found) {
@@ -264,16 +266,10 @@ struct BandPlan {
     }
 };
 
-/* Sorts candidate records by the canonical key and writes the first
- * min(k, size) as results; returns how many were written.                   */
-inline int64_t candidates_to_results(std::vector<gepi::Cand> &host, int64_t k, gepi_result *tops) {
-    std::sort(host.begin(), host.end(), [](const gepi::Cand &a, const gepi::Cand &b) {
-        const uint64_t ha = gepi::order_bits(a.score), hb = gepi::order_bits(b.score);
-        return ha < hb || (ha == hb && a.idx < b.idx);
-    });
-    const int64_t n = std::min<int64_t>((int64_t)host.size(), k);
+/* The first n records as results. */
+inline int64_t results_of(const gepi::Cand *rec, int64_t n, gepi_result *tops) {
     for (int64_t i = 0; i < n; i++) {
-        const gepi::Cand &c = host[(size_t)i];
+        const gepi::Cand &c = rec[i];
         gepi_result &r = tops[i];
         r.sA = (int64_t)(c.idx >> 32);
         r.sB = (int64_t)((c.idx >> 3) & 0x1FFFFFFFull);
@@ -286,6 +282,16 @@ inline int64_t candidates_to_results(std::vector<gepi::Cand> &host, int64_t k, g
         r.reserved = 0;
     }
     return n;
+}
+
+/* Sorts candidate records by the canonical key and writes the first
+ * min(k, size) as results; returns how many were written.                   */
+inline int64_t candidates_to_results(std::vector<gepi::Cand> &host, int64_t k, gepi_result *tops) {
+    std::sort(host.begin(), host.end(), [](const gepi::Cand &a, const gepi::Cand &b) {
+        const uint64_t ha = gepi::order_bits(a.score), hb = gepi::order_bits(b.score);
+        return ha < hb || (ha == hb && a.idx < b.idx);
+    });
+    return results_of(host.data(), std::min<int64_t>((int64_t)host.size(), k), tops);
 }
 
 /* Class compression words of a scan: [2][2 * w64], class 0 then class 1;

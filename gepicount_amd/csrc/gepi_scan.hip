@@ -42,6 +42,7 @@
 #include "gepi_count.h"
 #include "gepi_internal.h"
 #include "gepi_score.h"
+#include "gepi_sort.h"
 #include "gepi_stage.h"
 #include "gepi_topk.h"
 #include "gepi_host.h"
@@ -339,6 +340,9 @@ int bind_scratch(gepi_panel *p, ScanBufs &b, int32_t tmax, size_t cw_bytes, size
  * numbering k_topk_one does not know (it drops overflowed bands by fp4
  * tiles).                                                                  */
 constexpr unsigned long long WG_SELECT_MAX = 1ull << 18;
+/* Rankings up to this length are sorted on the host (0.3 ms), longer ones on
+ * the device: 1,000,000 records 82 ms there, 0.3 here.                      */
+constexpr int64_t SORT_HOST_MAX = 4096;
 inline bool wg_select(int path, unsigned long long count) {
     return (path == 3 || path == 4) && count <= WG_SELECT_MAX;
 }
@@ -771,12 +775,13 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
     plan.evals_tile = (double)evals_per_tile;
     plan.h = (double)ca.h0 + (double)ca.h1 * std::min(n0, n1);
     plan.k = (double)k;
+    plan.c = entropy ? GUESS_ENTROPY : GUESS_FISHER;
     plan.most = (double)pcap / 4;
     const int64_t first = plan.first(n_tiles);
     const bool hooks = forced_band || getenv("GEPI_CAND_CAP") || getenv("GEPI_PEND_CAP");
     const bool planned = fp4 && n_ks > 0 && !hooks && !par->intermediate && par->max_grid_area <= 0 &&
                          plan.sound(first, cap) &&
-                         (plan.guess() + 1.0) * (double)k <= (double)WG_SELECT_MAX;
+                         (plan.c + 1.0) * (double)k <= (double)WG_SELECT_MAX;
     if (planned) {
         if (!p->mail) HIP_TRY(hipHostMalloc(&p->mail, sizeof(HostMail), hipHostMallocDefault));
         HostMail *mail = static_cast<HostMail *>(p->mail);
@@ -841,10 +846,10 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
             redo.insert(redo.end(), jobs.begin() + nj, jobs.end());
             jobs.swap(redo);
             if (jobs.empty() && count == (unsigned long long)k) {
-                host.resize((size_t)k);
+                if (k <= SORT_HOST_MAX) host.resize((size_t)k);
                 if (by_mail)
                     memcpy(host.data(), mail->rec, sizeof(Cand) * (size_t)k);
-                else
+                else if (k <= SORT_HOST_MAX)
                     HIP_TRY(hipMemcpyAsync(host.data(), b.cand[0], sizeof(Cand) * k,
                                            hipMemcpyDeviceToHost, p->stream));
                 HIP_TRY(hipStreamSynchronize(p->stream));
@@ -861,21 +866,40 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
     } else {
         t0 = n_tiles;
     }
-    /* the second candidate list, where the multi-launch selection compacts
-     * from one into the other: allocated when it first runs */
-    auto second_list = [&]() -> int {
-        if (b.cand[1]) return GEPI_OK;
-        if (cap > p->buf2_cap) {
+    /* the second candidate list (n records), where the multi-launch selection
+     * compacts from one into the other, or the ranking is sorted: allocated
+     * when it is first needed */
+    auto second_list = [&](unsigned long long n) -> int {
+        if (noalloc) return GEPI_OK;
+        if (n > p->buf2_cap) {
             hipFree(p->d_cand[1]);
             p->d_cand[1] = nullptr;
             p->buf2_cap = 0;
-            HIP_TRY(hipMalloc(&p->d_cand[1], sizeof(Cand) * cap));
-            p->buf2_cap = cap;
-            st_local.bytes_allocated += (int64_t)(sizeof(Cand) * cap);
+            HIP_TRY(hipMalloc(&p->d_cand[1], sizeof(Cand) * n));
+            p->buf2_cap = n;
+            st_local.bytes_allocated += (int64_t)(sizeof(Cand) * n);
         }
         b.cand[1] = p->d_cand[1];
         return GEPI_OK;
     };
+    /* long rankings: a first band under a guessed threshold as well, where
+     * 1/50 of its evaluations would hold LOOP_GUESS times k (nearly all of a
+     * first band's become records without one: top-1,000,000 of 20,000 x 2,048
+     * 10 bands and 16.2M records then, 6 and 9.5M now).  If that was too
+     * strict the count stays below k, the following bands keep the threshold,
+     * and only a scan that ends so runs again without it                    */
+    bool loop_guess = false;
+    if (!planned && !hooks && !par->intermediate && par->max_grid_area <= 0 && n_ks > 0) {
+        plan.factor = 1.0;
+        plan.c = entropy ? LOOP_GUESS_ENTROPY : LOOP_GUESS_FISHER;
+        plan.most = std::min((double)pcap, (double)cap - (double)k) / 2;
+        const int64_t one = std::max<int64_t>(1, (int64_t)(plan.share(1) / 0.02));
+        if (one <= n_tiles / 4 && plan.survivors(one, plan.share(one)) <= 2.0 * plan.most) {
+            loop_guess = true;
+            HIP_TRY(init_state(plan.score(plan.share(one), n0 + n1)));
+            band = one;
+        }
+    }
     while (t0 < n_tiles) {
         const int64_t t1 = std::min<int64_t>(n_tiles, t0 + band);
         ea.cand = b.cand[cur];
@@ -914,7 +938,7 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
                 hs.count = kept;
                 hs.overflow = 0;
                 HIP_TRY(hipMemcpyAsync(b.state, &hs, sizeof hs, hipMemcpyHostToDevice, p->stream));
-                if ((rc = second_list()) != GEPI_OK) return rc;
+                if ((rc = second_list(cap)) != GEPI_OK) return rc;
                 launch_select(p, b, b.cand[cur], (uint32_t)k, kept);
                 k_compact<<<4096, 256, 0, p->stream>>>(b.cand[cur], b.state, b.cand[cur ^ 1],
                                                        t0, t1, tv, fp4 ? (int32_t)n_a4 : 0);
@@ -934,7 +958,7 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
             if (wg_select(path, hs.count)) {
                 k_topk_one<<<1, TOPK_THREADS, 0, p->stream>>>(topk_desc(b, cur, cap, k, par, 0, 0, n_a4));
             } else {
-                if ((rc = second_list()) != GEPI_OK) return rc;
+                if ((rc = second_list(cap)) != GEPI_OK) return rc;
                 launch_select(p, b, b.cand[cur], (uint32_t)k, hs.count);
                 k_compact<<<4096, 256, 0, p->stream>>>(b.cand[cur], b.state, b.cand[cur ^ 1],
                                                        0, 0, tv, fp4 ? (int32_t)n_a4 : 0);
@@ -955,6 +979,15 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
         band = std::max<int64_t>(1, std::min<int64_t>({max_band, next, band * 4}));
         if (forced_band) band = std::min<int64_t>(forced_band, (t1 - t0) * 4);
         t0 = t1;
+        if (loop_guess && t0 < n_tiles && count == (unsigned long long)k)
+            band = std::max<int64_t>(band, plan.next(t0, n_tiles - t0));
+        if (loop_guess && t0 >= n_tiles && count < (unsigned long long)k) {
+            loop_guess = false;
+            HIP_TRY(init_state(INFINITY));
+            count = exact_total = 0;
+            t0 = 0;
+            band = std::max<int64_t>(1, std::min<int64_t>(max_band, (2 * k) / evals_per_tile + 1));
+        }
         if (par->intermediate && g_progress_fn) {
             /* the records held so far, sorted, for the caller's report */
             std::vector<Cand> held((size_t)count);
@@ -975,16 +1008,45 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
             g_progress_fn(&pg, g_progress_user);
         }
     }
-    /* final extraction: exactly k records, sorted by key on the host */
+    /* final extraction: exactly k records, sorted by key */
     auto ts = std::chrono::steady_clock::now();
-    if (!finished) {
-        host.resize((size_t)count);
-        if (count > 0)
-            HIP_TRY(hipMemcpyAsync(host.data(), b.cand[cur], sizeof(Cand) * count,
-                                   hipMemcpyDeviceToHost, p->stream));
-        HIP_TRY(hipStreamSynchronize(p->stream));
+    int64_t n = 0;
+    if (k > SORT_HOST_MAX && count == (unsigned long long)k) {
+        if ((rc = second_list((unsigned long long)k)) != GEPI_OK) return rc;
+        const unsigned blocks = (unsigned)((k + SORT_TILE - 1) / SORT_TILE);
+        Cand *from = b.cand[cur], *to = b.cand[cur ^ 1];
+        k_sort_tiles<<<blocks, SORT_THREADS, 0, p->stream>>>(from, to, k);
+        for (int64_t run = SORT_TILE; run < k; run *= 2) {
+            std::swap(from, to);
+            k_merge<<<blocks, SORT_THREADS, 0, p->stream>>>(from, to, k, run);
+        }
+        HIP_TRY(hipGetLastError());
+        if (sizeof(gepi_result) * (size_t)k <= sizeof(Pend) * (size_t)pcap) {
+            /* the pending list has done its work: results are written there */
+            gepi_result *d_res = reinterpret_cast<gepi_result *>(b.pend);
+            k_results<<<(unsigned)((k + 255) / 256), 256, 0, p->stream>>>(to, d_res, k);
+            HIP_TRY(hipGetLastError());
+            HIP_TRY(hipMemcpyAsync(tops, d_res, sizeof(gepi_result) * (size_t)k, hipMemcpyDeviceToHost,
+                                   p->stream));
+            HIP_TRY(hipStreamSynchronize(p->stream));
+            n = k;
+        } else {
+            host.resize((size_t)k);
+            HIP_TRY(hipMemcpyAsync(host.data(), to, sizeof(Cand) * (size_t)k, hipMemcpyDeviceToHost,
+                                   p->stream));
+            HIP_TRY(hipStreamSynchronize(p->stream));
+            n = results_of(host.data(), k, tops);
+        }
+    } else {
+        if (!finished) {
+            host.resize((size_t)count);
+            if (count > 0)
+                HIP_TRY(hipMemcpyAsync(host.data(), b.cand[cur], sizeof(Cand) * count,
+                                       hipMemcpyDeviceToHost, p->stream));
+            HIP_TRY(hipStreamSynchronize(p->stream));
+        }
+        n = candidates_to_results(host, k, tops);
     }
-    const int64_t n = candidates_to_results(host, k, tops);
     *n_tops = n;
     ms_top += ms_since(ts);
     st_local.ms_count_kernels = ms_count;
