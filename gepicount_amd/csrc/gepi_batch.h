@@ -161,6 +161,13 @@ k_count_f4g_batch(const BatchDesc *__restrict__ d, BatchMap map) {
     count_f4g_unit<FFUN>(g, j.tile - g.tile_begin, sh);
 }
 
+/* The pairs put off by k_count_f4g_batch (pairs_run); blockIdx.y = scan. */
+template <int FFUN>
+__global__ void __launch_bounds__(PAIRS_THREADS) k_pairs_batch(const BatchDesc *__restrict__ d) {
+    const CountArgs g = d[blockIdx.y].g;
+    pairs_run<FFUN>(g, blockIdx.x, gridDim.x);
+}
+
 /* p[0..n) = v (one workgroup of 64 threads per 64 words). */
 __global__ void __launch_bounds__(64) k_fill_u32(uint32_t *p, int32_t n, uint32_t v) {
     const int32_t i = (int32_t)(blockIdx.x * 64 + threadIdx.x);

@@ -27,6 +27,7 @@ namespace {
 
 constexpr int64_t F4_TILE_EVALS = (int64_t)TM * TB4 * 20;
 constexpr int EXACT_BLOCKS_X = 64; /* blocks per scan of the batched exact pass */
+constexpr int PAIRS_BLOCKS_X = 256; /* the same of the pairs put off            */
 
 /* Job shape of an entropy scan with ks K steps under the default schedule:
  * wave tiles from 48 K steps, whole tiles below.  Measured on the MI355X
@@ -466,18 +467,21 @@ size_t Engine::estimate_footprint(const gepi_panel *p, int64_t topmost) {
     const unsigned long long pcap = std::max<unsigned long long>(cap, 1ull << 20);
     return round_block((size_t)n_u * n_var_pad * 3 * 64 + (size_t)n_var_pad * sizeof(float)) + round_block(cap * sizeof(Cand)) +
            round_block(pcap * sizeof(Pend)) + round_block((size_t)4 * p->w64 * sizeof(CompressWord)) +
-           round_block(sizeof(ScanState));
+           round_block(sizeof(ScanState)) +
+           round_block((size_t)pair_list_cap(n_var_pad / TM * (n_var_pad / TM + 1), 0, PAIRS_MOST_BATCH) * 48);
 }
 
 void Engine::drop(ScanItem *it, int status) {
     dfree(it->d_layout);
     dfree(it->d_cw);
     dfree(it->d_pend);
+    dfree(it->d_pairs);
     dfree(it->d_cand);
     dfree(it->d_state);
     it->d_layout = nullptr;
     it->d_cw = nullptr;
     it->d_pend = nullptr;
+    it->d_pairs = nullptr;
     it->d_cand = nullptr;
     it->d_state = nullptr;
     it->footprint = 0;
@@ -581,14 +585,17 @@ int Engine::add(ScanItem *it) {
     it->d_pend = (Pend *)dalloc(it->pcap * sizeof(Pend));
     it->d_cand = (Cand *)dalloc(it->cap * sizeof(Cand));
     it->d_state = (ScanState *)dalloc(sizeof(ScanState));
-    if (!it->d_layout || !it->d_cw || !it->d_pend || !it->d_cand || !it->d_state) {
+    it->pair_cap = it->geno ? pair_list_cap(it->n_tiles, it->n_k4, PAIRS_MOST_BATCH) : 0u;
+    if (it->pair_cap) it->d_pairs = (uint4 *)dalloc((size_t)it->pair_cap * 48);
+    if (!it->d_layout || !it->d_cw || !it->d_pend || (it->pair_cap && !it->d_pairs) || !it->d_cand || !it->d_state) {
         drop(it, gepi_fail(GEPI_ERR_NOMEM, "device memory for a scan of %lld variants",
                            (long long)it->n_var));
         return it->status;
     }
     it->footprint = round_block(lay) + round_block(it->h_cw.size() * sizeof(CompressWord)) +
                     round_block(it->pcap * sizeof(Pend)) + round_block(it->cap * sizeof(Cand)) +
-                    round_block(sizeof(ScanState));
+                    round_block(sizeof(ScanState)) +
+                    (it->pair_cap ? round_block((size_t)it->pair_cap * 48) : 0);
     HIP_TRY(hipMemcpyAsync(it->d_cw, it->h_cw.data(), it->h_cw.size() * sizeof(CompressWord),
                            hipMemcpyHostToDevice, stream));
     if (it->geno) {
@@ -783,6 +790,8 @@ int Engine::round(std::vector<ScanItem *> &finished) {
             d.g.st = it->d_state;
             d.g.pend = it->d_pend;
             d.g.pcap = it->pcap;
+            d.g.pairs = it->d_pairs;
+            d.g.pair_cap = it->pair_cap;
             d.g.lfact = tabs_.lfact;
             if (f == 5) {
                 d.g.park = d_park_;
@@ -869,6 +878,12 @@ int Engine::round(std::vector<ScanItem *> &finished) {
             }
             launch_count(f, per_cu > 0, grid, m);
         }
+        if (!bd[6].empty())
+            k_pairs_batch<GEPI_FFUNC_ENTROPY><<<dim3(PAIRS_BLOCKS_X, (unsigned)bd[6].size()), PAIRS_THREADS,
+                                                0, stream>>>(d_bdesc_[6]);
+        if (!bd[7].empty())
+            k_pairs_batch<GEPI_FFUNC_FISHERPV><<<dim3(PAIRS_BLOCKS_X, (unsigned)bd[7].size()), PAIRS_THREADS,
+                                                 0, stream>>>(d_bdesc_[7]);
         HIP_TRY(hipGetLastError());
         HIP_TRY(hipEventRecord(ev1_, stream));
         k_exact_batch<<<dim3(EXACT_BLOCKS_X, (unsigned)na), 256, 0, stream>>>(d_edesc_);

@@ -1199,21 +1199,28 @@ __device__ __forceinline__ void count_f4w_unit(const CountArgs &g, int64_t unit,
  * near as the single evaluations' chi-square.
  *
  * The screen costs about 95 VALU instructions per pair against 200 for the
- * 20 tests, and passes one pair in 100 to 1,000 once the threshold has
- * settled (per workgroup at 20,000 x 2,048: products 25.0 ns, screen 7.2, the
- * collected pairs 6.7; the kernel with the tests in the lanes 42.8).  Those are collected in LDS (their totals; the class-0 counts are
- * there already) and tested one per thread of the workgroup by the int32
- * filter, so the expensive code runs on full waves and exists once.
+ * 20 tests, and passes one pair in 30 to 200 (Fisher one in 10 to 30).  Those
+ * are collected in LDS (their totals; the class-0 counts are there already).
+ * Tested there, one per thread, they cost a workgroup the latency of one test
+ * (some 20 us, as long as a short K loop: at 20,000 x 2,048 the kernel took 973
+ * us in the last band, 818 without the tests, 611 without the screen too), so
+ * short scans copy them to a list of 48-byte records for a launch of their own
+ * with full waves (k_pairs: 4.2M pairs 105 us): 20,000 x 2,048 2.00 -> 1.80 ms,
+ * Fisher 2.92 -> 2.51, 30,001 x 3,001 4.95 -> 4.79; long ones, and what finds
+ * that list full, test them with the int32 filter in the kernel
+ * (pair_list_cap).
  * Accumulators start at g.sc_start, the largest fraction no count rounds
  * away, so that an empty cell divides 0 by it; g.sc_sub takes its effect off
  * the right side (a cell loses at most 2 (1 + 2k) times it).               */
 constexpr int F4G_LIST = 256;  /* pairs collected per workgroup               */
 constexpr int F4G_STAGE = 112; /* survivors staged per workgroup              */
+constexpr int PAIRS_THREADS = 256;
 struct F4GShared {
     uint32_t c0lds[4][F4W_PARK * 64];
     uint32_t list[F4G_LIST * 5]; /* 9 totals of 16 bits, then wave, lane, e   */
     PendStageN<F4G_STAGE> stage;
     uint32_t n;
+    unsigned long long base; /* the list's place in the scan's               */
 };
 static_assert(sizeof(F4GShared) <= 81920, "two workgroups per CU");
 
@@ -1247,23 +1254,26 @@ __device__ __forceinline__ void f4g_append(uint32_t *L, const float (&T)[9], uin
     L[4] = u[8] | (id << 16);
 }
 
-/* Tests a collected pair with the int32 filter.  unit: the workgroup's. */
-template <int FFUN>
-__device__ __forceinline__ void f4g_test(const CountArgs &g, F4GShared &sh, const FilterConsts &fc,
-                                         const uint32_t *L, int64_t unit) {
-    uint32_t r[5];
-#pragma unroll
-    for (int i = 0; i < 5; i++) r[i] = L[i];
-    const uint32_t id = r[4] >> 16, e = id & 15u, src = (id >> 4) & 63u, wv = id >> 10;
-    const uint16_t *c0 = reinterpret_cast<const uint16_t *>(sh.c0lds[wv]) + (e >> 1) * (9 * 128) +
-                         src * 2 + (e & 1);
-    int32_t x[2][3][3]; /* cells by class */
-#pragma unroll
-    for (int i = 0; i < 9; i++) {
-        const int32_t t = (int32_t)((r[i >> 1] >> (16 * (i & 1))) & 0xFFFFu);
-        x[0][i / 3][i % 3] = c0[i * 128];
-        x[1][i / 3][i % 3] = t - x[0][i / 3][i % 3];
-    }
+/* A pair's cells by class from its totals (9 halfwords from dword 0 of r, the
+ * id in the last) and class-0 counts.                                      */
+__device__ __forceinline__ int32_t f4g_total(const uint32_t (&r)[5], int i) {
+    return (int32_t)((r[i >> 1] >> (16 * (i & 1))) & 0xFFFFu);
+}
+
+/* The variants of a collected pair in its tile; id as f4g_append wrote it. */
+__device__ __forceinline__ void f4g_variants(uint32_t id, int64_t tile, int32_t n_a, int32_t &A,
+                                             int32_t &B) {
+    const int32_t e = (int32_t)(id & 15u), src = (int32_t)((id >> 4) & 63u), wv = (int32_t)(id >> 10);
+    int32_t ta, tb;
+    tile_of_f4(tile, n_a, ta, tb);
+    A = (2 * ta + (wv & 1)) * 32 + 4 * (src >> 5) + 8 * (e >> 2) + (e & 3);
+    B = tb * 32 + (src & 31);
+}
+
+/* The int32 filter on a pair's cells. */
+template <int FFUN, bool ROLLED, class PS>
+__device__ __forceinline__ void f4g_filter(const CountArgs &g, PS &ps, const FilterConsts &fc,
+                                           const int32_t (&x)[2][3][3], int32_t A, int32_t B) {
     int32_t c[2][3][3]; /* products of the allele and valid planes */
 #pragma unroll
     for (int k = 0; k < 2; k++) {
@@ -1281,12 +1291,69 @@ __device__ __forceinline__ void f4g_test(const CountArgs &g, F4GShared &sh, cons
             c[k][2][q] = c[k][0][q] + u[2][q];
         }
     }
-    int32_t ta, tb;
-    tile_of_f4(g.tile_begin + 2 * unit + (wv >> 1), g.n_var_pad / TM, ta, tb);
-    const int32_t A = (2 * ta + (int32_t)(wv & 1u)) * 32 + 4 * (int32_t)(src >> 5) +
-                      8 * (int32_t)(e >> 2) + (int32_t)(e & 3u);
-    const int32_t B = tb * 32 + (int32_t)(src & 31u);
-    filter_pair<FFUN, true>(g, sh.stage, fc, A, B, c);
+    filter_pair<FFUN, ROLLED>(g, ps, fc, A, B, c);
+}
+
+/* Collected pair L of the workgroup's unit: to place `at` of the scan's list
+ * for k_pairs while that has room, else tested here.  A record is the five
+ * dwords of the list, the nine class-0 counts and the tile.                */
+template <int FFUN>
+__device__ __forceinline__ void f4g_deal(const CountArgs &g, F4GShared &sh, const FilterConsts &fc,
+                                         const uint32_t *L, int64_t unit, unsigned long long at) {
+    uint32_t r[5];
+#pragma unroll
+    for (int i = 0; i < 5; i++) r[i] = L[i];
+    const uint32_t id = r[4] >> 16, e = id & 15u, src = (id >> 4) & 63u, wv = id >> 10;
+    const uint16_t *c0 = reinterpret_cast<const uint16_t *>(sh.c0lds[wv]) + (e >> 1) * (9 * 128) +
+                         src * 2 + (e & 1);
+    const int64_t tile = g.tile_begin + 2 * unit + (wv >> 1);
+    if (at < g.pair_cap) {
+        uint32_t h[9];
+#pragma unroll
+        for (int i = 0; i < 9; i++) h[i] = c0[i * 128];
+        uint4 *dst = g.pairs + at * 3;
+        dst[0] = make_uint4(r[0], r[1], r[2], r[3]);
+        dst[1] = make_uint4(r[4], h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16));
+        dst[2] = make_uint4(h[6] | (h[7] << 16), h[8], (uint32_t)tile, (uint32_t)(tile >> 32));
+        return;
+    }
+    int32_t x[2][3][3];
+#pragma unroll
+    for (int i = 0; i < 9; i++) {
+        x[0][i / 3][i % 3] = c0[i * 128];
+        x[1][i / 3][i % 3] = f4g_total(r, i) - x[0][i / 3][i % 3];
+    }
+    int32_t A, B;
+    f4g_variants(id, tile, g.n_var_pad / TM, A, B);
+    f4g_filter<FFUN, true>(g, sh.stage, fc, x, A, B);
+}
+
+/* The filter on the pairs that the count kernel of the band put off, one per
+ * thread, n_wg workgroups.  Called by every thread of a workgroup.         */
+template <int FFUN>
+__device__ __forceinline__ void pairs_run(const CountArgs &g, uint32_t wg, uint32_t n_wg) {
+    __shared__ PendStage stage;
+    const unsigned long long put = g.st->pair_count;
+    const uint32_t n = put < g.pair_cap ? (uint32_t)put : g.pair_cap;
+    if (wg * blockDim.x >= n) return; /* uniform over the workgroup */
+    stage_init(stage);
+    const FilterConsts fc = filter_consts(g.st, g);
+    __syncthreads();
+    for (uint32_t i = wg * blockDim.x + threadIdx.x; i < n; i += n_wg * blockDim.x) {
+        const uint4 a = g.pairs[(uint64_t)i * 3], b = g.pairs[(uint64_t)i * 3 + 1],
+                    d = g.pairs[(uint64_t)i * 3 + 2];
+        const uint32_t r[5] = {a.x, a.y, a.z, a.w, b.x}, h[5] = {b.y, b.z, b.w, d.x, d.y};
+        int32_t x[2][3][3];
+#pragma unroll
+        for (int k = 0; k < 9; k++) {
+            x[0][k / 3][k % 3] = f4g_total(h, k);
+            x[1][k / 3][k % 3] = f4g_total(r, k) - x[0][k / 3][k % 3];
+        }
+        int32_t A, B;
+        f4g_variants(r[4] >> 16, (int64_t)((uint64_t)d.w << 32 | d.z), g.n_var_pad / TM, A, B);
+        f4g_filter<FFUN, false>(g, stage, fc, x, A, B);
+    }
+    stage_flush(g, stage);
 }
 
 template <int FFUN>
@@ -1360,8 +1427,13 @@ __device__ __forceinline__ void count_f4g_unit(const CountArgs &g, int64_t unit,
     __syncthreads(); /* the list and every wave's class-0 counts are written */
     while (true) {
         const uint32_t n = sh.n < (uint32_t)F4G_LIST ? sh.n : (uint32_t)F4G_LIST;
+        if (n > 0 && g.pair_cap > 0) {
+            if (threadIdx.x == 0) sh.base = st_add(&g.st->pair_count, (unsigned long long)n);
+            __syncthreads();
+        }
+        const unsigned long long base = g.pair_cap > 0 ? sh.base : 0ull;
         for (uint32_t i = threadIdx.x; i < n; i += F4W_THREADS)
-            f4g_test<FFUN>(g, sh, fc, sh.list + i * 5, unit);
+            f4g_deal<FFUN>(g, sh, fc, sh.list + i * 5, unit, base + i);
         if (!__syncthreads_or(pend != 0)) break;
         /* the list was full (loose thresholds): the next of the elements left
          * over.  e is uniform here, so the accumulators are read by register
@@ -1388,6 +1460,11 @@ __global__ void __launch_bounds__(F4W_THREADS) __attribute__((amdgpu_waves_per_e
 k_count_f4g(CountArgs g) {
     __shared__ F4GShared sh;
     count_f4g_unit<FFUN>(g, band_unit((g.n_tiles + 1) >> 1), sh);
+}
+
+template <int FFUN>
+__global__ void __launch_bounds__(PAIRS_THREADS) k_pairs(CountArgs g) {
+    pairs_run<FFUN>(g, blockIdx.x, gridDim.x);
 }
 
 template <int FFUN, bool F32, bool PARK>

@@ -49,6 +49,7 @@ struct ScanState {
     unsigned long long pend_count;
     uint32_t pend_overflow;
     uint32_t pad1;
+    unsigned long long pair_count; /* variant pairs put off in this band (k_pairs)  */
     /* radix select */
     uint64_t key_hi, key_lo;
     uint32_t bits_done, rank, matched, done, gather_n, pad0;
@@ -88,6 +89,9 @@ struct CountArgs {
     float sc_p, sc_k, sc_q, sc_m, sc_start, sc_sub;
     float h0, h1;             /* chi-square coefficient per nat: h0 + h1 min(y, z)
                                * (chi2_slope)                                     */
+    uint4 *pairs;             /* pairs that passed the screen, for k_pairs: 3 uint4
+                               * each; null with pair_cap 0                       */
+    uint32_t pair_cap;
     ScanState *st;
     Pend *pend;
     unsigned long long pcap;

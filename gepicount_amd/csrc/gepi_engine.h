@@ -62,6 +62,8 @@ struct ScanItem {
     uint4 *d_layout = nullptr;
     gepi::CompressWord *d_cw = nullptr;
     gepi::Pend *d_pend = nullptr;
+    uint4 *d_pairs = nullptr; /* genotype planes: the pairs put off           */
+    uint32_t pair_cap = 0;
     gepi::Cand *d_cand = nullptr;
     gepi::ScanState *d_state = nullptr;
     size_t footprint = 0; /* device bytes held */

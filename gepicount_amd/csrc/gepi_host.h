@@ -67,6 +67,8 @@ struct gepi_panel {
     size_t park_bytes = 0;
     gepi::Cand *d_cand[2] = {nullptr, nullptr};
     gepi::Pend *d_pend = nullptr;
+    uint4 *d_pairs = nullptr;          /* pairs put off by the count kernel   */
+    size_t pairs_bytes = 0;
     unsigned long long buf_cap = 0;  /* records in the candidate buffer  */
     unsigned long long buf2_cap = 0; /* records in the second one        */
     unsigned long long pend_cap = 0; /* records in the pending list       */
@@ -169,6 +171,22 @@ inline void screen_consts(int32_t n0, int32_t n1, gepi::CountArgs &g) {
     const double start = std::ldexp(1.0, -std::min(24 - bits, 12));
     g.sc_start = (float)start;
     g.sc_sub = (float)(18.0 * start * (1.0 + 2.0 * k) + 1e-3);
+}
+
+/* Records of the list of pairs that the count kernel puts off (48 bytes): one
+ * for every 4 pairs of the scan, at most `most`, beyond which the kernel tests
+ * its pairs itself.  None from PAIRS_MAX_KSTEPS K steps on, where the other
+ * workgroup of the CU fills the time of a test with its longer K loop: whole
+ * scans of 20,000 variants, top-1,000, against tests in the kernel, took 0.90x
+ * the time with 256 samples (Fisher 0.88x), 0.90x (0.89x) with 1,024, 0.92x
+ * (0.92x) with 2,048, 0.98x (0.95x) with 4,096 and 1.00x (0.98x) with 8,192.  */
+constexpr int PAIRS_WG_PER_CU = 8;
+constexpr int64_t PAIRS_MOST = 1 << 22;       /* single scans: 201 MB          */
+constexpr int64_t PAIRS_MOST_BATCH = 1 << 21; /* a scan of the engine: 101 MB  */
+constexpr int32_t PAIRS_MAX_KSTEPS = 48;
+inline uint32_t pair_list_cap(int64_t n_tiles, int32_t ks, int64_t most) {
+    if (ks > PAIRS_MAX_KSTEPS) return 0;
+    return (uint32_t)std::min<int64_t>(std::max<int64_t>(n_tiles * (64 * 32 / 4), 4096), most);
 }
 
 /* ---- planned bands --------------------------------------------------------

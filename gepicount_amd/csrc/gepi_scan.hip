@@ -181,6 +181,7 @@ void panel_free(gepi_panel *p) {
     hipFree(p->d_cand[0]);
     hipFree(p->d_cand[1]);
     hipFree(p->d_pend);
+    hipFree(p->d_pairs);
     hipFree(p->d_state);
     hipFree(p->d_small);
     hipFree(p->tabs.lhi);
@@ -529,6 +530,7 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
         pcap = std::max<unsigned long long>((unsigned long long)std::max(atoll(env), 0ll),
                                             (unsigned long long)TILE_EVALS_MAX + 1024);
     }
+    const uint32_t pair_cap = geno && !noalloc ? pair_list_cap(n_tiles, n_ks, PAIRS_MOST) : 0u;
     ScanBufs b;
     if (noalloc) {
         /* the smallest lists that always complete: more, smaller bands */
@@ -559,6 +561,9 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
         if (fp4) grown(p->d_cw, p->cw_bytes, cw.size() * sizeof(CompressWord));
         if (fp4 &&
             (rc = grow(&p->d_cw, &p->cw_bytes, cw.size() * sizeof(CompressWord))) != GEPI_OK)
+            return rc;
+        if (pair_cap) grown(p->d_pairs, p->pairs_bytes, (size_t)pair_cap * 48);
+        if (pair_cap && (rc = grow(&p->d_pairs, &p->pairs_bytes, (size_t)pair_cap * 48)) != GEPI_OK)
             return rc;
         if (cap > p->buf_cap) alloc += (int64_t)(sizeof(Cand) * cap);
         if (pcap > p->pend_cap) alloc += (int64_t)(sizeof(Pend) * pcap);
@@ -670,6 +675,8 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
     ca.st = b.state;
     ca.pend = b.pend;
     ca.pcap = pcap;
+    ca.pairs = pair_cap ? p->d_pairs : nullptr;
+    ca.pair_cap = pair_cap;
     ca.park = f4w_park ? p->d_park : nullptr;
     ca.park_busy = f4w_park ? reinterpret_cast<uint32_t *>(
                                   reinterpret_cast<char *>(p->d_park) + park_rec_bytes)
@@ -761,6 +768,15 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
         }
     };
     auto launch_exact = [&]() {
+        if (pair_cap) {
+            /* at most PAIRS_WG_PER_CU workgroups per CU, none without work */
+            const unsigned grid = std::min<unsigned>((pair_cap + PAIRS_THREADS - 1) / PAIRS_THREADS,
+                                                     (unsigned)(PAIRS_WG_PER_CU * device_cus(p->device)));
+            if (entropy)
+                k_pairs<GEPI_FFUNC_ENTROPY><<<grid, PAIRS_THREADS, 0, p->stream>>>(ca);
+            else
+                k_pairs<GEPI_FFUNC_FISHERPV><<<grid, PAIRS_THREADS, 0, p->stream>>>(ca);
+        }
         if (entropy)
             k_exact<GEPI_FFUNC_ENTROPY><<<1024, 256, 0, p->stream>>>(ea);
         else

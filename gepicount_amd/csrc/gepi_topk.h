@@ -69,6 +69,7 @@ static __global__ void k_reset_pending(ScanState *st) {
     if (threadIdx.x != 0) return;
     st->pend_count = 0;
     st->pend_overflow = 0;
+    st->pair_count = 0;
 }
 
 struct SelPrefix {
@@ -515,6 +516,7 @@ __device__ __forceinline__ void topk_wg_body(const TopkDesc &d) {
         }
         st->pend_count = 0;
         st->pend_overflow = 0;
+        st->pair_count = 0;
     }
 }
 
