@@ -1184,7 +1184,7 @@ extern "C" int gepi_panel_create_bed(const uint8_t *bed_payload, int64_t n_varia
     const int64_t bytes = n_variants * bps;
     if (bytes > 0 && p->w64 > 0) {
         uint8_t *d_bed = nullptr;
-        if (hipMalloc(&d_bed, (size_t)bytes) != hipSuccess) {
+        if (hipMalloc(&d_bed, (size_t)bytes + BED_PAD) != hipSuccess) {
             panel_free(p);
             return gepi_fail(GEPI_ERR_NOMEM, "bed staging allocation failed");
         }
@@ -1232,9 +1232,8 @@ int panel_missing(gepi_panel *p, std::vector<int32_t> &var_miss, std::vector<int
     hipMemsetAsync(d_sv, 0, sizeof(int32_t) * (size_t)p->n_samples, p->stream);
     k_qa_variants<<<(unsigned)((p->n_var + 3) / 4), 256, 0, p->stream>>>(p->d_nat, p->n_var, p->w64,
                                                                         p->n_samples, d_vm);
-    const int32_t chunk = 1024;
-    dim3 grid((unsigned)((p->n_samples + 255) / 256), (unsigned)((p->n_var + chunk - 1) / chunk));
-    k_qa_samples<<<grid, 256, 0, p->stream>>>(p->d_nat, p->n_var, p->w64, p->n_samples, chunk, d_sv);
+    const dim3 grid((unsigned)((p->n_var + QA_VARS - 1) / QA_VARS), (unsigned)((p->w64 + 63) / 64));
+    k_qa_samples<<<grid, 256, 0, p->stream>>>(p->d_nat, p->n_var, p->w64, p->n_samples, d_sv);
     hipError_t e = hipGetLastError();
     if (e == hipSuccess)
         e = hipMemcpyAsync(var_miss.data(), d_vm, sizeof(int32_t) * (size_t)p->n_var,
