@@ -153,19 +153,31 @@ k_count_f4w_batch(const BatchDesc *__restrict__ d, BatchMap map) {
 template <int FFUN>
 __global__ void __launch_bounds__(F4W_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_count_f4g_batch(const BatchDesc *__restrict__ d, BatchMap map) {
-    __shared__ F4GShared sh;
+    __shared__ F4GShared<3> sh;
     const F4BatchOnceSrc src{d, map};
     const F4Job j = uniform_job(src.grab(0));
     if (!j.ok) return;
     const CountArgs g = d[j.item].g;
-    count_f4g_unit<FFUN>(g, j.tile - g.tile_begin, sh);
+    count_f4g_unit<FFUN, 3>(g, j.tile - g.tile_begin, sh);
 }
 
-/* The pairs put off by k_count_f4g_batch (pairs_run); blockIdx.y = scan. */
+/* ... and of panels without missing calls. */
 template <int FFUN>
+__global__ void __launch_bounds__(F4W_THREADS) __attribute__((amdgpu_waves_per_eu(3, 3)))
+k_count_f4c_batch(const BatchDesc *__restrict__ d, BatchMap map) {
+    __shared__ F4GShared<2> sh;
+    const F4BatchOnceSrc src{d, map};
+    const F4Job j = uniform_job(src.grab(0));
+    if (!j.ok) return;
+    const CountArgs g = d[j.item].g;
+    count_f4g_unit<FFUN, 2>(g, j.tile - g.tile_begin, sh);
+}
+
+/* The pairs put off by those (pairs_run); blockIdx.y = scan. */
+template <int FFUN, int NP>
 __global__ void __launch_bounds__(PAIRS_THREADS) k_pairs_batch(const BatchDesc *__restrict__ d) {
     const CountArgs g = d[blockIdx.y].g;
-    pairs_run<FFUN>(g, blockIdx.x, gridDim.x);
+    pairs_run<FFUN, NP>(g, blockIdx.x, gridDim.x);
 }
 
 /* p[0..n) = v (one workgroup of 64 threads per 64 words). */

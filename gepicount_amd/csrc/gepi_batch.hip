@@ -97,7 +97,11 @@ void Engine::launch_count(int g, bool persist, unsigned grid, const BatchMap &m)
     const BatchDesc *d = d_bdesc_[g];
     if (g >= 4) {
         /* wave tiles: one unit per workgroup, no persistent form */
-        if (g == 6)
+        if (g == 8)
+            k_count_f4c_batch<GEPI_FFUNC_ENTROPY><<<grid, F4W_THREADS, 0, stream>>>(d, m);
+        else if (g == 9)
+            k_count_f4c_batch<GEPI_FFUNC_FISHERPV><<<grid, F4W_THREADS, 0, stream>>>(d, m);
+        else if (g == 6)
             k_count_f4g_batch<GEPI_FFUNC_ENTROPY><<<grid, F4W_THREADS, 0, stream>>>(d, m);
         else if (g == 7)
             k_count_f4g_batch<GEPI_FFUNC_FISHERPV><<<grid, F4W_THREADS, 0, stream>>>(d, m);
@@ -465,7 +469,7 @@ size_t Engine::estimate_footprint(const gepi_panel *p, int64_t topmost) {
     const unsigned long long cap =
         std::max<unsigned long long>((unsigned long long)k + TILE_EVALS_MAX + 1024, 4ull * k);
     const unsigned long long pcap = std::max<unsigned long long>(cap, 1ull << 20);
-    return round_block((size_t)n_u * n_var_pad * 3 * 64 + (size_t)n_var_pad * sizeof(float)) + round_block(cap * sizeof(Cand)) +
+    return round_block((size_t)n_u * n_var_pad * 3 * 64 + (size_t)n_var_pad * 6 * sizeof(float)) + round_block(cap * sizeof(Cand)) +
            round_block(pcap * sizeof(Pend)) + round_block((size_t)4 * p->w64 * sizeof(CompressWord)) +
            round_block(sizeof(ScanState)) +
            round_block((size_t)pair_list_cap(n_var_pad / TM * (n_var_pad / TM + 1), 0, PAIRS_MOST_BATCH) * 48);
@@ -527,6 +531,7 @@ int Engine::add(ScanItem *it) {
     if (it->ffun != GEPI_FFUNC_ENTROPY && !use_graph_) it->shape = 2;
     if (it->shape == 2 && use_graph_) it->shape = 0;
     it->geno = it->shape == 2 && p->three_genotypes;
+    it->full = it->geno && p->complete;
     it->stats.count_path = it->shape == 2 ? 3 : 4;
     it->stats.n_class0 = it->n0;
     it->stats.n_class1 = it->n1;
@@ -571,7 +576,7 @@ int Engine::add(ScanItem *it) {
     /* three K steps per super-step (f4_super3, see count_f4_run) */
     const int32_t n_u = f4_super3(w0 / 4) + f4_super3(w1 / 4); /* 64-byte rows each */
     const size_t rows_bytes = (size_t)std::max(n_u, 1) * it->n_var_pad * 3 * 4 * sizeof(uint4);
-    const size_t lay = rows_bytes + (it->geno ? (size_t)it->n_var_pad * sizeof(float) : 0);
+    const size_t lay = rows_bytes + (it->geno ? (size_t)it->n_var_pad * sizeof(float) * (it->full ? 6 : 1) : 0);
     const size_t cw_words = it->h_cw.size();
     if (it->geno) {
         /* the super-steps' places follow the compression words */
@@ -598,11 +603,14 @@ int Engine::add(ScanItem *it) {
                     (it->pair_cap ? round_block((size_t)it->pair_cap * 48) : 0);
     HIP_TRY(hipMemcpyAsync(it->d_cw, it->h_cw.data(), it->h_cw.size() * sizeof(CompressWord),
                            hipMemcpyHostToDevice, stream));
+    CountArgs ca;
+    screen_consts(it->n0, it->n1, ca);
     if (it->geno) {
         it->d_miss = reinterpret_cast<const float *>(reinterpret_cast<char *>(it->d_layout) + rows_bytes);
         k_class_geno<<<dim3((unsigned)(it->n_var_pad / 64), (unsigned)n_u + 1), CLSG_THREADS, 0, stream>>>(
             p->d_nat, (int32_t)it->n_var, p->w64, it->d_cw,
-            reinterpret_cast<const SuperSrc *>(it->d_cw + cw_words), n_u, it->n0 + it->n1, it->d_layout,
+            reinterpret_cast<const SuperSrc *>(it->d_cw + cw_words), n_u, it->n0, it->n0 + it->n1,
+            it->full ? 3.0f * ca.sc_start : 0.0f, it->d_layout,
             const_cast<float *>(it->d_miss));
         HIP_TRY(hipGetLastError());
     } else if (it->n_k4 > 0) {
@@ -624,7 +632,6 @@ int Engine::add(ScanItem *it) {
     it->forced_band = 0;
     if (const char *env = getenv("GEPI_BAND_TILES")) it->forced_band = std::max<long long>(1, atoll(env));
     /* the first band under a guessed threshold, as in a planned single scan */
-    CountArgs ca;
     chi2_slope(it->n0, it->n1, &ca.h0, &ca.h1);
     BandPlan &pl = it->plan;
     pl = BandPlan{};
@@ -699,7 +706,7 @@ int Engine::round(std::vector<ScanItem *> &finished) {
     std::vector<TopkDesc> td(na);
     for (size_t i = 0; i < na; i++) {
         ScanItem *it = active_[i];
-        grp[(it->ffun == GEPI_FFUNC_ENTROPY ? 0 : 1) + 2 * (it->geno ? 3 : it->shape)].push_back(it);
+        grp[(it->ffun == GEPI_FFUNC_ENTROPY ? 0 : 1) + 2 * (it->full ? 4 : it->geno ? 3 : it->shape)].push_back(it);
         ExactDesc &e = ed[i];
         memset(&e, 0, sizeof e);
         e.e.st = it->d_state;
@@ -878,12 +885,14 @@ int Engine::round(std::vector<ScanItem *> &finished) {
             }
             launch_count(f, per_cu > 0, grid, m);
         }
-        if (!bd[6].empty())
-            k_pairs_batch<GEPI_FFUNC_ENTROPY><<<dim3(PAIRS_BLOCKS_X, (unsigned)bd[6].size()), PAIRS_THREADS,
-                                                0, stream>>>(d_bdesc_[6]);
-        if (!bd[7].empty())
-            k_pairs_batch<GEPI_FFUNC_FISHERPV><<<dim3(PAIRS_BLOCKS_X, (unsigned)bd[7].size()), PAIRS_THREADS,
-                                                 0, stream>>>(d_bdesc_[7]);
+        auto pairs = [&](auto kernel, int f) {
+            if (!bd[f].empty())
+                kernel<<<dim3(PAIRS_BLOCKS_X, (unsigned)bd[f].size()), PAIRS_THREADS, 0, stream>>>(d_bdesc_[f]);
+        };
+        pairs(k_pairs_batch<GEPI_FFUNC_ENTROPY, 3>, 6);
+        pairs(k_pairs_batch<GEPI_FFUNC_FISHERPV, 3>, 7);
+        pairs(k_pairs_batch<GEPI_FFUNC_ENTROPY, 2>, 8);
+        pairs(k_pairs_batch<GEPI_FFUNC_FISHERPV, 2>, 9);
         HIP_TRY(hipGetLastError());
         HIP_TRY(hipEventRecord(ev1_, stream));
         k_exact_batch<<<dim3(EXACT_BLOCKS_X, (unsigned)na), 256, 0, stream>>>(d_edesc_);

@@ -1004,13 +1004,15 @@ struct F4WShared {
     uint32_t n_park, park_slot;
 };
 
-/* The nine products of a 32 x 32-variant wave tile (groups gA, gB of the
- * grouped layout) over both classes: acc[p][q] ends at start plus the totals,
+/* The products of the first NP planes (9 of three, 4 of two) of a 32 x
+ * 32-variant wave tile (groups gA, gB of the grouped layout) over both
+ * classes: acc[p][q] ends at start plus the totals,
  * and the class-0 counts (below 2^16) of elements e and e + 1 go to dword
- * (e / 2 * 9 + 3p + q) * 64 of the lane's LDS column P.  start: 0, or a
+ * ((e / 2 NP + p) NP + q) * 64 of the lane's LDS column P.  start: 0, or a
  * fraction that no count rounds away (see count_f4g_unit).                */
+template <int NP>
 __device__ __forceinline__ void f4w_products(const CountArgs &g, int32_t gA, int32_t gB, bool live,
-                                             float start, uint32_t *P, v16f (&acc)[3][3]) {
+                                             float start, uint32_t *P, v16f (&acc)[NP][NP]) {
     const int lane = threadIdx.x & 63;
     const int32_t u1 = f4_super3(g.ks0), n_u = u1 + f4_super3(g.n_ks - g.ks0);
     const int32_t last = n_u > 0 ? n_u - 1 : 0; /* n_u == 0: super-step 0 exists */
@@ -1018,8 +1020,8 @@ __device__ __forceinline__ void f4w_products(const CountArgs &g, int32_t gA, int
     const int64_t ustride = (int64_t)g.n_var_pad * 192; /* bytes per super-step */
     const int loff = (lane >> 5) * 512 + (lane & 31) * 16;
 
-    /* c[cp][p]: A plane p, column h + 2cp; c[cp][3 + q]: B plane q */
-    uint4 c[2][6];
+    /* c[cp][p]: A plane p, column h + 2cp; c[cp][NP + q]: B plane q */
+    uint4 c[2][2 * NP];
     auto fetch = [&](int32_t u, int cp) {
         const char *base = lay + (int64_t)u * ustride;
         const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(
@@ -1027,16 +1029,16 @@ __device__ __forceinline__ void f4w_products(const CountArgs &g, int32_t gA, int
         const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(
             const_cast<char *>(base + (int64_t)gB * 6144), (short)0, 6144, F4_RSRC_WORD3);
 #pragma unroll
-        for (int p = 0; p < 3; p++) {
+        for (int p = 0; p < NP; p++) {
             c[cp][p] = as_u4(__builtin_amdgcn_raw_buffer_load_b128(ra, loff + p * 2048 + cp * 1024, 0, 0));
-            c[cp][3 + p] =
+            c[cp][NP + p] =
                 as_u4(__builtin_amdgcn_raw_buffer_load_b128(rb, loff + p * 2048 + cp * 1024, 0, 0));
         }
     };
 #pragma unroll
-    for (int p = 0; p < 3; p++)
+    for (int p = 0; p < NP; p++)
 #pragma unroll
-        for (int q = 0; q < 3; q++)
+        for (int q = 0; q < NP; q++)
 #pragma unroll
             for (int e = 0; e < 16; e++) acc[p][q][e] = start;
     /* One super-step: per column pair three chunks of 9 MFMAs; the pair's six
@@ -1055,10 +1057,10 @@ __device__ __forceinline__ void f4w_products(const CountArgs &g, int32_t gA, int
 #pragma unroll
             for (int b = 0; b < 3; b++) {
                 const uint32_t m = 0x11111111u << b;
-                v8i fa[3], fb[3];
+                v8i fa[NP], fb[NP];
 #pragma unroll
-                for (int q = 0; q < 3; q++) {
-                    fb[q] = frag_f4(c[cp][3 + q], m);
+                for (int q = 0; q < NP; q++) {
+                    fb[q] = frag_f4(c[cp][NP + q], m);
                     fa[q] = frag_f4(c[cp][q], m);
                 }
                 if (b == 2) {
@@ -1067,9 +1069,9 @@ __device__ __forceinline__ void f4w_products(const CountArgs &g, int32_t gA, int
                     __builtin_amdgcn_sched_barrier(0x6);
                 }
 #pragma unroll
-                for (int p = 0; p < 3; p++)
+                for (int p = 0; p < NP; p++)
 #pragma unroll
-                    for (int q = 0; q < 3; q++)
+                    for (int q = 0; q < NP; q++)
                         acc[p][q] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(
                             fa[p], fb[q], acc[p][q], F4_FMT, F4_FMT, 0, f4_scale(b), 0, f4_scale(b));
             }
@@ -1094,12 +1096,12 @@ __device__ __forceinline__ void f4w_products(const CountArgs &g, int32_t gA, int
         for (; u < u_end; u++) sstep(u);
         if (cls == 0) {
 #pragma unroll
-            for (int p = 0; p < 3; p++)
+            for (int p = 0; p < NP; p++)
 #pragma unroll
-                for (int q = 0; q < 3; q++)
+                for (int q = 0; q < NP; q++)
 #pragma unroll
                     for (int e = 0; e < 16; e += 2)
-                        P[(e / 2 * 9 + p * 3 + q) * 64] =
+                        P[(e / 2 * (NP * NP) + p * NP + q) * 64] =
                             (uint32_t)acc[p][q][e] | ((uint32_t)acc[p][q][e + 1] << 16);
         }
         u_end = nu_live;
@@ -1124,7 +1126,7 @@ __device__ __forceinline__ void count_f4w_unit(const CountArgs &g, int64_t unit,
     uint32_t *P = sh.c0lds[wave] + lane; /* dword d of this lane at P[64 d] */
 
     v16f acc[3][3];
-    f4w_products(g, gA, gB, live, 0.0f, P, acc);
+    f4w_products<3>(g, gA, gB, live, 0.0f, P, acc);
     const FilterConsts fc = filter_consts(g.st, g);
     __syncthreads(); /* the stage counter is cleared, the park region claimed */
     const bool parks = PARK && sh.park_slot != PARK_NONE;
@@ -1215,14 +1217,51 @@ __device__ __forceinline__ void count_f4w_unit(const CountArgs &g, int64_t unit,
 constexpr int F4G_LIST = 256;  /* pairs collected per workgroup               */
 constexpr int F4G_STAGE = 112; /* survivors staged per workgroup              */
 constexpr int PAIRS_THREADS = 256;
+/* NP: planes multiplied, 3, or 2 without missing calls (see below). */
+template <int NP>
 struct F4GShared {
-    uint32_t c0lds[4][F4W_PARK * 64];
-    uint32_t list[F4G_LIST * 5]; /* 9 totals of 16 bits, then wave, lane, e   */
+    uint32_t c0lds[4][8 * NP * NP * 64];
+    uint32_t list[F4G_LIST * 5]; /* totals of 16 bits, then wave, lane, e     */
     PendStageN<F4G_STAGE> stage;
     uint32_t n;
     unsigned long long base; /* the list's place in the scan's               */
 };
-static_assert(sizeof(F4GShared) <= 81920, "two workgroups per CU");
+static_assert(sizeof(F4GShared<3>) <= 81920, "two workgroups per CU");
+static_assert(sizeof(F4GShared<2>) <= 53248, "three workgroups per CU");
+
+/* Without missing calls in the panel a pair's table has its variants' own
+ * genotype counts as margins, so four products (homozygous 1 and heterozygous
+ * of both variants) give its nine cells: 4/9 of the matrix work, 64
+ * accumulators instead of 144 and so three waves per SIMD.  g.miss then holds
+ * the margins, six floats a variant: the totals of the three genotypes, each
+ * with three times sc_start (a cell made from them and from accumulators keeps
+ * one of it), and the class-0 counts.  All are whole multiples of sc_start
+ * below 2^24 of it, so the cells are exact.  Against nine products: 30,001 x
+ * 3,001 4.96 -> 3.15 ms, 20,000 x 256 0.77x the time, x 2,048 0.69x, x 8,192
+ * 0.57x (Fisher 0.83x, 0.77x, 0.64x), 4,000 x 1,000 0.93x.                 */
+template <int NP>
+struct F4GMargins {
+    float t[3], c[3];
+    __device__ __forceinline__ void load(const float *miss, int32_t v) {
+        const float2 *m = reinterpret_cast<const float2 *>(miss + (int64_t)v * 6);
+        const float2 a = m[0], b = m[1], d = m[2];
+        t[0] = a.x, t[1] = a.y, t[2] = b.x;
+        c[0] = b.y, c[1] = d.x, c[2] = d.y;
+    }
+};
+/* x[3][3] from its first two rows and columns and the margins of A and B. */
+template <class T>
+__device__ __forceinline__ void f4g_complete(T (&x)[9], const T (&p)[4], const T (&a)[3], const T (&b)[3]) {
+    x[0] = p[0];
+    x[1] = p[1];
+    x[2] = a[0] - p[0] - p[1];
+    x[3] = p[2];
+    x[4] = p[3];
+    x[5] = a[1] - p[2] - p[3];
+    x[6] = b[0] - p[0] - p[2];
+    x[7] = b[1] - p[1] - p[3];
+    x[8] = a[2] - x[6] - x[7];
+}
 
 /* (float) of the low (H = 0) or high half of w in one instruction. */
 template <int H>
@@ -1245,18 +1284,19 @@ __device__ __forceinline__ float screen_cell(float T, float c, float np, float k
 }
 
 /* A pair's record: its totals and where its class-0 counts are. */
-__device__ __forceinline__ void f4g_append(uint32_t *L, const float (&T)[9], uint32_t id) {
-    uint32_t u[9];
+template <int NC>
+__device__ __forceinline__ void f4g_append(uint32_t *L, const float (&T)[NC], uint32_t id) {
+    uint32_t u[NC];
 #pragma unroll
-    for (int i = 0; i < 9; i++) u[i] = (uint32_t)T[i];
+    for (int i = 0; i < NC; i++) u[i] = (uint32_t)T[i];
 #pragma unroll
-    for (int i = 0; i < 4; i++) L[i] = u[2 * i] | (u[2 * i + 1] << 16);
-    L[4] = u[8] | (id << 16);
+    for (int i = 0; i < NC / 2; i++) L[i] = u[2 * i] | (u[2 * i + 1] << 16);
+    L[4] = (NC & 1 ? u[NC - 1] : 0u) | (id << 16);
 }
 
-/* A pair's cells by class from its totals (9 halfwords from dword 0 of r, the
- * id in the last) and class-0 counts.                                      */
-__device__ __forceinline__ int32_t f4g_total(const uint32_t (&r)[5], int i) {
+/* Halfword i of r. */
+template <int N>
+__device__ __forceinline__ int32_t f4g_half(const uint32_t (&r)[N], int i) {
     return (int32_t)((r[i >> 1] >> (16 * (i & 1))) & 0xFFFFu);
 }
 
@@ -1270,19 +1310,44 @@ __device__ __forceinline__ void f4g_variants(uint32_t id, int64_t tile, int32_t 
     B = tb * 32 + (src & 31);
 }
 
-/* The int32 filter on a pair's cells. */
-template <int FFUN, bool ROLLED, class PS>
+/* The int32 filter on a pair's totals and class-0 counts. */
+template <int FFUN, int NP, bool ROLLED, class PS>
 __device__ __forceinline__ void f4g_filter(const CountArgs &g, PS &ps, const FilterConsts &fc,
-                                           const int32_t (&x)[2][3][3], int32_t A, int32_t B) {
+                                           const int32_t (&t)[NP * NP], const int32_t (&h)[NP * NP],
+                                           int32_t A, int32_t B) {
+    int32_t x[2][9]; /* cells by class */
+    if constexpr (NP == 2) {
+        F4GMargins<NP> ma, mb;
+        ma.load(g.miss, A);
+        mb.load(g.miss, B);
+        int32_t at[3], bt[3], ac[3], bc[3];
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            at[i] = (int32_t)ma.t[i]; /* truncated: without the start's share */
+            bt[i] = (int32_t)mb.t[i];
+            ac[i] = (int32_t)ma.c[i];
+            bc[i] = (int32_t)mb.c[i];
+        }
+        f4g_complete(x[1], t, at, bt);
+        f4g_complete(x[0], h, ac, bc);
+    } else {
+#pragma unroll
+        for (int i = 0; i < 9; i++) {
+            x[1][i] = t[i];
+            x[0][i] = h[i];
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 9; i++) x[1][i] -= x[0][i];
     int32_t c[2][3][3]; /* products of the allele and valid planes */
 #pragma unroll
     for (int k = 0; k < 2; k++) {
         int32_t u[3][3];
 #pragma unroll
         for (int i = 0; i < 3; i++) {
-            u[i][0] = x[k][i][0] + x[k][i][1];
-            u[i][1] = x[k][i][1] + x[k][i][2];
-            u[i][2] = u[i][0] + x[k][i][2];
+            u[i][0] = x[k][3 * i] + x[k][3 * i + 1];
+            u[i][1] = x[k][3 * i + 1] + x[k][3 * i + 2];
+            u[i][2] = u[i][0] + x[k][3 * i + 2];
         }
 #pragma unroll
         for (int q = 0; q < 3; q++) {
@@ -1296,41 +1361,46 @@ __device__ __forceinline__ void f4g_filter(const CountArgs &g, PS &ps, const Fil
 
 /* Collected pair L of the workgroup's unit: to place `at` of the scan's list
  * for k_pairs while that has room, else tested here.  A record is the five
- * dwords of the list, the nine class-0 counts and the tile.                */
-template <int FFUN>
-__device__ __forceinline__ void f4g_deal(const CountArgs &g, F4GShared &sh, const FilterConsts &fc,
+ * dwords of the list, the class-0 counts and the tile: three uint4, two of
+ * them with NP = 2.                                                        */
+template <int FFUN, int NP>
+__device__ __forceinline__ void f4g_deal(const CountArgs &g, F4GShared<NP> &sh, const FilterConsts &fc,
                                          const uint32_t *L, int64_t unit, unsigned long long at) {
+    constexpr int NC = NP * NP;
     uint32_t r[5];
 #pragma unroll
     for (int i = 0; i < 5; i++) r[i] = L[i];
     const uint32_t id = r[4] >> 16, e = id & 15u, src = (id >> 4) & 63u, wv = id >> 10;
-    const uint16_t *c0 = reinterpret_cast<const uint16_t *>(sh.c0lds[wv]) + (e >> 1) * (9 * 128) +
+    const uint16_t *c0 = reinterpret_cast<const uint16_t *>(sh.c0lds[wv]) + (e >> 1) * (NC * 128) +
                          src * 2 + (e & 1);
     const int64_t tile = g.tile_begin + 2 * unit + (wv >> 1);
-    if (at < g.pair_cap) {
-        uint32_t h[9];
+    int32_t h[NC];
 #pragma unroll
-        for (int i = 0; i < 9; i++) h[i] = c0[i * 128];
-        uint4 *dst = g.pairs + at * 3;
-        dst[0] = make_uint4(r[0], r[1], r[2], r[3]);
-        dst[1] = make_uint4(r[4], h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16));
-        dst[2] = make_uint4(h[6] | (h[7] << 16), h[8], (uint32_t)tile, (uint32_t)(tile >> 32));
+    for (int i = 0; i < NC; i++) h[i] = c0[i * 128];
+    if (at < g.pair_cap) {
+        auto two = [&](int i) { return (uint32_t)h[i] | ((uint32_t)h[i + 1] << 16); };
+        uint4 *dst = g.pairs + at * NP;
+        const uint32_t lo = (uint32_t)tile, hi = (uint32_t)(tile >> 32);
+        if constexpr (NP == 2) {
+            dst[0] = make_uint4(r[0], r[1], two(0), two(2));
+            dst[1] = make_uint4(r[4], 0u, lo, hi);
+        } else {
+            dst[0] = make_uint4(r[0], r[1], r[2], r[3]);
+            dst[1] = make_uint4(r[4], two(0), two(2), two(4));
+            dst[2] = make_uint4(two(6), (uint32_t)h[8], lo, hi);
+        }
         return;
     }
-    int32_t x[2][3][3];
+    int32_t t[NC], A, B;
 #pragma unroll
-    for (int i = 0; i < 9; i++) {
-        x[0][i / 3][i % 3] = c0[i * 128];
-        x[1][i / 3][i % 3] = f4g_total(r, i) - x[0][i / 3][i % 3];
-    }
-    int32_t A, B;
+    for (int i = 0; i < NC; i++) t[i] = f4g_half(r, i);
     f4g_variants(id, tile, g.n_var_pad / TM, A, B);
-    f4g_filter<FFUN, true>(g, sh.stage, fc, x, A, B);
+    f4g_filter<FFUN, NP, true>(g, sh.stage, fc, t, h, A, B);
 }
 
 /* The filter on the pairs that the count kernel of the band put off, one per
  * thread, n_wg workgroups.  Called by every thread of a workgroup.         */
-template <int FFUN>
+template <int FFUN, int NP>
 __device__ __forceinline__ void pairs_run(const CountArgs &g, uint32_t wg, uint32_t n_wg) {
     __shared__ PendStage stage;
     const unsigned long long put = g.st->pair_count;
@@ -1340,24 +1410,34 @@ __device__ __forceinline__ void pairs_run(const CountArgs &g, uint32_t wg, uint3
     const FilterConsts fc = filter_consts(g.st, g);
     __syncthreads();
     for (uint32_t i = wg * blockDim.x + threadIdx.x; i < n; i += n_wg * blockDim.x) {
-        const uint4 a = g.pairs[(uint64_t)i * 3], b = g.pairs[(uint64_t)i * 3 + 1],
-                    d = g.pairs[(uint64_t)i * 3 + 2];
-        const uint32_t r[5] = {a.x, a.y, a.z, a.w, b.x}, h[5] = {b.y, b.z, b.w, d.x, d.y};
-        int32_t x[2][3][3];
+        const uint4 *rec = g.pairs + (uint64_t)i * NP;
+        const uint4 a = rec[0], b = rec[1], d = rec[NP - 1];
+        int32_t t[NP * NP], h[NP * NP];
+        if constexpr (NP == 2) {
+            const uint32_t r[4] = {a.x, a.y, a.z, a.w};
 #pragma unroll
-        for (int k = 0; k < 9; k++) {
-            x[0][k / 3][k % 3] = f4g_total(h, k);
-            x[1][k / 3][k % 3] = f4g_total(r, k) - x[0][k / 3][k % 3];
+            for (int k = 0; k < 4; k++) {
+                t[k] = f4g_half(r, k);
+                h[k] = f4g_half(r, 4 + k);
+            }
+        } else {
+            const uint32_t r[5] = {a.x, a.y, a.z, a.w, b.x}, s[5] = {b.y, b.z, b.w, d.x, d.y};
+#pragma unroll
+            for (int k = 0; k < 9; k++) {
+                t[k] = f4g_half(r, k);
+                h[k] = f4g_half(s, k);
+            }
         }
         int32_t A, B;
-        f4g_variants(r[4] >> 16, (int64_t)((uint64_t)d.w << 32 | d.z), g.n_var_pad / TM, A, B);
-        f4g_filter<FFUN, false>(g, stage, fc, x, A, B);
+        f4g_variants(b.x >> 16, (int64_t)((uint64_t)d.w << 32 | d.z), g.n_var_pad / TM, A, B);
+        f4g_filter<FFUN, NP, false>(g, stage, fc, t, h, A, B);
     }
     stage_flush(g, stage);
 }
 
-template <int FFUN>
-__device__ __forceinline__ void count_f4g_unit(const CountArgs &g, int64_t unit, F4GShared &sh) {
+template <int FFUN, int NP>
+__device__ __forceinline__ void count_f4g_unit(const CountArgs &g, int64_t unit, F4GShared<NP> &sh) {
+    constexpr int NC = NP * NP;
     stage_init(sh.stage);
     if (threadIdx.x == 0) sh.n = 0;
     const int lane = threadIdx.x & 63;
@@ -1368,8 +1448,8 @@ __device__ __forceinline__ void count_f4g_unit(const CountArgs &g, int64_t unit,
     if (live) tile_of_f4(tile, g.n_var_pad / TM, ta, tb);
     const int32_t gA = 2 * ta + (wave & 1), gB = tb;
     uint32_t *P = sh.c0lds[wave] + lane;
-    v16f acc[3][3];
-    f4w_products(g, gA, gB, live, g.sc_start, P, acc);
+    v16f acc[NP][NP];
+    f4w_products<NP>(g, gA, gB, live, g.sc_start, P, acc);
 
     const FilterConsts fc = filter_consts(g.st, g);
     /* the right side is R (1 - a) - sc_sub, or negative: every pair passes */
@@ -1381,7 +1461,13 @@ __device__ __forceinline__ void count_f4g_unit(const CountArgs &g, int64_t unit,
     const int32_t B = gB * 32 + (lane & 31);
     const int32_t Ab = gA * 32 + 4 * (lane >> 5);
     const float RA = FFUN == GEPI_FFUNC_ENTROPY ? R : 0.0f;
-    const float rB = __builtin_fmaf(-RA, g.miss[B], R - g.sc_sub), np = -g.sc_p, kk = g.sc_k;
+    const float np = -g.sc_p, kk = g.sc_k;
+    float rB = R - g.sc_sub;
+    F4GMargins<NP> mB;
+    if constexpr (NP == 2)
+        mB.load(g.miss, B);
+    else
+        rB = __builtin_fmaf(-RA, g.miss[B], rB);
     __syncthreads(); /* the counters are cleared */
     uint32_t pend = 0; /* elements that found the list full */
     auto in_scan = [&](int e) {
@@ -1390,34 +1476,46 @@ __device__ __forceinline__ void count_f4g_unit(const CountArgs &g, int64_t unit,
     };
     /* the lanes of fl append their element e; true for those without room.
      * Every lane of the wave calls it: lane 0 reserves the places            */
-    auto collect = [&](bool fl, const float (&T)[9], int e) {
+    auto collect = [&](bool fl, const float (&T)[NC], int e) {
         const uint64_t m = __ballot(fl);
         uint32_t at = 0;
         if (lane == 0) at = atomicAdd(&sh.n, (uint32_t)__popcll(m));
         at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at) +
              __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
         const bool room = at < (uint32_t)F4G_LIST;
-        if (fl && room) f4g_append(sh.list + at * 5, T, (uint32_t)(wave << 10 | lane << 4 | e));
+        if (fl && room) f4g_append<NC>(sh.list + at * 5, T, (uint32_t)(wave << 10 | lane << 4 | e));
         return fl && !room;
     };
 #pragma unroll
     for (int j = 0; j < 8; j++) {
-        uint32_t w[9];
+        uint32_t w[NC];
 #pragma unroll
-        for (int i = 0; i < 9; i++) w[i] = P[(j * 9 + i) * 64];
+        for (int i = 0; i < NC; i++) w[i] = P[(j * NC + i) * 64];
         float4 mA = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        if (FFUN == GEPI_FFUNC_ENTROPY) mA = *reinterpret_cast<const float4 *>(g.miss + Ab + 8 * (j >> 1));
+        if (FFUN == GEPI_FFUNC_ENTROPY && NP == 3) mA = *reinterpret_cast<const float4 *>(g.miss + Ab + 8 * (j >> 1));
 #pragma unroll
         for (int hf = 0; hf < 2; hf++) {
             const int e = 2 * j + hf;
-            float T[9], q = 0.0f;
+            float T[NC], c[NC], q = 0.0f;
 #pragma unroll
-            for (int i = 0; i < 9; i++) {
-                T[i] = acc[i / 3][i % 3][e];
-                q = screen_cell(T[i], hf == 0 ? half_to_float<0>(w[i]) : half_to_float<1>(w[i]), np, kk, q);
+            for (int i = 0; i < NC; i++) {
+                T[i] = acc[i / NP][i % NP][e];
+                c[i] = hf == 0 ? half_to_float<0>(w[i]) : half_to_float<1>(w[i]);
+            }
+            if constexpr (NP == 2) {
+                F4GMargins<NP> mA;
+                mA.load(g.miss, Ab + 8 * (e >> 2) + (e & 3));
+                float Tx[9], cx[9];
+                f4g_complete(Tx, T, mA.t, mB.t);
+                f4g_complete(cx, c, mA.c, mB.c);
+#pragma unroll
+                for (int i = 0; i < 9; i++) q = screen_cell(Tx[i], cx[i], np, kk, q);
+            } else {
+#pragma unroll
+                for (int i = 0; i < NC; i++) q = screen_cell(T[i], c[i], np, kk, q);
             }
             const float mAe = (e & 3) == 0 ? mA.x : (e & 3) == 1 ? mA.y : (e & 3) == 2 ? mA.z : mA.w;
-            bool fl = q > __builtin_fmaf(-RA, mAe, rB);
+            bool fl = q > (NP == 3 ? __builtin_fmaf(-RA, mAe, rB) : rB);
             if (__ballot(fl)) {
                 fl = fl && in_scan(e);
                 if (__ballot(fl)) pend |= collect(fl, T, e) ? 1u << e : 0u;
@@ -1433,7 +1531,7 @@ __device__ __forceinline__ void count_f4g_unit(const CountArgs &g, int64_t unit,
         }
         const unsigned long long base = g.pair_cap > 0 ? sh.base : 0ull;
         for (uint32_t i = threadIdx.x; i < n; i += F4W_THREADS)
-            f4g_deal<FFUN>(g, sh, fc, sh.list + i * 5, unit, base + i);
+            f4g_deal<FFUN, NP>(g, sh, fc, sh.list + i * 5, unit, base + i);
         if (!__syncthreads_or(pend != 0)) break;
         /* the list was full (loose thresholds): the next of the elements left
          * over.  e is uniform here, so the accumulators are read by register
@@ -1444,9 +1542,9 @@ __device__ __forceinline__ void count_f4g_unit(const CountArgs &g, int64_t unit,
         for (int e = 0; e < 16; e++) {
             const bool fl = (pend >> e) & 1u;
             if (!__ballot(fl)) continue;
-            float T[9];
+            float T[NC];
 #pragma unroll
-            for (int i = 0; i < 9; i++) T[i] = acc[i / 3][i % 3][e];
+            for (int i = 0; i < NC; i++) T[i] = acc[i / NP][i % NP][e];
             const bool left = collect(fl, T, e); /* by every lane: lane 0 reserves */
             if (!left) pend &= ~(1u << e);
         }
@@ -1458,13 +1556,21 @@ __device__ __forceinline__ void count_f4g_unit(const CountArgs &g, int64_t unit,
 template <int FFUN>
 __global__ void __launch_bounds__(F4W_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_count_f4g(CountArgs g) {
-    __shared__ F4GShared sh;
-    count_f4g_unit<FFUN>(g, band_unit((g.n_tiles + 1) >> 1), sh);
+    __shared__ F4GShared<3> sh;
+    count_f4g_unit<FFUN, 3>(g, band_unit((g.n_tiles + 1) >> 1), sh);
 }
 
+/* The same without missing calls. */
 template <int FFUN>
+__global__ void __launch_bounds__(F4W_THREADS) __attribute__((amdgpu_waves_per_eu(3, 3)))
+k_count_f4c(CountArgs g) {
+    __shared__ F4GShared<2> sh;
+    count_f4g_unit<FFUN, 2>(g, band_unit((g.n_tiles + 1) >> 1), sh);
+}
+
+template <int FFUN, int NP>
 __global__ void __launch_bounds__(PAIRS_THREADS) k_pairs(CountArgs g) {
-    pairs_run<FFUN>(g, blockIdx.x, gridDim.x);
+    pairs_run<FFUN, NP>(g, blockIdx.x, gridDim.x);
 }
 
 template <int FFUN, bool F32, bool PARK>

@@ -83,14 +83,15 @@ struct CountArgs {
                                * the fp32 counts (f32_counts)                    */
     int32_t n0, n1;           /* class sizes (bounds of y and z: Fisher filter)   */
     /* wave tiles on genotype planes (count_f4g_unit): per variant the share
-     * of missing calls [n_var_pad]; p = n0/n, k, 2 p (1-p), 2 p (1-p) n; the
+     * of missing calls [n_var_pad], or the margins [n_var_pad][6] of a panel
+     * without missing calls (F4GMargins); p = n0/n, k, 2 p (1-p), 2 p (1-p) n; the
      * accumulators' start and what it takes off the screen's right side    */
     const float *miss;
     float sc_p, sc_k, sc_q, sc_m, sc_start, sc_sub;
     float h0, h1;             /* chi-square coefficient per nat: h0 + h1 min(y, z)
                                * (chi2_slope)                                     */
-    uint4 *pairs;             /* pairs that passed the screen, for k_pairs: 3 uint4
-                               * each; null with pair_cap 0                       */
+    uint4 *pairs;             /* pairs that passed the screen, for k_pairs: 3 (without
+                               * missing calls 2) uint4 each; null with pair_cap 0                       */
     uint32_t pair_cap;
     ScanState *st;
     Pend *pend;

@@ -54,6 +54,7 @@ struct ScanItem {
      * tiles on the grouped layout                                          */
     int32_t shape = 0;
     bool geno = false;    /* wave tiles on genotype planes */
+    bool full = false;         /* ... of a panel without missing calls            */
     const float *d_miss = nullptr; /* ... and their missing shares (in d_layout) */
     bool guessed = false; /* the first band runs under a guessed threshold    */
     BandPlan plan{};
@@ -134,7 +135,7 @@ class Engine {
     size_t in_use_ = 0;
     /* count launch groups: objective (g & 1) x job shape (g >> 1; 3: wave
      * tiles on genotype planes) */
-    static constexpr int NGROUP = 8, NGRAPH_COUNT = 16;
+    static constexpr int NGROUP = 10, NGRAPH_COUNT = 16;
     gepi::BatchDesc *d_bdesc_[NGROUP] = {};
     int64_t *d_map_[NGROUP] = {};
     gepi::ExactDesc *d_edesc_ = nullptr;

@@ -52,6 +52,7 @@ struct gepi_panel {
     /* every valid call carries an allele (always so for .bed genotypes), so
      * that three genotypes describe it (count_f4g_unit)                    */
     bool three_genotypes = true;
+    bool complete = false; /* no call of the panel is missing                */
     uint64_t *d_nat = nullptr;
     hipStream_t stream = nullptr;
     /* per-scan workspace, grown on demand and reused */

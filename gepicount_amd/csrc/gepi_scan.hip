@@ -445,6 +445,7 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
     const uint32_t park_slots = (uint32_t)(((4 * device_cus(p->device)) + 7) / 8 * 8);
     /* wave tiles on genotype planes, unless a valid call has no allele */
     const bool geno = path == 3 && p->three_genotypes;
+    const bool full = geno && p->complete; /* four products a pair, not nine */
     const bool f4w_park =
         path == 3 && !geno && !noalloc &&
         (par->ffun != GEPI_FFUNC_ENTROPY || (n0 + 127) / 128 + (n1 + 127) / 128 >= F4W_PARK_MIN_KSTEPS);
@@ -603,6 +604,9 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
     else
         HIP_TRY(hipMemcpyAsync(b.perm, perm.data(), perm.size() * 4, hipMemcpyHostToDevice,
                                p->stream));
+    CountArgs ca;
+    memset(&ca, 0, sizeof ca);
+    screen_consts(n0, n1, ca);
     HIP_TRY(hipEventRecord(p->ev0, p->stream));
     if (fp4) {
         const int64_t rows = n_var_pad * 3;
@@ -610,8 +614,8 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
         if (geno) {
             k_class_geno<<<dim3((unsigned)(n_var_pad / 64), (unsigned)n_u + 1), CLSG_THREADS, 0, p->stream>>>(
                 p->d_nat, (int32_t)n_var, p->w64, b.cw,
-                reinterpret_cast<const SuperSrc *>(b.cw + cw_words), n_u, n0 + n1,
-                reinterpret_cast<uint4 *>(b.clsk), reinterpret_cast<float *>(d_pc3));
+                reinterpret_cast<const SuperSrc *>(b.cw + cw_words), n_u, n0,
+                n0 + n1, full ? 3.0f * ca.sc_start : 0.0f, reinterpret_cast<uint4 *>(b.clsk), reinterpret_cast<float *>(d_pc3));
             HIP_TRY(hipGetLastError());
         } else if (n_ks > 0 && path == 3) {
             k_class_f4<3, true><<<cgrid, 256, 0, p->stream>>>(
@@ -653,8 +657,6 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
     };
 
     int cur = 0; /* active candidate buffer */
-    CountArgs ca;
-    memset(&ca, 0, sizeof ca);
     ca.planes = b.cls;
     ca.planes_k = b.clsk;
     ca.pc3 = d_pc3;
@@ -670,8 +672,7 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
     ca.n0 = n0;
     ca.n1 = n1;
     chi2_slope(n0, n1, &ca.h0, &ca.h1);
-    ca.miss = reinterpret_cast<const float *>(d_pc3);
-    screen_consts(n0, n1, ca);
+    ca.miss = reinterpret_cast<const float *>(d_pc3); /* six floats a variant fit */
     ca.st = b.state;
     ca.pend = b.pend;
     ca.pcap = pcap;
@@ -728,7 +729,12 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
         auto go = [&](auto kernel, unsigned threads) {
             hipExtLaunchKernelGGL(kernel, dim3(grid), dim3(threads), 0, p->stream, e0, e1, 0, ca);
         };
-        if (geno) {
+        if (full) {
+            if (entropy)
+                go(k_count_f4c<GEPI_FFUNC_ENTROPY>, F4W_THREADS);
+            else
+                go(k_count_f4c<GEPI_FFUNC_FISHERPV>, F4W_THREADS);
+        } else if (geno) {
             if (entropy)
                 go(k_count_f4g<GEPI_FFUNC_ENTROPY>, F4W_THREADS);
             else
@@ -772,10 +778,14 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
             /* at most PAIRS_WG_PER_CU workgroups per CU, none without work */
             const unsigned grid = std::min<unsigned>((pair_cap + PAIRS_THREADS - 1) / PAIRS_THREADS,
                                                      (unsigned)(PAIRS_WG_PER_CU * device_cus(p->device)));
-            if (entropy)
-                k_pairs<GEPI_FFUNC_ENTROPY><<<grid, PAIRS_THREADS, 0, p->stream>>>(ca);
+            if (entropy && full)
+                k_pairs<GEPI_FFUNC_ENTROPY, 2><<<grid, PAIRS_THREADS, 0, p->stream>>>(ca);
+            else if (entropy)
+                k_pairs<GEPI_FFUNC_ENTROPY, 3><<<grid, PAIRS_THREADS, 0, p->stream>>>(ca);
+            else if (full)
+                k_pairs<GEPI_FFUNC_FISHERPV, 2><<<grid, PAIRS_THREADS, 0, p->stream>>>(ca);
             else
-                k_pairs<GEPI_FFUNC_FISHERPV><<<grid, PAIRS_THREADS, 0, p->stream>>>(ca);
+                k_pairs<GEPI_FFUNC_FISHERPV, 3><<<grid, PAIRS_THREADS, 0, p->stream>>>(ca);
         }
         if (entropy)
             k_exact<GEPI_FFUNC_ENTROPY><<<1024, 256, 0, p->stream>>>(ea);
@@ -1083,7 +1093,7 @@ int upload_planes(gepi_panel *p, const uint64_t *bits, const uint64_t *valid, in
                   int32_t words) {
     const int64_t n_var = n_rows / 2;
     std::vector<uint64_t> nat((size_t)(n_var > 0 ? n_var : 1) * 3 * (words > 0 ? words : 1), 0);
-    uint64_t bare = 0; /* valid calls without an allele */
+    uint64_t bare = 0, lost = 0; /* valid calls without an allele; missing calls */
     for (int64_t v = 0; v < n_var; v++) {
         const uint64_t *b1 = bits + (size_t)(2 * v) * words, *b2 = b1 + words;
         const uint64_t *v1 = valid + (size_t)(2 * v) * words;
@@ -1093,8 +1103,11 @@ int upload_planes(gepi_panel *p, const uint64_t *bits, const uint64_t *valid, in
             o[words + w] = b2[w] & v1[w];
             o[2 * words + w] = v1[w];
             bare |= v1[w] & ~(b1[w] | b2[w]);
+            const int32_t left = p->n_samples - 64 * w;
+            lost |= ~v1[w] & (left >= 64 ? ~0ull : left > 0 ? (1ull << left) - 1ull : 0ull);
         }
     }
+    p->complete = bare == 0 && lost == 0;
     p->three_genotypes = bare == 0;
     /* on the panel's stream, after panel_alloc's zero fill of the same
      * buffer (a null-stream copy would not be ordered with that non-blocking
@@ -1190,8 +1203,11 @@ extern "C" int gepi_panel_create_bed(const uint8_t *bed_payload, int64_t n_varia
         }
         hipMemcpyAsync(d_bed, bed_payload, (size_t)bytes, hipMemcpyHostToDevice, p->stream);
         int64_t threads = n_variants * p->w64;
+        uint32_t *d_any = reinterpret_cast<uint32_t *>(p->d_small), any = 1;
+        hipMemsetAsync(d_any, 0, sizeof(uint32_t), p->stream);
         k_decode_bed<<<(unsigned)((threads + 255) / 256), 256, 0, p->stream>>>(
-            d_bed, n_variants, n_samples, p->w64, bps, p->d_nat);
+            d_bed, n_variants, n_samples, p->w64, bps, p->d_nat, d_any);
+        hipMemcpyAsync(&any, d_any, sizeof any, hipMemcpyDeviceToHost, p->stream);
         hipError_t e = hipStreamSynchronize(p->stream);
         hipError_t e2 = hipGetLastError();
         hipFree(d_bed);
@@ -1200,6 +1216,7 @@ extern "C" int gepi_panel_create_bed(const uint8_t *bed_payload, int64_t n_varia
             return gepi_fail(GEPI_ERR_DEVICE, "bed decode failed: %s",
                              hipGetErrorString(e != hipSuccess ? e : e2));
         }
+        p->complete = any == 0;
     }
     *out = p;
     return GEPI_OK;
@@ -1300,6 +1317,7 @@ extern "C" int gepi_panel_filter(gepi_panel *p, float max_miss_snps, float max_m
     }
     gepi_panel *q = new gepi_panel();
     q->three_genotypes = p->three_genotypes;
+    q->complete = p->complete;
     if ((rc = panel_alloc(q, p->device, (int64_t)keep.size(), p->n_samples)) != GEPI_OK) {
         panel_free(q);
         return rc;

@@ -52,7 +52,8 @@ constexpr int64_t BED_PAD = 32;
 static __global__ void __launch_bounds__(256) k_decode_bed(const uint8_t *__restrict__ bed,
                                                            int64_t n_var, int32_t n_samples,
                                                            int32_t w64, int64_t bps,
-                                                           uint64_t *__restrict__ nat) {
+                                                           uint64_t *__restrict__ nat,
+                                                           uint32_t *__restrict__ any_missing) {
     const int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (gid >= n_var * w64) return;
     const int64_t v = gid / w64;
@@ -74,7 +75,12 @@ static __global__ void __launch_bounds__(256) k_decode_bed(const uint8_t *__rest
     uint64_t *dst = nat + (v * 3) * w64 + wd;
     dst[0] = ~lo & in;              /* codes 0, 2 */
     dst[w64] = hi & in;             /* codes 2, 3 */
-    dst[2 * w64] = (~lo | hi) & in; /* all but 1  */
+    const uint64_t valid = (~lo | hi) & in; /* all but 1  */
+    dst[2 * w64] = valid;
+    /* read first: one line of L2, written by few */
+    if (valid != in &&
+        __hip_atomic_load(any_missing, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u)
+        __hip_atomic_store(any_missing, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 /* out[v][p][d] bit b = panel bit perm[32*d + b] (0 for perm < 0 or v >= n_var). */
@@ -352,14 +358,17 @@ struct SuperSrc {
  * host has located (src), so that a scan's super-steps are made in parallel
  * (one thread for a row's whole sample range took 384 us for 8,000 x 20,001
  * and 38 us for 20,000 x 2,048).  blockIdx.y = n_u: the variants' shares of
- * missing calls among the class samples, rounded up.                       */
+ * missing calls among the class samples, rounded up, or, with margin > 0, the
+ * margins that the products of a panel without missing calls leave out
+ * (F4GMargins), `margin` added to the totals.                              */
 constexpr int CLSG_THREADS = 192;
 static __global__ void __launch_bounds__(CLSG_THREADS)
     k_class_geno(const uint64_t *__restrict__ nat, int32_t n_var, int32_t w64,
                  const CompressWord *__restrict__ cw, const SuperSrc *__restrict__ src, int32_t n_u,
-                 int32_t n, uint4 *__restrict__ out, float *__restrict__ miss) {
+                 int32_t n0, int32_t n, float margin, uint4 *__restrict__ out,
+                 float *__restrict__ miss) {
     __shared__ uint64_t row[2][64][CLS_CHUNK + 1];
-    __shared__ int32_t valid[64];
+    __shared__ int32_t sum[4][64];
     const int tid = threadIdx.x, p = tid >> 6, vl = tid & 63;
     const int32_t v0 = blockIdx.x * 64, u = blockIdx.y;
     auto stage = [&](int32_t w0) {
@@ -373,24 +382,41 @@ static __global__ void __launch_bounds__(CLSG_THREADS)
         __syncthreads();
     };
     if (u == n_u) {
-        if (tid < 64) valid[tid] = 0;
-        int32_t c0 = 0;
+        for (int i = tid; i < 256; i += CLSG_THREADS) sum[i >> 6][i & 63] = 0;
+        /* margin = 0: valid calls; else homozygous 1 and heterozygous, by class */
+        int32_t k[4] = {0, 0, 0, 0};
         for (int32_t w0 = 0; w0 < w64; w0 += CLS_CHUNK) {
             stage(w0);
             const int32_t nw = w64 - w0 < CLS_CHUNK ? w64 - w0 : CLS_CHUNK;
             for (int32_t wd = p; wd < nw; wd += 3) { /* the waves share the words */
-                const uint64_t x = row[0][vl][wd] | row[1][vl][wd];
+                const uint64_t a1 = row[0][vl][wd], a2 = row[1][vl][wd];
                 const CompressWord *a = cw + 2 * (w0 + wd), *b = a + 2 * w64;
-                c0 += __popcll(x & (((uint64_t)a[1].m << 32) | a[0].m)) +
-                      __popcll(x & (((uint64_t)b[1].m << 32) | b[0].m));
+                const uint64_t m0 = ((uint64_t)a[1].m << 32) | a[0].m;
+                const uint64_t m1 = ((uint64_t)b[1].m << 32) | b[0].m;
+                const uint64_t x = margin == 0.0f ? a1 | a2 : a1 & ~a2, y = margin == 0.0f ? 0ull : a1 & a2;
+                k[0] += __popcll(x & m0);
+                k[1] += __popcll(x & m1);
+                k[2] += __popcll(y & m0);
+                k[3] += __popcll(y & m1);
             }
         }
         __syncthreads();
-        atomicAdd(&valid[vl], c0);
+#pragma unroll
+        for (int i = 0; i < 4; i++) atomicAdd(&sum[i][vl], k[i]);
         __syncthreads();
-        if (p == 0 && n > 0)
-            miss[v0 + vl] = (float)(n - valid[vl]) / (float)n * (1.0f + 1e-6f);
-        if (p == 0 && n <= 0) miss[v0 + vl] = 0.0f;
+        if (p != 0) return;
+        const int32_t x0 = sum[0][vl], x1 = sum[1][vl], y0 = sum[2][vl], y1 = sum[3][vl];
+        if (margin == 0.0f) {
+            miss[v0 + vl] = n > 0 ? (float)(n - x0 - x1) / (float)n * (1.0f + 1e-6f) : 0.0f;
+        } else {
+            float *o = miss + (int64_t)(v0 + vl) * 6;
+            o[0] = (float)(x0 + x1) + margin;
+            o[1] = (float)(y0 + y1) + margin;
+            o[2] = (float)(n - x0 - x1 - y0 - y1) + margin;
+            o[3] = (float)x0;
+            o[4] = (float)y0;
+            o[5] = (float)(n0 - x0 - y0);
+        }
         return;
     }
     const SuperSrc s = src[u];
