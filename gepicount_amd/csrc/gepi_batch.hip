@@ -472,7 +472,7 @@ size_t Engine::estimate_footprint(const gepi_panel *p, int64_t topmost) {
     return round_block((size_t)n_u * n_var_pad * 3 * 64 + (size_t)n_var_pad * 6 * sizeof(float)) + round_block(cap * sizeof(Cand)) +
            round_block(pcap * sizeof(Pend)) + round_block((size_t)4 * p->w64 * sizeof(CompressWord)) +
            round_block(sizeof(ScanState)) +
-           round_block((size_t)pair_list_cap(n_var_pad / TM * (n_var_pad / TM + 1), 0, PAIRS_MOST_BATCH) * 48);
+           round_block((size_t)pair_list_cap(n_var_pad / TM * (n_var_pad / TM + 1), 0, PAIRS_MOST_BATCH) * PAIR_BYTES);
 }
 
 void Engine::drop(ScanItem *it, int status) {
@@ -591,7 +591,7 @@ int Engine::add(ScanItem *it) {
     it->d_cand = (Cand *)dalloc(it->cap * sizeof(Cand));
     it->d_state = (ScanState *)dalloc(sizeof(ScanState));
     it->pair_cap = it->geno ? pair_list_cap(it->n_tiles, it->n_k4, PAIRS_MOST_BATCH) : 0u;
-    if (it->pair_cap) it->d_pairs = (uint4 *)dalloc((size_t)it->pair_cap * 48);
+    if (it->pair_cap) it->d_pairs = (uint4 *)dalloc((size_t)it->pair_cap * PAIR_BYTES);
     if (!it->d_layout || !it->d_cw || !it->d_pend || (it->pair_cap && !it->d_pairs) || !it->d_cand || !it->d_state) {
         drop(it, gepi_fail(GEPI_ERR_NOMEM, "device memory for a scan of %lld variants",
                            (long long)it->n_var));
@@ -600,7 +600,7 @@ int Engine::add(ScanItem *it) {
     it->footprint = round_block(lay) + round_block(it->h_cw.size() * sizeof(CompressWord)) +
                     round_block(it->pcap * sizeof(Pend)) + round_block(it->cap * sizeof(Cand)) +
                     round_block(sizeof(ScanState)) +
-                    (it->pair_cap ? round_block((size_t)it->pair_cap * 48) : 0);
+                    (it->pair_cap ? round_block((size_t)it->pair_cap * PAIR_BYTES) : 0);
     HIP_TRY(hipMemcpyAsync(it->d_cw, it->h_cw.data(), it->h_cw.size() * sizeof(CompressWord),
                            hipMemcpyHostToDevice, stream));
     CountArgs ca;

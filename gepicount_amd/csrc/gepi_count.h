@@ -935,11 +935,20 @@ constexpr uint32_t F4W_PAIR_CAP = 1024;
  * from 1,536 on. */
 constexpr int32_t F4W_MIN_KSTEPS = 10;
 /* ... and, on genotype planes, for scans of at least this many 64 x 32 tiles
- * (about 2,900 variants) whatever their samples: against the LDS-staged
- * kernel, whole scans of 64-1,100 samples took 0.71-0.84x the time on 20,000
- * variants (Fisher 0.72-0.80x), 0.81-0.95x (0.91-0.98x) on 4,000 and 0.95-1.09x
- * (1.20-1.33x) on 1,000, where one wave of workgroups is all there is.     */
-constexpr int64_t F4G_MIN_TILES = 2048;
+ * whatever their samples.  Whole scans of 64-1,500 samples, top-100 and
+ * top-1,000, against the LDS-staged kernel: entropy 0.96-1.13x the time on 500
+ * variants, 0.86-1.02x on 1,024 (272 tiles), 0.82-0.98x on 2,800, 0.74-0.90x on
+ * 10,000; Fisher 1.04-1.5x on 2,000 (1,056 tiles), 0.91-1.04x on 2,800-4,000
+ * with top-100, 0.69-0.74x on 20,000.                                       */
+constexpr int64_t F4G_MIN_TILES = 256;
+constexpr int64_t F4G_MIN_TILES_FISHER = 2048;
+/* Fisher's screen loses sqrt(2.55 m) of P(obs), so a long ranking's threshold
+ * passes most pairs through it: it takes the wave tiles where there are at
+ * least this many evaluations for each record of the ranking.  Against the
+ * LDS-staged kernel, 300-8,192 samples: 0.69-0.81x the time at 4e6 (20,000
+ * variants, top-1,000), 0.98x at 1e6, 1.07-1.6x at 4e5 and below; without
+ * missing calls 0.52-0.62x at 4e6, 0.87-1.12x at 4e5, 1.13-1.26x at 4e4.    */
+constexpr double F4G_FISHER_EVALS = 8e5, F4G_FISHER_EVALS_COMPLETE = 4e5;
 /* Entropy scans on wave tiles park flagged pairs from this many K steps of
  * 128 samples (Fisher scans always do).  Measured, entropy top-100 at 20,000
  * variants and top-1,000 at 40,000: parking took 1.13-1.38x the time at 24-40

@@ -68,11 +68,9 @@ struct gepi_panel {
     size_t park_bytes = 0;
     gepi::Cand *d_cand[2] = {nullptr, nullptr};
     gepi::Pend *d_pend = nullptr;
-    uint4 *d_pairs = nullptr;          /* pairs put off by the count kernel   */
-    size_t pairs_bytes = 0;
     unsigned long long buf_cap = 0;  /* records in the candidate buffer  */
     unsigned long long buf2_cap = 0; /* records in the second one        */
-    unsigned long long pend_cap = 0; /* records in the pending list       */
+    size_t pend_bytes = 0;           /* pending list, then pairs put off  */
     gepi::ScanState *d_state = nullptr;
     uint64_t *d_small = nullptr;
     DeviceTables tabs;
@@ -175,7 +173,8 @@ inline void screen_consts(int32_t n0, int32_t n1, gepi::CountArgs &g) {
 }
 
 /* Records of the list of pairs that the count kernel puts off (48 bytes): one
- * for every 4 pairs of the scan, at most `most`, beyond which the kernel tests
+ * for every 4 pairs of the scan (at 16 small scans with loose thresholds took
+ * 1.12x the time: 1,020 x 89, 2,000 x 1,000), at most `most`, beyond which the kernel tests
  * its pairs itself.  None from PAIRS_MAX_KSTEPS K steps on, where the other
  * workgroup of the CU fills the time of a test with its longer K loop: whole
  * scans of 20,000 variants, top-1,000, against tests in the kernel, took 0.90x
@@ -185,6 +184,7 @@ constexpr int PAIRS_WG_PER_CU = 8;
 constexpr int64_t PAIRS_MOST = 1 << 22;       /* single scans: 201 MB          */
 constexpr int64_t PAIRS_MOST_BATCH = 1 << 21; /* a scan of the engine: 101 MB  */
 constexpr int32_t PAIRS_MAX_KSTEPS = 48;
+constexpr size_t PAIR_BYTES = 48;
 inline uint32_t pair_list_cap(int64_t n_tiles, int32_t ks, int64_t most) {
     if (ks > PAIRS_MAX_KSTEPS) return 0;
     return (uint32_t)std::min<int64_t>(std::max<int64_t>(n_tiles * (64 * 32 / 4), 4096), most);
@@ -260,10 +260,13 @@ struct BandPlan {
         if (n_tiles <= 6400 && survivors(n_tiles, share(n_tiles)) <= 600000.0) return n_tiles;
         return std::min<int64_t>(n_tiles, std::max<int64_t>(1024, (int64_t)(share(1) / 4e-5)));
     }
-    /* whether a guess for n tiles tells anything and the lists hold it */
+    /* whether a guess for n tiles tells anything and the lists hold it.  Of
+     * entropy's survivors of the bound only those within a float's margin of
+     * the threshold become records, 1.0-1.2 times the share aimed at (with
+     * all of them counted, 1,024 x 256 top-1,000 ran four bands instead of one)  */
     bool sound(int64_t n, unsigned long long cap) const {
-        return share(n) <= 0.1 && 1.5 * (c + 1.0) * k <= (double)cap &&
-               survivors(n, share(n)) <= most;
+        const double records = entropy ? 1.5 * c * k : survivors(n, share(n));
+        return share(n) <= 0.1 && 1.5 * (c + 1.0) * k <= (double)cap && records <= most;
     }
     void learn(int64_t n, double q, unsigned long long found) {
         factor = std::min(64.0, std::max(0.25, (double)found / std::max(1.0, survivors(n, q))));

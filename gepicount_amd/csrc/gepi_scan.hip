@@ -181,7 +181,6 @@ void panel_free(gepi_panel *p) {
     hipFree(p->d_cand[0]);
     hipFree(p->d_cand[1]);
     hipFree(p->d_pend);
-    hipFree(p->d_pairs);
     hipFree(p->d_state);
     hipFree(p->d_small);
     hipFree(p->tabs.lhi);
@@ -420,16 +419,22 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
     /* fp4: wave tiles from F4W_MIN_KSTEPS K steps on (below, a class's
      * padding K steps, multiplied on the 3-step layout, cost more than the
      * wave tiles save), and on genotype planes, whose screen spares most of
-     * the filter, for any number of samples from F4G_MIN_TILES tiles on.
-     * Without genotype planes Fisher parks the one pair in 8 that it flags
-     * in a global list per workgroup, which the allocation-free scan has no
-     * room for, so there the LDS-staged kernel (parking in LDS) runs Fisher. */
+     * the filter, for any number of samples from F4G_MIN_TILES or
+     * F4G_MIN_TILES_FISHER tiles on; Fisher (above F4G_MIN_TILES) only where
+     * the ranking is short enough for the screen (F4G_FISHER_EVALS).  Without genotype planes
+     * Fisher parks the one pair in 8 that it flags in a global list per
+     * workgroup, which the allocation-free scan has no room for, so there
+     * the LDS-staged kernel (parking in LDS) runs Fisher.                   */
     if (path == 0) {
         const int32_t ks = (n0 + 127) / 128 + (n1 + 127) / 128;
         const bool fisher = par->ffun != GEPI_FFUNC_ENTROPY;
         const int64_t a4 = (n_var + TM - 1) / TM;
-        const bool wide = p->three_genotypes && !noalloc && a4 * (a4 + 1) >= F4G_MIN_TILES;
+        const bool wide = p->three_genotypes && !noalloc &&
+                          a4 * (a4 + 1) >= (fisher ? F4G_MIN_TILES_FISHER : F4G_MIN_TILES);
         path = wide || (ks >= F4W_MIN_KSTEPS && !(fisher && noalloc)) ? 3 : 4;
+        if (fisher && p->three_genotypes && a4 * (a4 + 1) >= F4G_MIN_TILES &&
+            (double)total_evals < (p->complete ? F4G_FISHER_EVALS_COMPLETE : F4G_FISHER_EVALS) * (double)par->topmost)
+            path = 4;
     }
     /* Wave tiles: Fisher scans park flagged variant pairs (its bound flags
      * about one pair in eight), entropy scans from F4W_PARK_MIN_KSTEPS K
@@ -563,11 +568,11 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
         if (fp4 &&
             (rc = grow(&p->d_cw, &p->cw_bytes, cw.size() * sizeof(CompressWord))) != GEPI_OK)
             return rc;
-        if (pair_cap) grown(p->d_pairs, p->pairs_bytes, (size_t)pair_cap * 48);
-        if (pair_cap && (rc = grow(&p->d_pairs, &p->pairs_bytes, (size_t)pair_cap * 48)) != GEPI_OK)
-            return rc;
         if (cap > p->buf_cap) alloc += (int64_t)(sizeof(Cand) * cap);
-        if (pcap > p->pend_cap) alloc += (int64_t)(sizeof(Pend) * pcap);
+        /* the pending list and the pairs put off: one allocation, as a drop-in
+         * call pays for each (two: 1,020 x 89 0.47 -> 0.52 ms)              */
+        const size_t lists = sizeof(Pend) * pcap + (size_t)pair_cap * PAIR_BYTES;
+        grown(p->d_pend, p->pend_bytes, lists);
         if (cap > p->buf_cap) {
             hipFree(p->d_cand[0]);
             p->d_cand[0] = nullptr;
@@ -575,13 +580,7 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
             HIP_TRY(hipMalloc(&p->d_cand[0], sizeof(Cand) * cap));
             p->buf_cap = cap;
         }
-        if (pcap > p->pend_cap) {
-            hipFree(p->d_pend);
-            p->d_pend = nullptr;
-            p->pend_cap = 0;
-            HIP_TRY(hipMalloc(&p->d_pend, sizeof(Pend) * pcap));
-            p->pend_cap = pcap;
-        }
+        if ((rc = grow(&p->d_pend, &p->pend_bytes, lists)) != GEPI_OK) return rc;
         b.cls = p->d_cls;
         b.clsk = p->d_clsk;
         b.perm = p->d_perm;
@@ -676,7 +675,7 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
     ca.st = b.state;
     ca.pend = b.pend;
     ca.pcap = pcap;
-    ca.pairs = pair_cap ? p->d_pairs : nullptr;
+    ca.pairs = pair_cap ? reinterpret_cast<uint4 *>(b.pend + pcap) : nullptr; /* 16-byte records */
     ca.pair_cap = pair_cap;
     ca.park = f4w_park ? p->d_park : nullptr;
     ca.park_busy = f4w_park ? reinterpret_cast<uint32_t *>(
