@@ -536,7 +536,13 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
         pcap = std::max<unsigned long long>((unsigned long long)std::max(atoll(env), 0ll),
                                             (unsigned long long)TILE_EVALS_MAX + 1024);
     }
-    const uint32_t pair_cap = geno && !noalloc ? pair_list_cap(n_tiles, n_ks, PAIRS_MOST) : 0u;
+    /* long rankings (those that are not planned below) pass so many pairs and
+     * records that the second launch costs what it spares: top-1,000,000 of
+     * 20,000 x 2,048 7.4 ms of count launches with the tests in them, 5.7 and
+     * 2.0 with k_pairs                                                      */
+    const double guess = par->ffun == GEPI_FFUNC_ENTROPY ? GUESS_ENTROPY : GUESS_FISHER;
+    const bool short_ranking = (guess + 1.0) * (double)k <= (double)WG_SELECT_MAX;
+    const uint32_t pair_cap = geno && !noalloc && short_ranking ? pair_list_cap(n_tiles, n_ks, PAIRS_MOST) : 0u;
     ScanBufs b;
     if (noalloc) {
         /* the smallest lists that always complete: more, smaller bands */
@@ -800,13 +806,13 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
     plan.evals_tile = (double)evals_per_tile;
     plan.h = (double)ca.h0 + (double)ca.h1 * std::min(n0, n1);
     plan.k = (double)k;
-    plan.c = entropy ? GUESS_ENTROPY : GUESS_FISHER;
+    plan.c = guess;
     plan.most = (double)pcap / 4;
     const int64_t first = plan.first(n_tiles);
     const bool hooks = forced_band || getenv("GEPI_CAND_CAP") || getenv("GEPI_PEND_CAP");
     const bool planned = fp4 && n_ks > 0 && !hooks && !par->intermediate && par->max_grid_area <= 0 &&
                          plan.sound(first, cap) &&
-                         (plan.c + 1.0) * (double)k <= (double)WG_SELECT_MAX;
+                         short_ranking;
     if (planned) {
         if (!p->mail) HIP_TRY(hipHostMalloc(&p->mail, sizeof(HostMail), hipHostMallocDefault));
         HostMail *mail = static_cast<HostMail *>(p->mail);
