@@ -639,7 +639,7 @@ int Engine::add(ScanItem *it) {
     pl.evals_tile = (double)F4_TILE_EVALS;
     pl.h = (double)ca.h0 + (double)ca.h1 * std::min(it->n0, it->n1);
     pl.k = (double)it->k;
-    pl.c = pl.entropy ? GUESS_ENTROPY : GUESS_FISHER;
+    pl.c = pl.entropy ? GUESS_ENTROPY : guess_fisher((double)it->k);
     pl.most = (double)it->pcap / 4;
     it->first = std::min(pl.first(it->n_tiles), it->max_band);
     it->guessed = it->n_k4 > 0 && !it->forced_band && !getenv("GEPI_CAND_CAP") && !getenv("GEPI_PEND_CAP") &&

@@ -213,7 +213,12 @@ inline uint32_t pair_list_cap(int64_t n_tiles, int32_t ks, int64_t most) {
  * fourfold, a host round trip (40 us) and a selection between two: 1,024 x
  * 256 0.73 -> 0.13 ms (5 bands -> 1), 3,001 x 777 Fisher 1.44 -> 0.29, 20,000
  * x 2,048 3.69 -> 2.38 (10 -> 3), 8,000 x 20,001 3.84 -> 2.50.               */
-constexpr double GUESS_ENTROPY = 8.0, GUESS_FISHER = 16.0;
+constexpr double GUESS_ENTROPY = 8.0;
+/* Fisher: 16 for the 100 best, where a few variants decide, down to 4 for long
+ * rankings, whose count varies less: each guessed evaluation that passes the
+ * bound costs a walk over its tables (3,000 x 2,000 top-10,000 1.85 -> 0.7 ms,
+ * 514 x 9,799 top-2,000 1.95 -> 0.75).                                      */
+inline double guess_fisher(double k) { return std::max(4.0, std::min(16.0, 16.0 * std::cbrt(100.0 / k))); }
 constexpr double LOOP_GUESS_ENTROPY = 2.0, LOOP_GUESS_FISHER = 4.0; /* long rankings */
 
 /* P(chi2_1 > t) and its inverse */

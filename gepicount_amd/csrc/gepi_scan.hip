@@ -528,7 +528,8 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
         /* capacity override for exercising the overflow recovery in tests */
         cap = std::max<unsigned long long>((unsigned long long)std::max(atoll(env), 0ll), cap_min);
     }
-    unsigned long long pcap = cap;
+    /* Fisher's bound passes up to nine evaluations for one within the threshold */
+    unsigned long long pcap = par->ffun == GEPI_FFUNC_ENTROPY ? cap : std::max<unsigned long long>(cap, 1ull << 20);
     if (const char *env = getenv("GEPI_PEND_CAP")) {
         /* pending-list capacity override for tests: a list larger than the
          * candidate buffers lets one band admit more candidates than fit,
@@ -540,7 +541,7 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
      * records that the second launch costs what it spares: top-1,000,000 of
      * 20,000 x 2,048 7.4 ms of count launches with the tests in them, 5.7 and
      * 2.0 with k_pairs                                                      */
-    const double guess = par->ffun == GEPI_FFUNC_ENTROPY ? GUESS_ENTROPY : GUESS_FISHER;
+    const double guess = par->ffun == GEPI_FFUNC_ENTROPY ? GUESS_ENTROPY : guess_fisher((double)k);
     const bool short_ranking = (guess + 1.0) * (double)k <= (double)WG_SELECT_MAX;
     const uint32_t pair_cap = geno && !noalloc && short_ranking ? pair_list_cap(n_tiles, n_ks, PAIRS_MOST) : 0u;
     ScanBufs b;
