@@ -202,7 +202,7 @@ def run_mix(args):
         "scan_latency_in_batch_ms": {"p50": lat[len(lat) // 2], "p99": lat[min(len(lat) - 1,
                                                                          int(0.99 * len(lat)))]},
         "roofline": {"bound": "mfma", "kernel": " + ".join(
-                         {3: "k_count_f4w_batch", 4: "k_count_f4_batch"}[cp]
+                         {3: "k_count_f4g_batch", 4: "k_count_f4_batch"}[cp]
                          for cp in sorted(set(st["count_path"] for _, st, _ in res))),
                      "achieved": ops / (k_ms / 1000.0) / 1e12, "peak": FP4_MFMA_PEAK_FLOPS / 1e12,
                      "unit": "TFLOP/s", "frac": ops / (k_ms / 1000.0) / FP4_MFMA_PEAK_FLOPS,
@@ -452,7 +452,7 @@ def main():
     if path in (3, 4):
         ops_total = var_pairs * 9 * 2.0 * (n0 + n1)
         peak, bound, unit, kernel = (FP4_MFMA_PEAK_FLOPS, "mfma", "TFLOP/s",
-                                     "k_count_f4w" if path == 3 else "k_count_f4")
+                                     "k_count_f4g" if path == 3 else "k_count_f4")
     elif path == 2:
         ops_total = var_pairs * 9 * 2.0 * (n0 + n1)
         peak, bound, unit, kernel = INT8_MFMA_PEAK_OPS, "mfma", "TOP/s", "k_count_mfma"
