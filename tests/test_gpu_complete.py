@@ -82,3 +82,14 @@ def test_batch():
         assert status == 0
         assert_same(got, orc.gold_scan(orc.Panel(bits, valid, m0, m1, n), 200, ffun=ffun), "batch")
     eng.close()
+
+
+@pytest.mark.parametrize("ffun", [0, 1])
+def test_without_allocation(ffun):
+    """The margins lie in the scan's fixed scratch there, and no list is kept."""
+    print("case complete noalloc", ffun, flush=True)
+    bits, valid, m0, m1, n = panel(109, 100, 700, 650, 3, 0.0)
+    p = ge.Panel.from_planes(bits, valid, n)
+    got, _ = p.scan_noalloc(m0, m1, topmost=600, ffun=ffun, count_path=3)
+    assert_same(got, orc.gold_scan(orc.Panel(bits, valid, m0, m1, n), 600, ffun=ffun), "noalloc")
+    p.close()
