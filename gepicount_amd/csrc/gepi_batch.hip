@@ -641,7 +641,12 @@ int Engine::add(ScanItem *it) {
     pl.k = (double)it->k;
     pl.c = pl.entropy ? GUESS_ENTROPY : guess_fisher((double)it->k);
     pl.most = (double)it->pcap / 4;
+    if (!pl.entropy) {
+        pl.walks = EXACT_BLOCKS_X * 256;
+        pl.spread = 4.0;
+    }
     it->first = std::min(pl.first(it->n_tiles), it->max_band);
+    it->misjudged = false;
     it->guessed = it->n_k4 > 0 && !it->forced_band && !getenv("GEPI_CAND_CAP") && !getenv("GEPI_PEND_CAP") &&
                   pl.sound(it->first, it->cap);
     int rs;
@@ -711,11 +716,12 @@ int Engine::round(std::vector<ScanItem *> &finished) {
         memset(&e, 0, sizeof e);
         e.e.st = it->d_state;
         e.e.pend = it->d_pend;
-        e.e.pcap = it->pcap;
+        e.e.pcap = it->room();
         e.e.cand = it->d_cand;
         e.e.cap = it->cap;
         e.e.lhi = tabs_.lhi;
         e.e.llo = tabs_.llo;
+        e.e.truncated = it->plan.scored();
         e.ffun = it->ffun;
         TopkDesc &t = td[i];
         t.st = it->d_state;
@@ -727,7 +733,7 @@ int Engine::round(std::vector<ScanItem *> &finished) {
         t.k = (uint32_t)it->k;
         t.ffun = it->ffun;
         t.n_a4 = (int32_t)(it->n_var_pad / TM);
-        t.pad = 0;
+        t.truncated = 1;
     }
     /* per objective: descriptors with the longest K loops first (their
      * workgroups are dispatched first; short ones fill the tail), and the
@@ -796,9 +802,11 @@ int Engine::round(std::vector<ScanItem *> &finished) {
             screen_consts(it->n0, it->n1, d.g);
             d.g.st = it->d_state;
             d.g.pend = it->d_pend;
-            d.g.pcap = it->pcap;
+            d.g.pcap = it->room();
             d.g.pairs = it->d_pairs;
             d.g.pair_cap = it->pair_cap;
+            d.g.watch = it->guessed && it->t0 < it->first ? 1 : 0;
+            d.g.pair_from = it->guessed && it->t0 == 0 ? pairs_from(it->band_used) : 0;
             d.g.lfact = tabs_.lfact;
             if (f == 5) {
                 d.g.park = d_park_;
@@ -919,16 +927,13 @@ int Engine::round(std::vector<ScanItem *> &finished) {
         const ItemReport &r = rep[i];
         const int64_t used = it->band_used;
         it->stats.bands++;
-        if (r.pend_overflow) {
-            it->stats.pend_overflows++;
-            it->band = std::max<int64_t>(1, used / 4);
-            still.push_back(it);
-            continue;
-        }
-        if (r.cand_overflow) {
-            it->stats.cand_overflows++;
+        if (r.pend_overflow || r.cand_overflow) {
+            (r.pend_overflow ? it->stats.pend_overflows : it->stats.cand_overflows)++;
             it->count = r.count;
-            it->band = std::max<int64_t>(1, used / 4);
+            /* a guess that was far too loose (BandPlan::room)              */
+            const double found = std::min((double)it->plan.scored(), (double)it->room());
+            it->band = it->guessed && it->t0 < it->first ? it->plan.again(used, found) : std::max<int64_t>(1, used / 4);
+            it->misjudged = true;
             still.push_back(it);
             continue;
         }
@@ -946,7 +951,7 @@ int Engine::round(std::vector<ScanItem *> &finished) {
                 next, (int64_t)((double)((it->cap - (unsigned long long)it->k) / 2) / adm_rate));
         it->t0 += used;
         int64_t grow = used * 4;
-        if (it->guessed && it->t0 < it->n_tiles) {
+        if (it->guessed && !it->misjudged && it->t0 < it->n_tiles) {
             if (it->t0 == used) it->plan.learn(used, it->plan.share(it->first), r.pend_count);
             grow = it->plan.next(it->t0, it->n_tiles - it->t0);
         }

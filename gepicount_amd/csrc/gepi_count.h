@@ -406,6 +406,7 @@ __device__ __forceinline__ void count_f4_tile(const CountArgs &g, int64_t tile) 
     __shared__ __attribute__((aligned(16))) uint4 lds[2][F4_UNITS];
     __shared__ PendStage stage;
     __shared__ F4Corr corr;
+    __shared__ uint32_t full;
     /* Fisher flags a variant pair in about 13% of lanes: those pairs are
      * parked and finished one per thread after the tile (entropy's few are
      * finished in the lane, and its kernels hold no parking space) */
@@ -414,6 +415,7 @@ __device__ __forceinline__ void count_f4_tile(const CountArgs &g, int64_t tile) 
     PairList *pairs = PARK ? reinterpret_cast<PairList *>(&park) : nullptr;
     stage_init(stage);
     if (PARK && threadIdx.x == 0) pairs->n = 0;
+    if (threadIdx.x == 0) full = band_full(g);
     int32_t ta, tb;
     tile_of_f4(tile, g.n_var_pad / TM, ta, tb);
 
@@ -477,6 +479,7 @@ __device__ __forceinline__ void count_f4_tile(const CountArgs &g, int64_t tile) 
     put(lds[0]);
     fetch(last < 1 ? last : 1);
     __syncthreads();
+    if (full) return;
 
     /* lane's fragment rows: A (i, p) is row (32wa + 16i + l16)*3 + p, B q is
      * row 192 + (16wb + l16)*3 + q; the lane takes 16-byte column lg.      */
@@ -1020,7 +1023,7 @@ struct F4WShared {
  * ((e / 2 NP + p) NP + q) * 64 of the lane's LDS column P.  start: 0, or a
  * fraction that no count rounds away (see count_f4g_unit).                */
 template <int NP>
-__device__ __forceinline__ void f4w_products(const CountArgs &g, int32_t gA, int32_t gB, bool live,
+__device__ __forceinline__ void f4w_products(const CountArgs &g, int32_t gA, int32_t gB, bool &live,
                                              float start, uint32_t *P, v16f (&acc)[NP][NP]) {
     const int lane = threadIdx.x & 63;
     const int32_t u1 = f4_super3(g.ks0), n_u = u1 + f4_super3(g.n_ks - g.ks0);
@@ -1086,6 +1089,8 @@ __device__ __forceinline__ void f4w_products(const CountArgs &g, int32_t gA, int
             }
         }
     };
+    /* a band that is full needs no products (live is false then)           */
+    live = live && !__builtin_amdgcn_readfirstlane((int)band_full(g));
     const int32_t nu_live = live ? n_u : 0;
     const int32_t u1_live = live ? u1 : 0;
     if (live) {
@@ -1128,7 +1133,7 @@ __device__ __forceinline__ void count_f4w_unit(const CountArgs &g, int64_t unit,
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int64_t tile = g.tile_begin + 2 * unit + (wave >> 1);
-    const bool live = tile < g.tile_begin + g.n_tiles;
+    bool live = tile < g.tile_begin + g.n_tiles;
     int32_t ta = 0, tb = 0;
     if (live) tile_of_f4(tile, g.n_var_pad / TM, ta, tb);
     const int32_t gA = 2 * ta + (wave & 1), gB = tb;
@@ -1420,7 +1425,9 @@ __device__ __forceinline__ void pairs_run(const CountArgs &g, uint32_t wg, uint3
     __syncthreads();
     for (uint32_t i = wg * blockDim.x + threadIdx.x; i < n; i += n_wg * blockDim.x) {
         const uint4 *rec = g.pairs + (uint64_t)i * NP;
+        const bool full = band_full(g);
         const uint4 a = rec[0], b = rec[1], d = rec[NP - 1];
+        if (full) break;
         int32_t t[NP * NP], h[NP * NP];
         if constexpr (NP == 2) {
             const uint32_t r[4] = {a.x, a.y, a.z, a.w};
@@ -1452,7 +1459,7 @@ __device__ __forceinline__ void count_f4g_unit(const CountArgs &g, int64_t unit,
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int64_t tile = g.tile_begin + 2 * unit + (wave >> 1);
-    const bool live = tile < g.tile_begin + g.n_tiles;
+    bool live = tile < g.tile_begin + g.n_tiles;
     int32_t ta = 0, tb = 0;
     if (live) tile_of_f4(tile, g.n_var_pad / TM, ta, tb);
     const int32_t gA = 2 * ta + (wave & 1), gB = tb;
@@ -1531,16 +1538,19 @@ __device__ __forceinline__ void count_f4g_unit(const CountArgs &g, int64_t unit,
             }
         }
     }
+    /* every place that is reserved in the list of pairs is written */
+    const bool lists = g.pair_cap > 0 && unit >= g.pair_from;
     __syncthreads(); /* the list and every wave's class-0 counts are written */
     while (true) {
         const uint32_t n = sh.n < (uint32_t)F4G_LIST ? sh.n : (uint32_t)F4G_LIST;
-        if (n > 0 && g.pair_cap > 0) {
+        if (n > 0 && lists) {
             if (threadIdx.x == 0) sh.base = st_add(&g.st->pair_count, (unsigned long long)n);
             __syncthreads();
         }
-        const unsigned long long base = g.pair_cap > 0 ? sh.base : 0ull;
+        const unsigned long long base = lists ? sh.base : (unsigned long long)g.pair_cap;
         for (uint32_t i = threadIdx.x; i < n; i += F4W_THREADS)
             f4g_deal<FFUN, NP>(g, sh, fc, sh.list + i * 5, unit, base + i);
+        if (pend && band_full(g)) pend = 0;
         if (!__syncthreads_or(pend != 0)) break;
         /* the list was full (loose thresholds): the next of the elements left
          * over.  e is uniform here, so the accumulators are read by register

@@ -59,6 +59,11 @@ struct ScanItem {
     bool guessed = false; /* the first band runs under a guessed threshold    */
     BandPlan plan{};
     int64_t first = 0;    /* tiles of that band                               */
+    bool misjudged = false; /* it overflowed a list: it is redone in parts */
+    unsigned long long room() const { /* in the pending list of the next band */
+        if (!guessed || t0 >= first) return pcap;
+        return misjudged ? plan.room_again(pcap) : plan.room(plan.records(first), pcap);
+    }
     unsigned long long cap = 0, pcap = 0, count = 0, exact_total = 0;
     uint4 *d_layout = nullptr;
     gepi::CompressWord *d_cw = nullptr;

@@ -190,6 +190,12 @@ inline uint32_t pair_list_cap(int64_t n_tiles, int32_t ks, int64_t most) {
     return (uint32_t)std::min<int64_t>(std::max<int64_t>(n_tiles * (64 * 32 / 4), 4096), most);
 }
 
+/* Units (two tiles) at the start of a band of n tiles under a guessed
+ * threshold that test their pairs in the kernel, so that a guess far too
+ * loose shows before the list of pairs has filled (band_full): none in a band
+ * whose workgroups are all resident at once.                              */
+inline int32_t pairs_from(int64_t n_tiles) { return n_tiles >= 2048 ? (int32_t)std::min<int64_t>(n_tiles / 512, 64) : 0; }
+
 /* ---- planned bands --------------------------------------------------------
  * A scan's bands need no answer from the device between them: a band's
  * count, exact and top-k launches find the threshold, the lists and an
@@ -205,7 +211,8 @@ inline uint32_t pair_list_cap(int64_t n_tiles, int32_t ks, int64_t most) {
  * evaluations are expected: few enough to be cheap, and if the k best are
  * among them (nearly always: the count says so) the threshold was valid.
  * The others run under the k-th key so far.  A scan that ends with fewer than
- * k records is run again without the guess.  (Guessing the whole scan's
+ * k records is run again without the guess, and a band that finds far more
+ * than expected stops and gives the threshold that it is redone under (room).  (Guessing the whole scan's
  * threshold after the pilot saved 10-15% where it held, but the tail hangs
  * on the few variants with the largest effects of their own: over seeds the
  * k-th key had 0.17 to 2 times the expected evaluations beyond it.)
@@ -240,6 +247,8 @@ struct BandPlan {
     double most;        /* survivors a band may have                         */
     double c;           /* GUESS or LOOP_GUESS of the objective              */
     double factor = 1.0; /* survivors measured over survivors expected       */
+    double spread = 16.0; /* survivors a list takes over those expected (room) */
+    double walks = 65536; /* records scored in little more than one's time     */
 
     /* Expected survivors of the chi-square bound per evaluation under the
      * threshold that admits a share q: its cut is h/2 of the quantile (a few
@@ -269,11 +278,44 @@ struct BandPlan {
      * entropy's survivors of the bound only those within a float's margin of
      * the threshold become records, 1.0-1.2 times the share aimed at (with
      * all of them counted, 1,024 x 256 top-1,000 ran four bands instead of one)  */
+    double records(int64_t n) const { return entropy ? 1.5 * c * k : survivors(n, share(n)); }
     bool sound(int64_t n, unsigned long long cap) const {
-        const double records = entropy ? 1.5 * c * k : survivors(n, share(n));
-        return share(n) <= 0.1 && 1.5 * (c + 1.0) * k <= (double)cap && records <= most;
+        return share(n) <= 0.1 && 1.5 * (c + 1.0) * k <= (double)cap && records(n) <= most;
     }
+    /* Places that a planned band may fill in the pending list (of pcap):
+     * `spread` times what is expected (unrelated phenotypes gave up to 8 times,
+     * with rare alleles and uneven classes).  More of them means a threshold
+     * far too loose: phenotypes that follow ancestry, linked or associated
+     * variants, where nearly every evaluation may pass a guess made for
+     * unrelated ones.  The rest of the band is left out (band_full), the
+     * list's first `scored` records get their scores, the k-th key becomes the
+     * threshold, and the band is redone in pieces.  Phenotypes that follow two
+     * ancestries, against bands that grow from one tile without a guess and
+     * against a guess with full lists: 20,000 x 2,048 entropy top-10,000 22.0
+     * and 168.6 -> 3.6 ms, Fisher top-1,000 6.7 and 124.7 -> 4.5; 3,001 x 777
+     * entropy top-100 1.17 and 12.6 -> 0.66, Fisher 1.44 and 18.3 -> 0.99; 4
+     * scans of 5,000 x 1,000 batched, Fisher top-100, 3.7 and 31.0 -> 3.0.  */
+    unsigned long long room(double expected, unsigned long long pcap) const {
+        return std::min<unsigned long long>(pcap, (unsigned long long)std::max(65536.0, spread * expected));
+    }
+    uint32_t scored() const { return (uint32_t)std::min(walks / 4 + 8.0 * k, 4.0e9); }
+    /* Redoing a band of n tiles after that: the k-th of `found` records lets
+     * through a share of at most k / found, so its first tiles are as many as
+     * pass `aim` evaluations then (at most a quarter: a band of one tile
+     * always fits); the following ones grow fourfold with the threshold.   */
+    double aim() const { return std::max(walks, 2.0 * k); }
+    int64_t again(int64_t n, double found) const {
+        const double tiles = aim() * std::max(1.0, found / k) / evals_tile;
+        return std::max<int64_t>(1, std::min<int64_t>(n / 4, (int64_t)tiles));
+    }
+    unsigned long long room_again(unsigned long long pcap) const {
+        return std::min<unsigned long long>(pcap, (unsigned long long)std::max(4.0 * aim(), gepi::TILE_EVALS_MAX + 1024.0));
+    }
+    /* the threshold that lets through what is expected after `done` tiles */
+    double share_after(int64_t done) const { return 1.3 * k / ((double)done * evals_tile); }
+    /* survivors found in n tiles under the threshold that admits a share q */
     void learn(int64_t n, double q, unsigned long long found) {
+        factor = 1.0;
         factor = std::min(64.0, std::max(0.25, (double)found / std::max(1.0, survivors(n, q))));
     }
     /* Tiles of the band that follows `done` tiles.  About 250,000 survivors
@@ -282,8 +324,7 @@ struct BandPlan {
      * times for entropy (the pairs that pass the screen cost more under an
      * older threshold).                                                     */
     int64_t next(int64_t done, int64_t left) const {
-        const double q = 1.3 * k / ((double)done * evals_tile);
-        const double per = factor * evals_tile * pass(q);
+        const double per = survivors(1, share_after(done));
         const double cheap = std::min(std::max(250000.0 / per, 3.0 * (double)done),
                                       (entropy ? 8.0 : 3.0) * (double)done);
         const double tiles = std::min({cheap, most / per, 1048576.0, (double)left});

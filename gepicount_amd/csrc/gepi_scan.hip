@@ -349,7 +349,7 @@ inline bool wg_select(int path, unsigned long long count) {
 
 TopkDesc topk_desc(const ScanBufs &b, int cur, unsigned long long cap, int64_t k,
                    const gepi_params *par, int64_t t0, int64_t t1, int64_t n_a4,
-                   ItemReport *report = nullptr) {
+                   ItemReport *report = nullptr, bool truncated = false) {
     TopkDesc d;
     memset(&d, 0, sizeof d);
     d.st = b.state;
@@ -361,6 +361,7 @@ TopkDesc topk_desc(const ScanBufs &b, int cur, unsigned long long cap, int64_t k
     d.k = (uint32_t)k;
     d.ffun = par->ffun;
     d.n_a4 = (int32_t)n_a4;
+    d.truncated = truncated;
     return d;
 }
 
@@ -700,6 +701,7 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
     ea.cap = cap;
     ea.lhi = b.lhi;
     ea.llo = b.llo;
+    ea.truncated = 0;
 
     const int64_t evals_per_tile = pairs_per_tile * 20;
     /* Bands grow 4x per band up to 8e9 evaluations (195,000 fp4 tiles): each
@@ -809,6 +811,7 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
     plan.k = (double)k;
     plan.c = guess;
     plan.most = (double)pcap / 4;
+    if (!entropy) plan.spread = 8.0;
     const int64_t first = plan.first(n_tiles);
     const bool hooks = forced_band || getenv("GEPI_CAND_CAP") || getenv("GEPI_PEND_CAP");
     const bool planned = fp4 && n_ks > 0 && !hooks && !par->intermediate && par->max_grid_area <= 0 &&
@@ -825,18 +828,33 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
         const double q = plan.share(first);
         HIP_TRY(init_state(plan.score(q, n0 + n1)));
         ea.cand = b.cand[0];
+        ea.truncated = plan.scored();
+        /* one workgroup selects: lists beyond what it passes over quickly are
+         * the fault of a threshold that is too loose as well               */
+        const unsigned long long cap_plan = std::max<unsigned long long>(
+            {cap_min, std::min(cap, WG_SELECT_MAX), std::min(cap, (unsigned long long)(8.0 * (guess + 1.0) * (double)k))});
+        ea.cap = cap_plan;
         struct Job {
             int64_t t0, t1;
+            unsigned long long room; /* in the pending list */
         };
-        std::vector<Job> jobs(1, Job{0, first}), redo;
+        std::vector<Job> jobs(1, Job{0, first, plan.room(plan.records(first), pcap)}), redo;
+        /* pieces of tiles [c0, c1) that grow fourfold with the threshold */
+        auto pieces = [](std::vector<Job> &to, int64_t c0, int64_t c1, int64_t n, unsigned long long room) {
+            for (int64_t c = c0; c < c1; c += n, n = std::min<int64_t>(1048576, 3 * (c - c0)))
+                to.push_back(Job{c, std::min(c1, c + n), room});
+        };
         int64_t upto = first; /* tiles given to jobs so far */
         while (!jobs.empty()) {
             const int nj = (int)std::min<size_t>(jobs.size(), PLAN_BANDS);
             for (int j = 0; j < nj; j++) {
+                ca.pcap = ea.pcap = jobs[j].room;
+                ca.watch = jobs[j].t0 < first ? 1 : 0;
+                ca.pair_from = jobs[j].t0 == 0 ? pairs_from(jobs[j].t1) : 0;
                 launch_count(jobs[j].t0, jobs[j].t1, p->band_ev[2 * j], p->band_ev[2 * j + 1]);
                 launch_exact();
                 k_topk_one<<<1, TOPK_THREADS, 0, p->stream>>>(topk_desc(
-                    b, 0, cap, k, par, jobs[j].t0, jobs[j].t1, n_a4, &mail->report[j]));
+                    b, 0, cap_plan, k, par, jobs[j].t0, jobs[j].t1, n_a4, &mail->report[j], true));
             }
             HIP_TRY(hipGetLastError());
             /* the records, in case these bands are the last */
@@ -860,23 +878,29 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
                     /* survivors or candidates lost (the band's candidates are
                      * dropped already): redo it in pieces                   */
                     (r.pend_overflow ? st_local.pend_overflows : st_local.cand_overflows)++;
-                    const int64_t n = jobs[j].t1 - jobs[j].t0, piece = std::max<int64_t>(1, n / 4);
-                    for (int64_t c = jobs[j].t0; c < jobs[j].t1; c += piece)
-                        redo.push_back(Job{c, std::min(jobs[j].t1, c + piece)});
+                    const Job &o = jobs[j];
+                    pieces(redo, o.t0, o.t1, plan.again(o.t1 - o.t0, std::min((double)plan.scored(), (double)o.room)),
+                           plan.room_again(pcap));
                 } else {
                     exact_total += r.pend_count;
                 }
             }
-            if (upto < n_tiles) {
-                /* after the pilot: was its threshold sound, how many
-                 * survivors did it have, and the other bands             */
-                if (redo.empty() && count < (unsigned long long)k / 4) break;
-                plan.learn(first, q, mail->report[0].pend_count);
-                for (; upto < n_tiles; upto = redo.back().t1)
-                    redo.push_back(Job{upto, upto + plan.next(upto, n_tiles - upto)});
-            }
+            const Job last = jobs[(size_t)nj - 1];
             redo.insert(redo.end(), jobs.begin() + nj, jobs.end());
             jobs.swap(redo);
+            /* too few under the guessed threshold: run it without */
+            if (jobs.empty() && count < (unsigned long long)(upto < n_tiles ? k / 4 : k)) break;
+            if (jobs.empty() && upto < n_tiles) {
+                /* after the pilot: how many survivors it had, and the
+                 * other bands                                            */
+                plan.learn(last.t1 - last.t0, last.t0 > 0 ? plan.share_after(last.t0) : q,
+                           mail->report[nj - 1].pend_count);
+                while (upto < n_tiles) {
+                    const int64_t n = plan.next(upto, n_tiles - upto);
+                    jobs.push_back(Job{upto, upto + n, plan.room((double)n * plan.survivors(1, plan.share_after(upto)), pcap)});
+                    upto += n;
+                }
+            }
             if (jobs.empty() && count == (unsigned long long)k) {
                 if (k <= SORT_HOST_MAX) host.resize((size_t)k);
                 if (by_mail)
@@ -888,6 +912,10 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
                 finished = true;
             }
         }
+        ea.truncated = 0;
+        ca.watch = ca.pair_from = 0;
+        ca.pcap = ea.pcap = pcap;
+        ea.cap = cap;
         /* fewer than k records under the guessed threshold: run it without */
         if (!finished) count = exact_total = 0;
     }

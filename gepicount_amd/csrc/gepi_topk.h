@@ -23,16 +23,18 @@ struct ExactArgs {
     Cand *cand;
     unsigned long long cap;
     const double *lhi, *llo;
+    uint32_t truncated; /* records to score of a list that overflowed (TopkDesc) */
 };
 
 /* Exact score of pending evaluations [start, n) with the given stride;
- * admits keys <= the threshold.  Nothing when the pending list overflowed. */
+ * admits keys <= the threshold.  When the pending list overflowed, its first
+ * e.truncated records (all its pcap places are written then).              */
 template <int FFUN>
 __device__ __forceinline__ void exact_range(const ExactArgs &e, unsigned long long start,
                                             unsigned long long stride) {
-    if (e.st->pend_overflow) return;
     unsigned long long n = e.st->pend_count;
     if (n > e.pcap) n = e.pcap;
+    if (e.st->pend_overflow && n > e.truncated) n = e.truncated;
     const double thr_s = e.st->thr_score;
     const uint64_t thr_i = e.st->thr_idx;
     for (unsigned long long i = start; i < n; i += stride) {
@@ -53,6 +55,7 @@ __device__ __forceinline__ void exact_range(const ExactArgs &e, unsigned long lo
                 e.cand[pos] = c;
             } else {
                 atomicOr(&e.st->overflow, 1u);
+                return; /* the band is redone */
             }
         }
     }
@@ -69,6 +72,7 @@ static __global__ void k_reset_pending(ScanState *st) {
     if (threadIdx.x != 0) return;
     st->pend_count = 0;
     st->pend_overflow = 0;
+    st->full = 0;
     st->pair_count = 0;
 }
 
@@ -317,7 +321,8 @@ struct TopkDesc {
     uint32_t k;
     int32_t ffun;
     int32_t n_a4;             /* A blocks of the scan (fp4 tile numbering)    */
-    int32_t pad;
+    int32_t truncated;        /* of an overflowed pending list the first records
+                               * were scored: their k-th key is a threshold    */
 };
 
 constexpr int TOPK_THREADS = 1024;
@@ -338,11 +343,13 @@ __device__ __forceinline__ uint32_t wide_digit(uint64_t hi, uint64_t lo, uint32_
 }
 
 /* Top-k maintenance of one scan by one 1024-thread workgroup: after a
- * candidate overflow, the k-th key among the records kept becomes the
- * threshold and the band's records (fp4 tile numbering) are dropped (the
- * band is redone); otherwise, with more than k candidates, exactly the k
- * smallest keys are kept, compacted in place (in no order).  Resets the
- * pending list for the next round; writes a report when d.report is set.
+ * candidate overflow, or one of a pending list that was scored truncated,
+ * the k-th key among the records kept (if there are k: it belongs to a real
+ * evaluation, so no better one is lost) becomes the threshold and the band's
+ * records (fp4 tile numbering) are dropped (the band is redone); otherwise,
+ * with more than k candidates, exactly the k smallest keys are kept,
+ * compacted in place (in no order).  Resets the pending list for the next
+ * round; writes a report when d.report is set.
  *
  * One CU, so its latencies are what it costs: per pass the bins are summed
  * by all threads (one thread reading 256 bins in turn took 7 us), the last
@@ -364,17 +371,20 @@ __device__ __forceinline__ void topk_wg_body(const TopkDesc &d) {
     const unsigned long long pend_n = st->pend_count;
     __syncthreads(); /* every thread has read the state before it changes */
     const unsigned long long n = raw < d.cap ? raw : d.cap;
-    const bool work = !pend_ovf && (cand_ovf || n > d.k);
+    const bool lost = pend_ovf && !d.truncated;         /* nothing was scored  */
+    const bool drop = !lost && (pend_ovf || cand_ovf);  /* this band's records */
+    const bool work = !lost && (drop || n > d.k);
     if (work) {
+        const bool pick = n >= d.k;
         if (t == 0) {
-            s_hi = 0;
-            s_lo = 0;
+            s_hi = pick ? 0 : ~0ull;
+            s_lo = pick ? 0 : ~0ull;
             s_bits = 0;
             s_rank = d.k;
             s_done = 0;
         }
         /* radix select of the k-th smallest key, digits MSB first */
-        while (true) {
+        while (pick) {
             for (int i = t; i < TOPK_BINS; i += TOPK_THREADS) hist[i] = 0;
             __syncthreads();
             SelPrefix pre;
@@ -427,7 +437,7 @@ __device__ __forceinline__ void topk_wg_body(const TopkDesc &d) {
             __syncthreads();
             if (s_done) break;
         }
-        if (s_done == 2) {
+        if (pick && s_done == 2) {
             /* the remaining matching keys fit in LDS: each is ranked by
              * counting the smaller ones (keys are distinct) */
             SelPrefix pre;
@@ -462,6 +472,7 @@ __device__ __forceinline__ void topk_wg_body(const TopkDesc &d) {
         }
         /* in-place compaction: a chunk is read before any of it is written,
          * and writes never pass the read position */
+        if (!pick) __syncthreads(); /* s_hi and s_lo are written */
         const uint64_t khi = s_hi, klo = s_lo;
         if (t == 0) s_wptr = 0;
         constexpr int PER = 4;
@@ -477,7 +488,7 @@ __device__ __forceinline__ void topk_wg_body(const TopkDesc &d) {
             for (int j = 0; j < PER; j++) {
                 const unsigned long long i = base + (unsigned)(j * TOPK_THREADS + t);
                 bool kp = i < n && key_le(order_bits(c[j].score), c[j].idx, khi, klo);
-                if (kp && cand_ovf) {
+                if (kp && drop) {
                     const int64_t a = (int64_t)(c[j].idx >> 32) >> 1;
                     const int64_t b = (int64_t)((c[j].idx >> 3) & 0x1FFFFFFFull) >> 1;
                     const int64_t tl = tile_index(a, b, TM, d.n_a4);
@@ -501,14 +512,14 @@ __device__ __forceinline__ void topk_wg_body(const TopkDesc &d) {
             st->count = s_wptr;
             st->count2 = 0;
             st->overflow = 0;
-            adopt_threshold(st, khi, klo, d.ffun);
+            if (pick) adopt_threshold(st, khi, klo, d.ffun);
         }
     }
     if (t == 0) {
         if (d.report) {
         ItemReport r;
         r.raw_count = raw;
-        r.count = work ? s_wptr : (pend_ovf ? raw : n);
+        r.count = work ? s_wptr : n;
         r.pend_count = pend_n;
         r.pend_overflow = pend_ovf;
         r.cand_overflow = pend_ovf ? 0u : cand_ovf;
@@ -516,6 +527,7 @@ __device__ __forceinline__ void topk_wg_body(const TopkDesc &d) {
         }
         st->pend_count = 0;
         st->pend_overflow = 0;
+        st->full = 0;
         st->pair_count = 0;
     }
 }
