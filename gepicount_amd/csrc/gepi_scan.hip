@@ -517,20 +517,59 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
      * one-tile band admits at most TILE_EVALS_MAX, so cap >= k +
      * TILE_EVALS_MAX lets a band shrunk to one tile always complete.        */
     const unsigned long long cap_min = (unsigned long long)k + TILE_EVALS_MAX + 1024;
-    /* 4k or 2^23 records, for k up to 16,384 no more than a 64th of the evaluations:
-     * bands are sized for the lists, and a drop-in call allocates them anew
-     * (a list of 2^23 records cost 0.5 ms to allocate and free, with 80 bytes
-     * a record three fifths of a 1,020 x 89 call)                           */
-    unsigned long long cap = std::max<unsigned long long>(
+    /* 4k or 2^23 records where bands are sized from what they find (for short
+     * rankings no more than there are evaluations).  A planned scan's bands are sized for the
+     * lists and a drop-in call allocates them anew, so for k up to 16,384 those
+     * hold 64k or a 64th of the evaluations (a list of 2^23 records cost 0.5 ms
+     * to allocate and free, with 80 bytes a record three fifths of a 1,020 x 89
+     * call); one whose guess fails grows them.                             */
+    const unsigned long long cap_full = std::max<unsigned long long>(
+        cap_min, k > 16384 ? (unsigned long long)std::max<int64_t>(4 * k, 1 << 23)
+                           : (unsigned long long)std::min<int64_t>(total_evals, 1 << 23));
+    const unsigned long long cap_small = std::max<unsigned long long>(
         cap_min, std::min<unsigned long long>(
-                     (unsigned long long)std::max<int64_t>(4 * k, 1 << 23),
-                     std::max<unsigned long long>({(unsigned long long)total_evals / 64, k > 16384 ? 1ull << 23 : 1ull << 18})));
+                     cap_full, std::max<unsigned long long>({(unsigned long long)total_evals / 64,
+                                                             k > 16384 ? 1ull << 23 : 64ull * (unsigned long long)k,
+                                                             1ull << 18})));
+    const bool entropy = par->ffun == GEPI_FFUNC_ENTROPY;
+    /* Fisher's bound passes up to nine evaluations for one within the threshold */
+    auto pend_cap = [&](unsigned long long c) {
+        return entropy || noalloc ? c : std::max<unsigned long long>(c, 1ull << 20);
+    };
+    /* noalloc: the smallest lists that always complete: more, smaller bands */
+    unsigned long long cap = noalloc ? cap_min : cap_small, pcap = pend_cap(cap);
+    /* all bands enqueued at once (BandPlan): fp4, rankings that one workgroup
+     * selects */
+    const int64_t evals_per_tile = pairs_per_tile * 20;
+    /* band-size override for exercising the overflow recovery in tests: the
+     * first band and the growth limit, ignoring the survivor-rate estimate */
+    int64_t forced_band = 0;
+    if (const char *env = getenv("GEPI_BAND_TILES")) forced_band = std::max<long long>(1, atoll(env));
+    const bool hooks = forced_band || getenv("GEPI_CAND_CAP") || getenv("GEPI_PEND_CAP");
+    const double guess = entropy ? GUESS_ENTROPY : guess_fisher((double)k);
+    const bool short_ranking = (guess + 1.0) * (double)k <= (double)WG_SELECT_MAX;
+    float h0, h1;
+    chi2_slope(n0, n1, &h0, &h1);
+    BandPlan plan;
+    plan.entropy = entropy;
+    plan.evals_tile = (double)evals_per_tile;
+    plan.h = (double)h0 + (double)h1 * std::min(n0, n1);
+    plan.k = (double)k;
+    plan.c = guess;
+    plan.most = (double)pcap / 4;
+    if (!entropy) plan.spread = 8.0;
+    const int64_t first = plan.first(n_tiles);
+    const bool planned = fp4 && n_ks > 0 && !hooks && !par->intermediate && par->max_grid_area <= 0 &&
+                         plan.sound(first, cap) && short_ranking;
+    if (!planned && !noalloc) {
+        cap = cap_full;
+        pcap = pend_cap(cap);
+    }
     if (const char *env = getenv("GEPI_CAND_CAP")) {
         /* capacity override for exercising the overflow recovery in tests */
         cap = std::max<unsigned long long>((unsigned long long)std::max(atoll(env), 0ll), cap_min);
+        pcap = pend_cap(cap);
     }
-    /* Fisher's bound passes up to nine evaluations for one within the threshold */
-    unsigned long long pcap = par->ffun == GEPI_FFUNC_ENTROPY ? cap : std::max<unsigned long long>(cap, 1ull << 20);
     if (const char *env = getenv("GEPI_PEND_CAP")) {
         /* pending-list capacity override for tests: a list larger than the
          * candidate buffers lets one band admit more candidates than fit,
@@ -538,16 +577,33 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
         pcap = std::max<unsigned long long>((unsigned long long)std::max(atoll(env), 0ll),
                                             (unsigned long long)TILE_EVALS_MAX + 1024);
     }
-    /* long rankings (those that are not planned below) pass so many pairs and
+    /* long rankings (those that are not planned) pass so many pairs and
      * records that the second launch costs what it spares: top-1,000,000 of
      * 20,000 x 2,048 7.4 ms of count launches with the tests in them, 5.7 and
      * 2.0 with k_pairs                                                      */
-    const double guess = par->ffun == GEPI_FFUNC_ENTROPY ? GUESS_ENTROPY : guess_fisher((double)k);
-    const bool short_ranking = (guess + 1.0) * (double)k <= (double)WG_SELECT_MAX;
     const uint32_t pair_cap = geno && !noalloc && short_ranking ? pair_list_cap(n_tiles, n_ks, PAIRS_MOST) : 0u;
     ScanBufs b;
+    /* the candidate and pending lists of cap and pcap records, the pairs put
+     * off after the latter: one allocation, as a drop-in call pays for each
+     * (two: 1,020 x 89 0.47 -> 0.52 ms)                                     */
+    auto grow_lists = [&]() -> int {
+        if (cap > p->buf_cap) {
+            st_local.bytes_allocated += (int64_t)(sizeof(Cand) * cap);
+            hipFree(p->d_cand[0]);
+            p->d_cand[0] = nullptr;
+            p->buf_cap = 0;
+            HIP_TRY(hipMalloc(&p->d_cand[0], sizeof(Cand) * cap));
+            p->buf_cap = cap;
+        }
+        const size_t lists = sizeof(Pend) * pcap + (size_t)pair_cap * PAIR_BYTES;
+        if (lists > p->pend_bytes || !p->d_pend) st_local.bytes_allocated += (int64_t)lists;
+        int e;
+        if ((e = grow(&p->d_pend, &p->pend_bytes, lists)) != GEPI_OK) return e;
+        b.cand[0] = p->d_cand[0];
+        b.pend = p->d_pend;
+        return GEPI_OK;
+    };
     if (noalloc) {
-        /* the smallest lists that always complete: more, smaller bands */
         cap = pcap = cap_min;
         if ((rc = bind_scratch(p, b, n0 + n1 + 1, cw.size() * sizeof(CompressWord), clsk_bytes,
                                cap, pcap)) != GEPI_OK)
@@ -576,25 +632,11 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
         if (fp4 &&
             (rc = grow(&p->d_cw, &p->cw_bytes, cw.size() * sizeof(CompressWord))) != GEPI_OK)
             return rc;
-        if (cap > p->buf_cap) alloc += (int64_t)(sizeof(Cand) * cap);
-        /* the pending list and the pairs put off: one allocation, as a drop-in
-         * call pays for each (two: 1,020 x 89 0.47 -> 0.52 ms)              */
-        const size_t lists = sizeof(Pend) * pcap + (size_t)pair_cap * PAIR_BYTES;
-        grown(p->d_pend, p->pend_bytes, lists);
-        if (cap > p->buf_cap) {
-            hipFree(p->d_cand[0]);
-            p->d_cand[0] = nullptr;
-            p->buf_cap = 0;
-            HIP_TRY(hipMalloc(&p->d_cand[0], sizeof(Cand) * cap));
-            p->buf_cap = cap;
-        }
-        if ((rc = grow(&p->d_pend, &p->pend_bytes, lists)) != GEPI_OK) return rc;
+        if ((rc = grow_lists()) != GEPI_OK) return rc;
         b.cls = p->d_cls;
         b.clsk = p->d_clsk;
         b.perm = p->d_perm;
         b.cw = p->d_cw;
-        b.cand[0] = p->d_cand[0];
-        b.pend = p->d_pend;
         b.state = p->d_state;
         b.small = p->d_small;
         b.lhi = p->tabs.lhi;
@@ -678,12 +720,10 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
     ca.f32 = f32_counts(n0, n1) ? 1 : 0;
     ca.n0 = n0;
     ca.n1 = n1;
-    chi2_slope(n0, n1, &ca.h0, &ca.h1);
+    ca.h0 = h0;
+    ca.h1 = h1;
     ca.miss = reinterpret_cast<const float *>(d_pc3); /* six floats a variant fit */
     ca.st = b.state;
-    ca.pend = b.pend;
-    ca.pcap = pcap;
-    ca.pairs = pair_cap ? reinterpret_cast<uint4 *>(b.pend + pcap) : nullptr; /* 16-byte records */
     ca.pair_cap = pair_cap;
     ca.park = f4w_park ? p->d_park : nullptr;
     ca.park_busy = f4w_park ? reinterpret_cast<uint32_t *>(
@@ -696,15 +736,21 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
     ca.lfact = b.lfact;
     ExactArgs ea;
     ea.st = b.state;
-    ea.pend = b.pend;
-    ea.pcap = pcap;
-    ea.cap = cap;
+    auto set_lists = [&]() {
+        ca.pend = b.pend;
+        ca.pcap = pcap;
+        ca.pairs = pair_cap ? reinterpret_cast<uint4 *>(b.pend + pcap) : nullptr; /* 16-byte records */
+        ea.pend = b.pend;
+        ea.pcap = pcap;
+        ea.cap = cap;
+    };
+    set_lists();
     ea.lhi = b.lhi;
     ea.llo = b.llo;
     ea.truncated = 0;
 
-    const int64_t evals_per_tile = pairs_per_tile * 20;
-    /* Bands grow 4x per band up to 8e9 evaluations (195,000 fp4 tiles): each
+    /* Bands grow 8x per band while they are small (a round trip is most of
+     * them), then 4x, up to 8e9 evaluations (195,000 fp4 tiles): each
      * band costs a threshold selection and a host round trip (~0.2 ms), and
      * at the final threshold a band's survivors stay far below the pending
      * list (the next band is also sized from the measured survivor rate). */
@@ -712,18 +758,11 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
     if (par->max_grid_area > 0)
         max_band = std::max<int64_t>(1, ((int64_t)par->max_grid_area << 20) / evals_per_tile);
     int64_t band = std::max<int64_t>(1, std::min<int64_t>(max_band, (2 * k) / evals_per_tile + 1));
-    /* band-size override for exercising the overflow recovery in tests: the
-     * first band and the growth limit, ignoring the survivor-rate estimate */
-    int64_t forced_band = 0;
-    if (const char *env = getenv("GEPI_BAND_TILES")) {
-        forced_band = std::max<long long>(1, atoll(env));
-        band = forced_band;
-    }
+    if (forced_band) band = forced_band;
     double ms_count = 0.0, ms_top = 0.0;
     int64_t t0 = 0;
     unsigned long long count = 0, exact_total = 0;
     int bands = 0;
-    const bool entropy = par->ffun == GEPI_FFUNC_ENTROPY;
     /* fp4: the filter runs on the fp32 accumulators when every product of a
      * class-0 and a class-1 count is exact in float */
     const bool f32 = ca.f32 != 0;
@@ -804,19 +843,6 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
     /* ---- all bands enqueued at once (fp4, small k) ---- */
     std::vector<Cand> host;
     bool finished = false, prepare_read = false;
-    BandPlan plan;
-    plan.entropy = entropy;
-    plan.evals_tile = (double)evals_per_tile;
-    plan.h = (double)ca.h0 + (double)ca.h1 * std::min(n0, n1);
-    plan.k = (double)k;
-    plan.c = guess;
-    plan.most = (double)pcap / 4;
-    if (!entropy) plan.spread = 8.0;
-    const int64_t first = plan.first(n_tiles);
-    const bool hooks = forced_band || getenv("GEPI_CAND_CAP") || getenv("GEPI_PEND_CAP");
-    const bool planned = fp4 && n_ks > 0 && !hooks && !par->intermediate && par->max_grid_area <= 0 &&
-                         plan.sound(first, cap) &&
-                         short_ranking;
     if (planned) {
         if (!p->mail) HIP_TRY(hipHostMalloc(&p->mail, sizeof(HostMail), hipHostMallocDefault));
         HostMail *mail = static_cast<HostMail *>(p->mail);
@@ -825,7 +851,7 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
             HIP_TRY(hipEventCreate(&e));
             p->band_ev.push_back(e);
         }
-        const double q = plan.share(first);
+        double q = plan.share(first);
         HIP_TRY(init_state(plan.score(q, n0 + n1)));
         ea.cand = b.cand[0];
         ea.truncated = plan.scored();
@@ -845,6 +871,7 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
                 to.push_back(Job{c, std::min(c1, c + n), room});
         };
         int64_t upto = first; /* tiles given to jobs so far */
+        bool looser = false;
         while (!jobs.empty()) {
             const int nj = (int)std::min<size_t>(jobs.size(), PLAN_BANDS);
             for (int j = 0; j < nj; j++) {
@@ -888,8 +915,20 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
             const Job last = jobs[(size_t)nj - 1];
             redo.insert(redo.end(), jobs.begin() + nj, jobs.end());
             jobs.swap(redo);
-            /* too few under the guessed threshold: run it without */
-            if (jobs.empty() && count < (unsigned long long)(upto < n_tiles ? k / 4 : k)) break;
+            if (jobs.empty() && count < (unsigned long long)(upto < n_tiles ? k / 4 : k)) {
+                /* too few under the guessed threshold: once more under one
+                 * that is looser by what is missing, if that is not far off
+                 * (alleles of 1%: 1,024 x 256 Fisher top-100 0.78 -> 0.19 ms),
+                 * else without one                                       */
+                if (looser || 32 * count < (unsigned long long)k || q * 4.0 * (double)k > 0.1 * (double)count) break;
+                looser = true;
+                q *= 4.0 * (double)k / (double)count;
+                HIP_TRY(init_state(plan.score(q, n0 + n1)));
+                exact_total = 0;
+                upto = first;
+                jobs.push_back(Job{0, first, plan.room(plan.records(first), pcap)});
+                continue;
+            }
             if (jobs.empty() && upto < n_tiles) {
                 /* after the pilot: how many survivors it had, and the
                  * other bands                                            */
@@ -914,15 +953,22 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
         }
         ea.truncated = 0;
         ca.watch = ca.pair_from = 0;
-        ca.pcap = ea.pcap = pcap;
-        ea.cap = cap;
-        /* fewer than k records under the guessed threshold: run it without */
-        if (!finished) count = exact_total = 0;
+        if (!finished) {
+            count = exact_total = 0;
+            if (!noalloc && cap < cap_full) {
+                cap = cap_full;
+                pcap = pend_cap(cap);
+                if ((rc = grow_lists()) != GEPI_OK) return rc;
+            }
+        }
+        set_lists();
     }
     if (!finished) {
         HIP_TRY(init_state(INFINITY));
-        HIP_TRY(hipStreamSynchronize(p->stream));
-        if (!prepare_read) read_prepare();
+        if (!prepare_read) {
+            HIP_TRY(hipStreamSynchronize(p->stream));
+            read_prepare();
+        }
     } else {
         t0 = n_tiles;
     }
@@ -1036,7 +1082,7 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
                             (double)(t1 - t0);
         const int64_t room = (int64_t)(cap - (unsigned long long)k) / 2;
         const int64_t next = rate > 0.0 ? (int64_t)((double)room / rate) : max_band;
-        band = std::max<int64_t>(1, std::min<int64_t>({max_band, next, band * 4}));
+        band = std::max<int64_t>(1, std::min<int64_t>({max_band, next, band * (band < 64 ? 8 : 4)}));
         if (forced_band) band = std::min<int64_t>(forced_band, (t1 - t0) * 4);
         t0 = t1;
         if (loop_guess && t0 < n_tiles && count == (unsigned long long)k)

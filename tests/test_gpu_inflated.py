@@ -54,6 +54,35 @@ def test_ancestry(monkeypatch, n_var, n, k, ffun, noalloc):
     assert st["bands"] <= 24, st
 
 
+@pytest.mark.parametrize("ffun", [0, 1])
+@pytest.mark.parametrize("k", [200, 10000])
+def test_monomorphic(monkeypatch, k, ffun):
+    print("case monomorphic", k, ffun, flush=True)
+    bits, valid, m0, m1 = monomorphic_panel(43, 1500, 130, 90)
+    with ge.Panel.from_planes(bits, valid, 130) as panel:
+        got, st = panel.scan(m0, m1, topmost=k, ffun=ffun)
+        ref, _ = band_by_band(monkeypatch, panel, m0, m1, k, ffun, 64)
+    assert_same(got, ref, "monomorphic")
+    assert st["bands"] <= 12, st
+
+
+@pytest.mark.parametrize("ffun", [0, 1])
+def test_rare(monkeypatch, ffun):
+    """Alleles of at most 1%, whose scores are few and far apart: the guess finds
+    a part of the ranking (a looser one follows) or next to nothing of it."""
+    print("case rare", ffun, flush=True)
+    rng = np.random.default_rng(5)
+    f = rng.uniform(0.002, 0.01, 1024)[:, None]
+    g = (rng.random((1024, 256)) < f).astype(np.uint8) + (rng.random((1024, 256)) < f)
+    bits, valid = orc.planes_from_codes(np.array([3, 2, 0], np.uint8)[g])
+    m0, m1 = orc.masks_from_classes((rng.random(256) < 0.4).astype(int))
+    with ge.Panel.from_planes(bits, valid, 256) as panel:
+        got, st = panel.scan(m0, m1, topmost=100, ffun=ffun)
+        ref, _ = band_by_band(monkeypatch, panel, m0, m1, 100, ffun, 64)
+    assert_same(got, ref, "rare")
+    assert st["bands"] <= 6, st
+
+
 def test_batch():
     """Guesses that overflow and that fail next to ones that hold, both
     objectives, on allele and genotype planes, in one batch."""
