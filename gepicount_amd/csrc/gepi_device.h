@@ -27,6 +27,21 @@ struct Cand {
     uint32_t w, x, y, z;
 };
 
+/* A record read or written field by field: as a copy of the struct half of an
+ * array of them stays in private memory, and the runtime allocates device
+ * memory for a queue's first kernel with any (24 MiB here).               */
+__device__ __forceinline__ Cand load_cand(const Cand *p) {
+    return Cand{p->score, p->idx, p->w, p->x, p->y, p->z};
+}
+__device__ __forceinline__ void store_cand(Cand *p, const Cand &c) {
+    p->score = c.score;
+    p->idx = c.idx;
+    p->w = c.w;
+    p->x = c.x;
+    p->y = c.y;
+    p->z = c.z;
+}
+
 /* An evaluation that passed the single-precision filter.  16 bytes. */
 struct Pend {
     uint16_t w, x, y, z;

@@ -107,7 +107,7 @@ static __global__ void __launch_bounds__(SORT_THREADS)
     for (int u = 0; u < SORT_PER; u++) {
         const int i = threadIdx.x + u * SORT_THREADS;
         if (i < (int)dn) {
-            c[u] = i < ca ? a[a0 + i] : b[b0 + i - ca];
+            c[u] = load_cand(i < ca ? a + a0 + i : b + b0 + i - ca);
             const SortKey k = key_of(c[u]);
             hi[i] = k.hi;
             lo[i] = k.lo;
@@ -129,7 +129,7 @@ static __global__ void __launch_bounds__(SORT_THREADS)
             else
                 h = mid;
         }
-        dst[o0 + (i < ca ? i : i - ca) + l] = c[u];
+        store_cand(dst + o0 + (i < ca ? i : i - ca) + l, c[u]);
     }
 }
 

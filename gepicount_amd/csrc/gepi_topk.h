@@ -219,7 +219,7 @@ static __global__ void __launch_bounds__(256) k_compact(const Cand *__restrict__
         for (int j = 0; j < COMPACT_PER; j++) {
             const unsigned long long i = base + j * 256u + threadIdx.x;
             if (i >= n) continue;
-            c[j] = src[i];
+            c[j] = load_cand(src + i);
             const uint64_t hi = order_bits(c[j].score);
             bool kp = hi < khi || (hi == khi && c[j].idx <= klo);
             if (kp && drop_t1 > drop_t0) {
@@ -236,7 +236,7 @@ static __global__ void __launch_bounds__(256) k_compact(const Cand *__restrict__
         __syncthreads();
 #pragma unroll
         for (int j = 0; j < COMPACT_PER; j++)
-            if ((keep >> j) & 1u) dst[s_base + at++] = c[j];
+            if ((keep >> j) & 1u) store_cand(dst + s_base + at++, c[j]);
         __syncthreads();
     }
 }
@@ -482,7 +482,7 @@ __device__ __forceinline__ void topk_wg_body(const TopkDesc &d) {
 #pragma unroll
             for (int j = 0; j < PER; j++) {
                 const unsigned long long i = base + (unsigned)(j * TOPK_THREADS + t);
-                if (i < n) c[j] = d.cand[i];
+                if (i < n) c[j] = load_cand(d.cand + i);
             }
 #pragma unroll
             for (int j = 0; j < PER; j++) {
@@ -504,7 +504,7 @@ __device__ __forceinline__ void topk_wg_body(const TopkDesc &d) {
                 uint32_t w0 = 0;
                 if (lane == 0 && m) w0 = atomicAdd(&s_wptr, (uint32_t)__popcll(m));
                 w0 = __shfl(w0, 0);
-                if (kp) d.cand[w0 + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = c[j];
+                if (kp) store_cand(d.cand + w0 + (uint32_t)__popcll(m & ((1ull << lane) - 1ull)), c[j]);
             }
         }
         __syncthreads();

@@ -97,3 +97,31 @@ def test_noalloc_rejects_what_does_not_fit():
         got, _ = h.scan_noalloc(m0, m1, topmost=100)
         ref, _ = h.scan(m0, m1, topmost=100)
         assert_same(got, ref, "after rejection")
+
+
+def fresh_panels(count):
+    """Panels that no scan has run on, each with its stream, and masks for them;
+    the library's kernels and scratch array have been used before."""
+    p = synth.make_panel(spec=dict(n_var=300, n_samples=700, n_case=310, maf=("uniform", 0.01, 0.5),
+                                   miss=0.02, planted=0, seed=78))
+    m0, m1 = synth.masks_from_pheno(p["pheno"])
+    made = [ge.Panel.from_bed(p["payload"], p["n_var"], p["n_samples"]) for _ in range(count + 1)]
+    for k, ffun in ((50, 0), (6000, 0), (3000, 1)):
+        made[0].scan_noalloc(m0, m1, topmost=k, ffun=ffun)
+    made.pop(0).close()
+    return made, m0, m1
+
+
+def test_noalloc_first_calls_leave_device_memory():
+    """Kernels that need private memory have the runtime allocate it for a
+    queue's first one: more panels than there are hardware queues, short and
+    sorted rankings, both objectives."""
+    print("case noalloc first calls", flush=True)
+    panels, m0, m1 = fresh_panels(8)
+    for h in panels:
+        for k, ffun in ((50, 0), (6000, 0), (3000, 1)):
+            before = free_bytes()
+            h.scan_noalloc(m0, m1, topmost=k, ffun=ffun)
+            assert free_bytes() == before, (k, ffun)
+    for h in panels:
+        h.close()
