@@ -75,7 +75,8 @@ struct gepi_panel {
     uint64_t *d_small = nullptr;
     DeviceTables tabs;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
-    std::vector<hipEvent_t> band_ev; /* two per band of a planned scan */
+    std::vector<hipEvent_t> band_ev; /* two per band of a planned scan: some from
+                                      * the start, more as bands need them      */
     /* pinned, mapped: the band reports and small result lists the device
      * writes (HostMail) */
     void *mail = nullptr;

@@ -33,7 +33,9 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
+#include <cstddef>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -144,13 +146,28 @@ static __device__ __align__(256) unsigned char scratch[SCRATCH_BYTES];
 namespace {
 
 /* What a planned scan's kernels write for the host (pinned memory): a
- * report per enqueued band, and the final records when they are few. */
+ * report per enqueued band, and the final records when they are few.  The
+ * allocation-free scan has neither this nor more events than a panel is
+ * created with: its reports lie in front of its records in the scratch, so
+ * that one copy brings both (two took 20 us more).                         */
 constexpr int PLAN_BANDS = 48;        /* bands enqueued between two waits       */
+constexpr int PLAN_BANDS_NOALLOC = 4;
 constexpr int64_t MAIL_RECORDS = 2048;
+constexpr size_t REPORT_PENDS = PLAN_BANDS_NOALLOC * sizeof(ItemReport) / sizeof(Pend);
 struct HostMail {
     ItemReport report[PLAN_BANDS];
     Cand rec[MAIL_RECORDS];
 };
+
+/* The two events of each of n bands. */
+int band_events(gepi_panel *p, int n) {
+    while (p->band_ev.size() < 2 * (size_t)n) {
+        hipEvent_t e;
+        HIP_TRY(hipEventCreate(&e));
+        p->band_ev.push_back(e);
+    }
+    return GEPI_OK;
+}
 
 int panel_alloc(gepi_panel *p, int device, int64_t n_var, int32_t n_samples) {
     p->device = device;
@@ -165,7 +182,7 @@ int panel_alloc(gepi_panel *p, int device, int64_t n_var, int32_t n_samples) {
     HIP_TRY(hipMalloc(&p->d_small, sizeof(uint64_t) * 2 * SEL_SMALL));
     HIP_TRY(hipEventCreate(&p->ev0));
     HIP_TRY(hipEventCreate(&p->ev1));
-    return GEPI_OK;
+    return band_events(p, PLAN_BANDS_NOALLOC);
 }
 
 void panel_free(gepi_panel *p) {
@@ -608,6 +625,7 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
         if ((rc = bind_scratch(p, b, n0 + n1 + 1, cw.size() * sizeof(CompressWord), clsk_bytes,
                                cap, pcap)) != GEPI_OK)
             return rc;
+        pcap -= REPORT_PENDS; /* the places of the reports: the end of the list */
     } else {
         /* device bytes allocated by this call: buffers that grow */
         int64_t &alloc = st_local.bytes_allocated;
@@ -844,13 +862,18 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
     std::vector<Cand> host;
     bool finished = false, prepare_read = false;
     if (planned) {
-        if (!p->mail) HIP_TRY(hipHostMalloc(&p->mail, sizeof(HostMail), hipHostMallocDefault));
-        HostMail *mail = static_cast<HostMail *>(p->mail);
-        while (p->band_ev.size() < 2 * PLAN_BANDS) {
-            hipEvent_t e;
-            HIP_TRY(hipEventCreate(&e));
-            p->band_ev.push_back(e);
-        }
+        if (!noalloc && !p->mail)
+            HIP_TRY(hipHostMalloc(&p->mail, sizeof(HostMail), hipHostMallocDefault));
+        HostMail *mail = noalloc ? nullptr : static_cast<HostMail *>(p->mail);
+        struct Copied {
+            ItemReport report[PLAN_BANDS_NOALLOC];
+            Cand rec[SORT_HOST_MAX];
+        };
+        static_assert(offsetof(Copied, rec) == REPORT_PENDS * sizeof(Pend), "as in the scratch");
+        std::unique_ptr<Copied> copied(noalloc ? new Copied : nullptr);
+        ItemReport *dev_report = noalloc ? reinterpret_cast<ItemReport *>(b.cand[0]) - PLAN_BANDS_NOALLOC : mail->report;
+        const ItemReport *report = noalloc ? copied->report : mail->report;
+        const size_t most_bands = noalloc ? PLAN_BANDS_NOALLOC : PLAN_BANDS;
         double q = plan.share(first);
         HIP_TRY(init_state(plan.score(q, n0 + n1)));
         ea.cand = b.cand[0];
@@ -873,7 +896,8 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
         int64_t upto = first; /* tiles given to jobs so far */
         bool looser = false;
         while (!jobs.empty()) {
-            const int nj = (int)std::min<size_t>(jobs.size(), PLAN_BANDS);
+            const int nj = (int)std::min<size_t>(jobs.size(), most_bands);
+            if ((rc = band_events(p, nj)) != GEPI_OK) return rc;
             for (int j = 0; j < nj; j++) {
                 ca.pcap = ea.pcap = jobs[j].room;
                 ca.watch = jobs[j].t0 < first ? 1 : 0;
@@ -881,21 +905,26 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
                 launch_count(jobs[j].t0, jobs[j].t1, p->band_ev[2 * j], p->band_ev[2 * j + 1]);
                 launch_exact();
                 k_topk_one<<<1, TOPK_THREADS, 0, p->stream>>>(topk_desc(
-                    b, 0, cap_plan, k, par, jobs[j].t0, jobs[j].t1, n_a4, &mail->report[j], true));
+                    b, 0, cap_plan, k, par, jobs[j].t0, jobs[j].t1, n_a4, dev_report + j, true));
             }
             HIP_TRY(hipGetLastError());
             /* the records, in case these bands are the last */
             const bool last_jobs = upto == n_tiles && nj == (int)jobs.size();
-            const bool by_mail = k <= MAIL_RECORDS;
+            const bool by_mail = k <= MAIL_RECORDS && !noalloc;
             if (last_jobs && by_mail)
                 HIP_TRY(hipMemcpyAsync(mail->rec, b.cand[0], sizeof(Cand) * k, hipMemcpyDeviceToHost,
                                        p->stream));
+            if (noalloc)
+                HIP_TRY(hipMemcpyAsync(copied.get(), dev_report,
+                                       offsetof(Copied, rec) +
+                                           (last_jobs && k <= SORT_HOST_MAX ? sizeof(Cand) * (size_t)k : 0),
+                                       hipMemcpyDeviceToHost, p->stream));
             HIP_TRY(hipStreamSynchronize(p->stream));
             if (!prepare_read) read_prepare();
             prepare_read = true;
             redo.clear();
             for (int j = 0; j < nj; j++) {
-                const ItemReport &r = mail->report[j];
+                const ItemReport &r = report[j];
                 float ms = 0;
                 hipEventElapsedTime(&ms, p->band_ev[2 * j], p->band_ev[2 * j + 1]);
                 ms_count += ms;
@@ -933,7 +962,7 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
                 /* after the pilot: how many survivors it had, and the
                  * other bands                                            */
                 plan.learn(last.t1 - last.t0, last.t0 > 0 ? plan.share_after(last.t0) : q,
-                           mail->report[nj - 1].pend_count);
+                           report[nj - 1].pend_count);
                 while (upto < n_tiles) {
                     const int64_t n = plan.next(upto, n_tiles - upto);
                     jobs.push_back(Job{upto, upto + n, plan.room((double)n * plan.survivors(1, plan.share_after(upto)), pcap)});
@@ -942,8 +971,8 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
             }
             if (jobs.empty() && count == (unsigned long long)k) {
                 if (k <= SORT_HOST_MAX) host.resize((size_t)k);
-                if (by_mail)
-                    memcpy(host.data(), mail->rec, sizeof(Cand) * (size_t)k);
+                if (by_mail || (noalloc && k <= SORT_HOST_MAX))
+                    memcpy(host.data(), noalloc ? copied->rec : mail->rec, sizeof(Cand) * (size_t)k);
                 else if (k <= SORT_HOST_MAX)
                     HIP_TRY(hipMemcpyAsync(host.data(), b.cand[0], sizeof(Cand) * k,
                                            hipMemcpyDeviceToHost, p->stream));

@@ -125,3 +125,23 @@ def test_noalloc_first_calls_leave_device_memory():
             assert free_bytes() == before, (k, ffun)
     for h in panels:
         h.close()
+
+
+def test_noalloc_first_calls_map_nothing():
+    """Device and pinned host memory that the runtime hands out is mapped from
+    the render node: a panel's first scans map none."""
+    print("case noalloc mappings", flush=True)
+
+    def mapped():
+        with open("/proc/self/maps") as f:
+            return {line.split()[0] for line in f if "/dev/dri/" in line}
+
+    panels, m0, m1 = fresh_panels(3)
+    for h in panels:
+        for k, ffun in ((50, 0), (6000, 0), (3000, 1)):
+            before = mapped()
+            _, st = h.scan_noalloc(m0, m1, topmost=k, ffun=ffun)
+            assert mapped() <= before, (k, ffun)
+            assert st["bytes_allocated"] == 0
+    for h in panels:
+        h.close()
