@@ -621,7 +621,12 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
         return GEPI_OK;
     };
     if (noalloc) {
-        cap = pcap = cap_min;
+        cap = cap_min;
+        /* the super-steps' places take theirs from the pending list's slack,
+         * so that they refuse no scan                                       */
+        pcap = cap_min - (align256(cw.size() * sizeof(CompressWord)) - align256(cw_words * sizeof(CompressWord))) / sizeof(Pend);
+        static_assert(align256((GEPI_MAX_SAMPLES / 384 + 2) * sizeof(SuperSrc)) + 256 + REPORT_PENDS * sizeof(Pend) <=
+                          1024 * sizeof(Pend), "the slack of cap_min holds them");
         if ((rc = bind_scratch(p, b, n0 + n1 + 1, cw.size() * sizeof(CompressWord), clsk_bytes,
                                cap, pcap)) != GEPI_OK)
             return rc;

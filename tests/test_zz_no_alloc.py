@@ -145,3 +145,38 @@ def test_noalloc_first_calls_map_nothing():
             assert st["bytes_allocated"] == 0
     for h in panels:
         h.close()
+
+
+def test_noalloc_longest_ranking():
+    """The scratch array holds as long a ranking of a panel on genotype planes as
+    of one on allele planes (a valid call without an allele): the places of its
+    super-steps take none of it.  The longest that the second one's message
+    leaves room for, and one more."""
+    print("case noalloc longest ranking", flush=True)
+    n_var, n = 400, 40000
+    rng = np.random.default_rng(79)
+    codes = rng.choice(np.array([0, 2, 3], np.uint8), size=(n_var, n))
+    bits, valid = orc.planes_from_codes(codes)
+    m0, m1 = orc.masks_from_classes(np.arange(n) % 2)
+    bare = bits.copy()
+    bare[0:2, 0] = 0
+    with ge.Panel.from_planes(bare, valid, n) as h:
+        with pytest.raises(ge.GepiError) as e:
+            h.scan_noalloc(m0, m1, topmost=1500000, count_path=3)
+    words = str(e.value).split()
+    need, have = int(words[words.index("needs") + 1]), int(words[words.index("its") + 1])
+    records = int(words[words.index("lists") + 1])
+
+    def lists(cap):
+        return -(-16 * cap // 256) * 256 + 2 * (-(-32 * cap // 256) * 256)
+
+    cap = records
+    while need - lists(records) + lists(cap) > have:
+        cap -= 1
+    k = 1500000 - (records - cap)
+    with ge.Panel.from_planes(bits, valid, n) as h:
+        got, _ = h.scan_noalloc(m0, m1, topmost=k, count_path=3)
+        assert len(got) == k
+        assert_same(got, h.scan(m0, m1, topmost=k, count_path=3)[0], "longest")
+        with pytest.raises(ge.GepiError):
+            h.scan_noalloc(m0, m1, topmost=k + 16, count_path=3)
