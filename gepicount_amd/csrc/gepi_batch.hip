@@ -176,7 +176,7 @@ void Engine::release() {
     free_.clear();
     for (auto &b : live_) hipFree(b.first);
     live_.clear();
-    in_use_ = 0;
+    in_use_ = in_lists_ = 0;
     for (int i = 0; i < NGROUP; i++) {
         hipFree(d_bdesc_[i]);
         hipFree(d_map_[i]);
@@ -235,6 +235,13 @@ void Engine::dfree(void *p) {
     in_use_ -= it->second;
     free_.insert({it->second, p});
     live_.erase(it);
+}
+
+void Engine::free_list(ScanItem *it) {
+    if (it->d_pairs) in_lists_ -= live_[it->d_pairs];
+    dfree(it->d_pairs);
+    it->d_pairs = nullptr;
+    it->pair_cap = 0;
 }
 
 const gepi_tune_class *Engine::tune_of(int32_t n_k4) const {
@@ -471,24 +478,21 @@ size_t Engine::estimate_footprint(const gepi_panel *p, int64_t topmost) {
     const unsigned long long pcap = std::max<unsigned long long>(cap, 1ull << 20);
     return round_block((size_t)n_u * n_var_pad * 3 * 64 + (size_t)n_var_pad * 6 * sizeof(float)) + round_block(cap * sizeof(Cand)) +
            round_block(pcap * sizeof(Pend)) + round_block((size_t)4 * p->w64 * sizeof(CompressWord)) +
-           round_block(sizeof(ScanState)) +
-           round_block((size_t)pair_list_cap(n_var_pad / TM * (n_var_pad / TM + 1), 0, PAIRS_MOST_BATCH) * PAIR_BYTES);
+           round_block(sizeof(ScanState));
 }
 
 void Engine::drop(ScanItem *it, int status) {
     dfree(it->d_layout);
     dfree(it->d_cw);
     dfree(it->d_pend);
-    dfree(it->d_pairs);
+    free_list(it);
     dfree(it->d_cand);
     dfree(it->d_state);
     it->d_layout = nullptr;
     it->d_cw = nullptr;
     it->d_pend = nullptr;
-    it->d_pairs = nullptr;
     it->d_cand = nullptr;
     it->d_state = nullptr;
-    it->footprint = 0;
     it->status = status;
     it->done = true;
     it->stats.ms_scan = ms_since(it->t_added);
@@ -590,17 +594,21 @@ int Engine::add(ScanItem *it) {
     it->d_pend = (Pend *)dalloc(it->pcap * sizeof(Pend));
     it->d_cand = (Cand *)dalloc(it->cap * sizeof(Cand));
     it->d_state = (ScanState *)dalloc(sizeof(ScanState));
-    it->pair_cap = it->geno ? pair_list_cap(it->n_tiles, it->n_k4, PAIRS_MOST_BATCH) : 0u;
-    if (it->pair_cap) it->d_pairs = (uint4 *)dalloc((size_t)it->pair_cap * PAIR_BYTES);
-    if (!it->d_layout || !it->d_cw || !it->d_pend || (it->pair_cap && !it->d_pairs) || !it->d_cand || !it->d_state) {
+    if (!it->d_layout || !it->d_cw || !it->d_pend || !it->d_cand || !it->d_state) {
         drop(it, gepi_fail(GEPI_ERR_NOMEM, "device memory for a scan of %lld variants",
                            (long long)it->n_var));
         return it->status;
     }
-    it->footprint = round_block(lay) + round_block(it->h_cw.size() * sizeof(CompressWord)) +
-                    round_block(it->pcap * sizeof(Pend)) + round_block(it->cap * sizeof(Cand)) +
-                    round_block(sizeof(ScanState)) +
-                    (it->pair_cap ? round_block((size_t)it->pair_cap * PAIR_BYTES) : 0);
+    /* the list of pairs put off, where it fits: the count kernel tests its
+     * pairs itself without one                                             */
+    it->pair_cap = it->geno ? pair_list_cap(it->n_tiles, it->n_k4, PAIRS_MOST_BATCH) : 0u;
+    const size_t list = round_block((size_t)it->pair_cap * PAIR_BYTES);
+    if (it->pair_cap && (list > budget || in_use_ > budget - list ||
+                         !(it->d_pairs = (uint4 *)dalloc(list)))) {
+        (void)hipGetLastError();
+        it->pair_cap = 0;
+    }
+    if (it->d_pairs) in_lists_ += live_[it->d_pairs];
     HIP_TRY(hipMemcpyAsync(it->d_cw, it->h_cw.data(), it->h_cw.size() * sizeof(CompressWord),
                            hipMemcpyHostToDevice, stream));
     CountArgs ca;
@@ -692,6 +700,9 @@ int Engine::round(std::vector<ScanItem *> &finished) {
     const size_t na = active_.size();
     int rc;
     if ((rc = grow_desc(na)) != GEPI_OK) return rc;
+    /* lists of pairs hold nothing between rounds */
+    for (ScanItem *it : active_)
+        if (in_use_ > budget && it->d_pairs) free_list(it);
     /* bands, scaled down uniformly when the round's workgroup budget is set */
     int64_t total_wg = 0;
     for (ScanItem *it : active_) {

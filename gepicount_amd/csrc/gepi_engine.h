@@ -72,7 +72,6 @@ struct ScanItem {
     uint32_t pair_cap = 0;
     gepi::Cand *d_cand = nullptr;
     gepi::ScanState *d_state = nullptr;
-    size_t footprint = 0; /* device bytes held */
     std::vector<gepi::CompressWord> h_cw;
 };
 
@@ -90,7 +89,10 @@ class Engine {
     size_t active_count() const { return active_.size(); }
     /* Device bytes a scan of this panel would hold (admission control). */
     static size_t estimate_footprint(const gepi_panel *p, int64_t topmost);
-    size_t bytes_in_use() const { return in_use_; }
+    /* What the active scans hold and cannot do without (their lists of pairs
+     * put off are optional, and are given back when they pass the budget). */
+    size_t bytes_needed() const { return in_use_ - in_lists_; }
+    size_t budget = SIZE_MAX; /* device bytes of the active scans */
     /* Workgroups per count round (0 = unlimited): bounds round latency. */
     int64_t round_wg_budget = 0;
     double ms_count = 0.0;
@@ -110,6 +112,7 @@ class Engine {
   private:
     void *dalloc(size_t bytes);
     void dfree(void *p);
+    void free_list(ScanItem *it);
     int finish(ScanItem *it);
     /* Starts a scan (again): its state admits what scores at most thr. */
     int start(ScanItem *it, double thr, int64_t band);
@@ -137,7 +140,7 @@ class Engine {
     std::vector<ScanItem *> active_;
     std::multimap<size_t, void *> free_;
     std::map<void *, size_t> live_;
-    size_t in_use_ = 0;
+    size_t in_use_ = 0, in_lists_ = 0;
     /* count launch groups: objective (g & 1) x job shape (g >> 1; 3: wave
      * tiles on genotype planes) */
     static constexpr int NGROUP = 10, NGRAPH_COUNT = 16;

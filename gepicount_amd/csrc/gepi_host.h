@@ -175,8 +175,8 @@ inline void screen_consts(int32_t n0, int32_t n1, gepi::CountArgs &g) {
 
 /* Records of the list of pairs that the count kernel puts off (48 bytes): one
  * for every 4 pairs of the scan (at 16 small scans with loose thresholds took
- * 1.12x the time: 1,020 x 89, 2,000 x 1,000), at most `most`, beyond which the kernel tests
- * its pairs itself.  None from PAIRS_MAX_KSTEPS K steps on, where the other
+ * 1.12x the time: 1,020 x 89, 2,000 x 1,000), at most `most`, beyond which the
+ * kernel tests its pairs itself, as it does where no list fits.  None from PAIRS_MAX_KSTEPS K steps on, where the other
  * workgroup of the CU fills the time of a test with its longer K loop: whole
  * scans of 20,000 variants, top-1,000, against tests in the kernel, took 0.90x
  * the time with 256 samples (Fisher 0.88x), 0.90x (0.89x) with 1,024, 0.92x
@@ -188,6 +188,8 @@ constexpr int32_t PAIRS_MAX_KSTEPS = 48;
 constexpr size_t PAIR_BYTES = 48;
 inline uint32_t pair_list_cap(int64_t n_tiles, int32_t ks, int64_t most) {
     if (ks > PAIRS_MAX_KSTEPS) return 0;
+    /* test hook: at most so many records (0: as where the list does not fit) */
+    if (const char *env = getenv("GEPI_PAIR_CAP")) most = std::min<int64_t>(most, std::max(atoll(env), 0ll));
     return (uint32_t)std::min<int64_t>(std::max<int64_t>(n_tiles * (64 * 32 / 4), 4096), most);
 }
 

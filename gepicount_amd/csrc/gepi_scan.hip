@@ -598,8 +598,10 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
      * records that the second launch costs what it spares: top-1,000,000 of
      * 20,000 x 2,048 7.4 ms of count launches with the tests in them, 5.7 and
      * 2.0 with k_pairs                                                      */
-    const uint32_t pair_cap = geno && !noalloc && short_ranking ? pair_list_cap(n_tiles, n_ks, PAIRS_MOST) : 0u;
+    uint32_t pair_cap = geno && !noalloc && short_ranking ? pair_list_cap(n_tiles, n_ks, PAIRS_MOST) : 0u;
     ScanBufs b;
+    CountArgs ca;
+    memset(&ca, 0, sizeof ca);
     /* the candidate and pending lists of cap and pcap records, the pairs put
      * off after the latter: one allocation, as a drop-in call pays for each
      * (two: 1,020 x 89 0.47 -> 0.52 ms)                                     */
@@ -612,10 +614,18 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
             HIP_TRY(hipMalloc(&p->d_cand[0], sizeof(Cand) * cap));
             p->buf_cap = cap;
         }
-        const size_t lists = sizeof(Pend) * pcap + (size_t)pair_cap * PAIR_BYTES;
-        if (lists > p->pend_bytes || !p->d_pend) st_local.bytes_allocated += (int64_t)lists;
-        int e;
-        if ((e = grow(&p->d_pend, &p->pend_bytes, lists)) != GEPI_OK) return e;
+        size_t lists = sizeof(Pend) * pcap + (size_t)pair_cap * PAIR_BYTES;
+        const bool grows = lists > p->pend_bytes || !p->d_pend;
+        int e = grow(&p->d_pend, &p->pend_bytes, lists);
+        if (e != GEPI_OK && pair_cap) {
+            /* a scan that fits without the pairs put off runs without them */
+            (void)hipGetLastError();
+            pair_cap = ca.pair_cap = 0;
+            lists = sizeof(Pend) * pcap;
+            e = grow(&p->d_pend, &p->pend_bytes, lists);
+        }
+        if (e != GEPI_OK) return e;
+        if (grows) st_local.bytes_allocated += (int64_t)lists;
         b.cand[0] = p->d_cand[0];
         b.pend = p->d_pend;
         return GEPI_OK;
@@ -676,8 +686,6 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
     else
         HIP_TRY(hipMemcpyAsync(b.perm, perm.data(), perm.size() * 4, hipMemcpyHostToDevice,
                                p->stream));
-    CountArgs ca;
-    memset(&ca, 0, sizeof ca);
     screen_consts(n0, n1, ca);
     HIP_TRY(hipEventRecord(p->ev0, p->stream));
     if (fp4) {

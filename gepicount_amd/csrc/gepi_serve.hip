@@ -141,7 +141,7 @@ struct gepi_server {
                 std::unique_lock<std::mutex> lk(mu);
                 cv_work.wait(lk, [&] { return stop || !queue.empty() || !eng.idle(); });
                 if (stop && queue.empty() && eng.idle()) return;
-                size_t planned = eng.bytes_in_use();
+                size_t planned = eng.bytes_needed();
                 while (!queue.empty()) {
                     Request *r = queue.front();
                     const size_t fp = Engine::estimate_footprint(r->item.panel, r->item.topmost);
@@ -213,6 +213,7 @@ extern "C" int gepi_server_create(const gepi_server_params *par, gepi_server **o
         HIP_TRY(hipMemGetInfo(&fr, &tot));
         s->budget = (int64_t)(fr / 4 * 3);
     }
+    s->eng.budget = (size_t)s->budget;
     s->worker = std::thread([srv = s.get()] { srv->run(); });
     *out = s.release();
     return GEPI_OK;

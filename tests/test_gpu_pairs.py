@@ -47,3 +47,50 @@ def test_batch():
         assert status == 0
         assert_same(got, orc.gold_scan(orc.Panel(bits, valid, m0, m1, n), k, ffun=ffun), "batch")
     eng.close()
+
+
+@pytest.mark.parametrize("cap", ["0", "100"])
+def test_list_left_out(monkeypatch, cap):
+    """No list, as where it does not fit, and a short one: single scans, the engine
+    and a server whose budget leaves no room for it."""
+    print("case pairs left out", cap, flush=True)
+    monkeypatch.setenv("GEPI_PAIR_CAP", cap)
+    made = [panel(120 + i, 970 + i, 40, 35, 2, 0.02) for i in range(2)]
+    refs = [orc.gold_scan(orc.Panel(b, v, m0, m1, n), 200, ffun=i) for i, (b, v, m0, m1, n) in enumerate(made)]
+    ps = [ge.Panel.from_planes(b, v, n) for b, v, _, _, n in made]
+    for i, (p, (_, _, m0, m1, _)) in enumerate(zip(ps, made)):
+        got, _ = p.scan(m0, m1, topmost=200, ffun=i, count_path=3)
+        assert_same(got, refs[i], "alone")
+    with ge.Engine() as eng:
+        res, _ = eng.scan_batch([dict(panel=p, mask_ctrl=m0, mask_case=m1, topmost=200, ffun=i)
+                                 for i, (p, (_, _, m0, m1, _)) in enumerate(zip(ps, made))])
+    for r, ref in zip(res, refs):
+        assert_same(r[0], ref, "batch")
+    for p in ps:
+        p.close()
+
+
+def test_list_does_not_count_against_the_budget():
+    """Requests are admitted by what they cannot do without: while a large scan
+    runs, ten of about 31 MB each join it under a budget that holds them (and
+    two of them with their lists of pairs, 101 MB each)."""
+    print("case pairs budget", flush=True)
+    rng = np.random.default_rng(7)
+
+    def bed(n_var, n):
+        m0, m1 = orc.masks_from_classes(rng.integers(0, 2, n))
+        return rng.integers(0, 256, size=(n_var, (n + 3) // 4), dtype=np.uint8), n_var, n, m0, m1
+
+    large, small = bed(50000, 4000), [bed(20000, 256) for _ in range(10)]
+    with ge.Server(hbm_budget=560 << 20) as srv:
+        ids = [srv.add_panel_bed(*x[:3]) for x in [large] + small]
+        asks = [(i, x[3], x[4]) for i, x in zip(ids, [large] + small)]
+        tickets = [srv.submit(i, m0, m1, topmost=100) for i, m0, m1 in asks]
+        res = [srv.wait(t) for t in tickets]
+        st = srv.stats()
+    assert st["failed"] == 0
+    assert st["max_active"] >= 8, st
+    for (got, _, status), x in zip(res[1:4], small):
+        assert status == 0
+        with ge.Panel.from_bed(*x[:3]) as p:
+            assert_same(got, p.scan(x[3], x[4], topmost=100)[0], "served")
