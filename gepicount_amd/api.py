@@ -419,7 +419,9 @@ class Engine:
         table: one dict per size class (max_ksteps, wg_per_cu, tile,
         band_evals, ms_best, ms_default), ascending max_ksteps; tile 0 is the
         64 x 32-variant count job, 1 the 32 x 32 half tile, 2 wave tiles (two
-        64 x 32 tiles as four 32 x 32 wave tiles, the kernel of count path 3).
+        64 x 32 tiles as four 32 x 32 wave tiles, the kernel of count path 3);
+        reserved 1 where the class keeps the default shape, which each scan's
+        size decides (tile is the one of the trial's scans).
         tile schedules entropy scans; Fisher scans run wave tiles in every
         class (not in captured-graph rounds)."""
         out = (TuneClass * 16)()
@@ -435,6 +437,7 @@ class Engine:
             arr[i].max_ksteps = int(c["max_ksteps"])
             arr[i].wg_per_cu = int(c["wg_per_cu"])
             arr[i].tile = int(c.get("tile", 0))
+            arr[i].reserved = int(c.get("reserved", 0))
             arr[i].band_evals = float(c["band_evals"])
             arr[i].ms_best = float(c.get("ms_best", 0.0))
             arr[i].ms_default = float(c.get("ms_default", 0.0))

@@ -396,6 +396,7 @@ int Engine::autotune(int32_t repeats) {
             best.band_evals = 2e9;
             ms_best = ms_dflt;
         }
+        best.reserved = best.tile == dtile ? 1 : 0;
         best.ms_best = ms_best;
         best.ms_default = ms_dflt;
         table.push_back(best);
@@ -426,6 +427,7 @@ int Engine::autotune(int32_t repeats) {
             for (size_t c = 0; c < table.size(); c++) {
                 table[c].wg_per_cu = 2;
                 table[c].tile = dflt_tile((int)c);
+                table[c].reserved = 1;
                 table[c].band_evals = 2e9;
                 table[c].ms_best = table[c].ms_default;
             }
@@ -526,12 +528,14 @@ int Engine::add(ScanItem *it) {
     it->stats.evals = total;
     /* the job shape decides the class layout (wave tiles read the grouped
      * one): Fisher scans run wave tiles, which park flagged pairs; entropy
-     * scans their class's tile (no table: batch_shape_default); captured
-     * rounds have no wave-tile launch                                      */
+     * scans their class's tile (no table, or a class that keeps the default,
+     * which its trial's large panels on genotype planes stand for:
+     * batch_shape_default by the scan); captured rounds have no wave-tile
+     * launch                                                               */
     const int32_t ks = (it->n0 + 127) / 128 + (it->n1 + 127) / 128;
     const gepi_tune_class *tc = tune_of(ks);
     const int64_t a4 = (p->n_var + TM - 1) / TM;
-    it->shape = tc ? tc->tile : batch_shape_default(ks, a4 * (a4 + 1), p->three_genotypes);
+    it->shape = tc && tc->reserved != 1 ? tc->tile : batch_shape_default(ks, a4 * (a4 + 1), p->three_genotypes);
     if (it->ffun != GEPI_FFUNC_ENTROPY && !use_graph_) it->shape = 2;
     if (it->shape == 2 && use_graph_) it->shape = 0;
     it->geno = it->shape == 2 && p->three_genotypes;

@@ -249,7 +249,9 @@ typedef struct gepi_tune_class {
                             class (they park flagged pairs); captured rounds
                             (GEPI_ENGINE_GRAPH=1) have no wave-tile launch and
                             run whole tiles in its place.                    */
-    int32_t reserved;
+    int32_t reserved;    /* 1 (set by the autotuner): the class keeps the
+                            default job shape, which each scan's size decides;
+                            tile names the one of the trial's scans          */
     double band_evals;   /* evaluations per scan and round                    */
     double ms_best;      /* autotune trial of the class: chosen schedule      */
     double ms_default;   /* the same trial under the default schedule         */
