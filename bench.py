@@ -74,6 +74,15 @@ def copy_calibration(mib):
     print(json.dumps({"copy_calibration_mib": mib, "bytes_each_way": mib << 20}))
 
 
+def count_kernel(path, complete):
+    """The count kernel of a path and the plane products it forms per variant
+    pair: nine, or on wave tiles four for a panel without missing calls (the
+    other cells of a pair's genotype table follow from its margins)."""
+    if path == 3:
+        return ("k_count_f4c", 4) if complete else ("k_count_f4g", 9)
+    return {4: "k_count_f4", 2: "k_count_mfma"}.get(path, "k_count_popc"), 9
+
+
 def class_words(n):
     return ((n + 127) // 128) * 4
 
@@ -441,24 +450,24 @@ def main():
     total = time.perf_counter() - t0
     ms_per_step = 1000.0 * total / args.steps
 
-    # count kernel roofline.  All paths form 9 plane products per variant pair
-    # over the n class samples.  Popcount: 2 VALU ops (and, bcnt) per 32-bit
-    # word of each product.  MFMA: 9 x n MACs = 18 n ops per variant pair
-    # (int8 operands, or fp4 operands with fp32 accumulation).
+    # count kernel roofline: the plane products of a variant pair over the n
+    # class samples.  Popcount: 2 VALU ops (and, bcnt) per 32-bit word of each
+    # product.  MFMA: n MACs = 2 n ops per product (int8 operands, or fp4
+    # operands with fp32 accumulation).
     var_pairs = n_var * (n_var + 1) // 2
     path = stats[-1]["count_path"]
     k_ms = statistics.mean(s["ms_count_kernels"] for s in stats)
     launches = statistics.mean(s["bands"] for s in stats)
+    kernel, products = count_kernel(path, not panel.qa()[0].any())
     if path in (3, 4):
-        ops_total = var_pairs * 9 * 2.0 * (n0 + n1)
-        peak, bound, unit, kernel = (FP4_MFMA_PEAK_FLOPS, "mfma", "TFLOP/s",
-                                     "k_count_f4g" if path == 3 else "k_count_f4")
+        ops_total = var_pairs * products * 2.0 * (n0 + n1)
+        peak, bound, unit = FP4_MFMA_PEAK_FLOPS, "mfma", "TFLOP/s"
     elif path == 2:
-        ops_total = var_pairs * 9 * 2.0 * (n0 + n1)
-        peak, bound, unit, kernel = INT8_MFMA_PEAK_OPS, "mfma", "TOP/s", "k_count_mfma"
+        ops_total = var_pairs * products * 2.0 * (n0 + n1)
+        peak, bound, unit = INT8_MFMA_PEAK_OPS, "mfma", "TOP/s"
     else:
-        ops_total = var_pairs * 9 * 2 * ((n0 + n1) / 32.0)
-        peak, bound, unit, kernel = VALU_PEAK_OPS, "valu", "Tops/s", "k_count_popc"
+        ops_total = var_pairs * products * 2 * ((n0 + n1) / 32.0)
+        peak, bound, unit = VALU_PEAK_OPS, "valu", "Tops/s"
     achieved = ops_total / (k_ms / 1000.0)
     roof = {"bound": bound, "kernel": kernel, "achieved": achieved / 1e12, "peak": peak / 1e12,
             "unit": unit, "frac": achieved / peak, "traffic": None,
