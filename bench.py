@@ -31,6 +31,8 @@ VALU_PEAK_OPS = 256 * 64 * 2.4e9
 INT8_MFMA_PEAK_OPS = 5.0e15
 # MI355X dense fp4 (e2m1) matrix peak
 FP4_MFMA_PEAK_FLOPS = 10.1e15
+# compute type by count path (popcount: u32)
+DTYPES = {3: "fp4 (e2m1, fp32 accumulate)", 4: "fp4 (e2m1, fp32 accumulate)", 2: "i8"}
 
 
 def parse():
@@ -490,7 +492,7 @@ def main():
         "metric": METRIC, "value": evals / statistics.mean(times), "unit": "evals/s",
         "n_gpus": 1, "steps": args.steps, "warmup": args.warmup, "ms_per_step": ms_per_step,
         "higher_is_better": True, "scaling": "weak", "vs_baseline": None,
-        "dtype": {3: "fp4 (e2m1, fp32 accumulate)", 2: "i8"}.get(path, "u32"),
+        "dtype": DTYPES.get(path, "u32"),
         "data": "synthetic",
         "config": {"workload": "%s: %d variants x %d samples (%d cases / %d controls), top-%d, %s"
                                % (args.workload, n_var, n, n1, n0, args.topk,
