@@ -535,10 +535,13 @@ int Engine::add(ScanItem *it) {
     const int32_t ks = (it->n0 + 127) / 128 + (it->n1 + 127) / 128;
     const gepi_tune_class *tc = tune_of(ks);
     const int64_t a4 = (p->n_var + TM - 1) / TM;
-    it->shape = tc && tc->reserved != 1 ? tc->tile : batch_shape_default(ks, a4 * (a4 + 1), p->three_genotypes);
+    /* classes too uneven for the screen keep the allele planes */
+    const bool screens = p->three_genotypes &&
+                         screen_pays(it->n0, it->n1, it->ffun != GEPI_FFUNC_ENTROPY, p->complete);
+    it->shape = tc && tc->reserved != 1 ? tc->tile : batch_shape_default(ks, a4 * (a4 + 1), screens);
     if (it->ffun != GEPI_FFUNC_ENTROPY && !use_graph_) it->shape = 2;
     if (it->shape == 2 && use_graph_) it->shape = 0;
-    it->geno = it->shape == 2 && p->three_genotypes;
+    it->geno = it->shape == 2 && screens;
     it->full = it->geno && p->complete;
     it->stats.count_path = it->shape == 2 ? 3 : 4;
     it->stats.n_class0 = it->n0;

@@ -173,6 +173,26 @@ inline void screen_consts(int32_t n0, int32_t n1, gepi::CountArgs &g) {
     g.sc_sub = (float)(18.0 * start * (1.0 + 2.0 * k) + 1e-3);
 }
 
+/* Whether the screen of the genotype table is near enough to spare the tests
+ * that come after it: its k grows as 1/s with the smaller class's share s, and
+ * k|u| with the spread of a cell's u, sqrt(s (1-s) / n).  Whole scans of 20,000
+ * variants, top-100 and top-1,000, against the LDS-staged kernel's time (with
+ * missing calls; without): entropy with 2,048 samples 0.79-0.82 at s = 0.1 (0.59-
+ * 0.63), 0.94-1.04 at 0.05 (0.70-0.79), 1.35 at 0.03 (1.01-1.26), 2.3 at 0.015;
+ * with 512 samples 1.01-1.05 at 0.2 (0.79-0.85), 1.13-1.17 at 0.1 (0.89-0.92),
+ * 1.25-1.34 at 0.05; Fisher with 2,048 samples 0.86-1.07 at 0.2 (0.65-0.83),
+ * 1.04-1.30 at 0.1 (0.83-1.03), 1.42-1.83 at 0.05, with 512 samples 1.10-1.40 at
+ * 0.2 (0.97-1.17), 1.5-1.8 at 0.1.  Where it does not pay, the wave tiles run on
+ * allele planes from F4W_MIN_KSTEPS K steps on (0.81-0.87 of the LDS-staged
+ * kernel's time there with 2,048 samples).                                 */
+inline bool screen_pays(int32_t n0, int32_t n1, bool fisher, bool complete) {
+    const double n = (double)n0 + n1, s = n > 0 ? std::min(n0, n1) / n : 0.0;
+    if (s <= 0.0) return true; /* nothing is associated: every pair passes any filter */
+    const double k = (2.0 * -std::log1p(-s) * (1.0 - s) / s - 1.0) / s, spread = k * k * s * (1.0 - s) / n;
+    if (fisher) return complete ? s >= 0.08 && spread <= 4e-3 : s >= 0.12 && spread <= 2.5e-3;
+    return complete ? s >= 0.045 && spread <= 1.4e-2 : s >= 0.06 && spread <= 7e-3;
+}
+
 /* Records of the list of pairs that the count kernel puts off (48 bytes): one
  * for every 4 pairs of the scan (at 16 small scans with loose thresholds took
  * 1.12x the time: 1,020 x 89, 2,000 x 1,000), at most `most`, beyond which the

@@ -439,7 +439,8 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
      * wave tiles save), and on genotype planes, whose screen spares most of
      * the filter, for any number of samples from F4G_MIN_TILES or
      * F4G_MIN_TILES_FISHER tiles on; Fisher (above F4G_MIN_TILES) only where
-     * the ranking is short enough for the screen (F4G_FISHER_EVALS).  Without genotype planes
+     * the ranking is short enough for the screen (F4G_FISHER_EVALS).  Classes
+     * too uneven for the screen (screen_pays) keep the allele planes.  On those
      * Fisher parks the one pair in 8 that it flags in a global list per
      * workgroup, which the allocation-free scan has no room for, so there
      * the LDS-staged kernel (parking in LDS) runs Fisher.                   */
@@ -447,10 +448,11 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
         const int32_t ks = (n0 + 127) / 128 + (n1 + 127) / 128;
         const bool fisher = par->ffun != GEPI_FFUNC_ENTROPY;
         const int64_t a4 = (n_var + TM - 1) / TM;
-        const bool wide = p->three_genotypes && !noalloc &&
+        const bool screens = p->three_genotypes && screen_pays(n0, n1, fisher, p->complete);
+        const bool wide = screens && !noalloc &&
                           a4 * (a4 + 1) >= (fisher ? F4G_MIN_TILES_FISHER : F4G_MIN_TILES);
         path = wide || (ks >= F4W_MIN_KSTEPS && !(fisher && noalloc)) ? 3 : 4;
-        if (fisher && p->three_genotypes && a4 * (a4 + 1) >= F4G_MIN_TILES &&
+        if (fisher && screens && a4 * (a4 + 1) >= F4G_MIN_TILES &&
             (double)total_evals < (p->complete ? F4G_FISHER_EVALS_COMPLETE : F4G_FISHER_EVALS) * (double)par->topmost)
             path = 4;
     }
@@ -466,8 +468,9 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
      * than 0.02 evaluations per variant pair through); the large scan
      * (65 K steps) 126.0 ms parking and 129.2 ms not.                     */
     const uint32_t park_slots = (uint32_t)(((4 * device_cus(p->device)) + 7) / 8 * 8);
-    /* wave tiles on genotype planes, unless a valid call has no allele */
-    const bool geno = path == 3 && p->three_genotypes;
+    /* wave tiles on genotype planes, unless a valid call has no allele or the
+     * classes are too uneven for the screen                                */
+    const bool geno = path == 3 && p->three_genotypes && screen_pays(n0, n1, par->ffun != GEPI_FFUNC_ENTROPY, p->complete);
     const bool full = geno && p->complete; /* four products a pair, not nine */
     const bool f4w_park =
         path == 3 && !geno && !noalloc &&
