@@ -264,7 +264,8 @@ inline double chi2_quantile(double p) {
 
 struct BandPlan {
     bool entropy;
-    double evals_tile;  /* evaluations per tile                              */
+    double evals_tile;  /* evaluations per tile, on average: less than a whole
+                         * tile's on small panels                             */
     double h;           /* chi-square coefficient per nat (chi2_slope)       */
     double k;
     double most;        /* survivors a band may have                         */

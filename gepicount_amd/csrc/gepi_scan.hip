@@ -572,7 +572,7 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
     chi2_slope(n0, n1, &h0, &h1);
     BandPlan plan;
     plan.entropy = entropy;
-    plan.evals_tile = (double)evals_per_tile;
+    plan.evals_tile = (double)total_evals / (double)n_tiles;
     plan.h = (double)h0 + (double)h1 * std::min(n0, n1);
     plan.k = (double)k;
     plan.c = guess;
@@ -791,7 +791,10 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
     int64_t max_band = std::max<int64_t>(64, (int64_t)(8.0e9 / (double)evals_per_tile));
     if (par->max_grid_area > 0)
         max_band = std::max<int64_t>(1, ((int64_t)par->max_grid_area << 20) / evals_per_tile);
-    int64_t band = std::max<int64_t>(1, std::min<int64_t>(max_band, (2 * k) / evals_per_tile + 1));
+    /* the first one: about a whole tile's evaluations, or twice the ranking's */
+    const int64_t band_first =
+        std::max<int64_t>(1, std::min<int64_t>(max_band, (int64_t)((double)(2 * k + evals_per_tile) / plan.evals_tile)));
+    int64_t band = band_first;
     if (forced_band) band = forced_band;
     double ms_count = 0.0, ms_top = 0.0;
     int64_t t0 = 0;
@@ -1137,7 +1140,7 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
             HIP_TRY(init_state(INFINITY));
             count = exact_total = 0;
             t0 = 0;
-            band = std::max<int64_t>(1, std::min<int64_t>(max_band, (2 * k) / evals_per_tile + 1));
+            band = band_first;
         }
         if (par->intermediate && g_progress_fn) {
             /* the records held so far, sorted, for the caller's report */

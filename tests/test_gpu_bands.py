@@ -73,3 +73,16 @@ def test_planned_guess_fails(ffun):
     got, st = ge.process_gpu_1(bits, valid, m0, m1, 130, topmost=1500, ffun=ffun)
     ref = orc.gold_scan(orc.Panel(bits, valid, m0, m1, 130), 1500, ffun=ffun)
     assert_same(got, ref, "planned-guess")
+
+
+@pytest.mark.parametrize("n_var,n,k", [(1, 40, 3), (2, 50, 10), (20, 300, 1000), (64, 100, 2000)])
+@pytest.mark.parametrize("ffun", [0, 1])
+def test_tiny_panels(n_var, n, k, ffun):
+    """A tile of these holds a fraction of a whole tile's evaluations: no guess
+    for a ranking of much of the panel, and not a band that is lost."""
+    print("case tiny", n_var, n, k, ffun, flush=True)
+    bits, valid, m0, m1 = random_panel(73, n_var, n, 0.01)
+    with ge.Panel.from_planes(bits, valid, n) as panel:
+        got, st = panel.scan(m0, m1, topmost=k, ffun=ffun)
+    assert st["bands"] <= 2, st
+    assert_same(got, orc.gold_scan(orc.Panel(bits, valid, m0, m1, n), k, ffun=ffun), "tiny")
