@@ -653,6 +653,7 @@ int Engine::add(ScanItem *it) {
     pl.entropy = it->ffun == GEPI_FFUNC_ENTROPY;
     pl.evals_tile = (double)total / (double)it->n_tiles;
     pl.h = (double)ca.h0 + (double)ca.h1 * std::min(it->n0, it->n1);
+    pl.sd = fisher_spread(it->n0, it->n1);
     pl.k = (double)it->k;
     pl.c = pl.entropy ? GUESS_ENTROPY : guess_fisher((double)it->k);
     pl.most = (double)it->pcap / 4;

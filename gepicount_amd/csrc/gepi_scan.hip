@@ -574,10 +574,11 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
     plan.entropy = entropy;
     plan.evals_tile = (double)total_evals / (double)n_tiles;
     plan.h = (double)h0 + (double)h1 * std::min(n0, n1);
+    plan.sd = fisher_spread(n0, n1);
     plan.k = (double)k;
     plan.c = guess;
     plan.most = (double)pcap / 4;
-    if (!entropy) plan.spread = 8.0;
+    if (!entropy) plan.spread = 3.0;
     const int64_t first = plan.first(n_tiles);
     const bool planned = fp4 && n_ks > 0 && !hooks && !par->intermediate && par->max_grid_area <= 0 &&
                          plan.sound(first, cap) && short_ranking;

@@ -116,3 +116,25 @@ def test_batch():
     assert bs["rounds"] <= 12, bs
     for it in items:
         it["panel"].close()
+
+
+@pytest.mark.parametrize("n_var,n,k", [(300, 20000, 5000), (420, 46340, 20000)])
+def test_fisher_many_samples(monkeypatch, n_var, n, k):
+    """A table of many samples has a small probability whatever its p, so that
+    the check of P(obs) passes nearly all evaluations under a loose threshold:
+    no guess, in a single scan and batched."""
+    print("case fisher many samples", n_var, n, k, flush=True)
+    rng = np.random.default_rng(45)
+    g = rng.integers(0, 2, (n_var, n)).astype(np.uint8) + (rng.random((n_var, n)) < 0.3)
+    codes = np.array([3, 2, 0], np.uint8)[g]
+    codes[::2][:, ::97] = 1
+    bits, valid = orc.planes_from_codes(codes)
+    m0, m1 = orc.masks_from_classes((rng.random(n) < 0.4).astype(int))
+    with ge.Panel.from_planes(bits, valid, n) as panel:
+        got, st = panel.scan(m0, m1, topmost=k, ffun=1)
+        with ge.Engine() as eng:
+            (res,), bs = eng.scan_batch([dict(panel=panel, mask_ctrl=m0, mask_case=m1, topmost=k, ffun=1)])
+        ref, _ = band_by_band(monkeypatch, panel, m0, m1, k, 1, 20)
+    assert_same(got, ref, "alone")
+    assert_same(res[0], ref, "batch")
+    assert st["bands"] <= 10 and bs["rounds"] <= 12, (st, bs)
