@@ -726,10 +726,8 @@ __device__ __forceinline__ void count_f4_run(const Src &src) {
         if (hasB1) W[dB + D64] = pb1;
     };
 
-    if (tid == 0) {
-        s_job[0] = src.grab(0);
-        stage.n = 0;
-    }
+    stage_init(stage);
+    if (tid == 0) s_job[0] = src.grab(0);
     __syncthreads();
     F4Job job = uniform_job(s_job[0]);
     if (!job.ok) return;
@@ -865,6 +863,7 @@ __device__ __forceinline__ void count_f4_run(const Src &src) {
         __syncthreads(); /* super-step 0 staged; the flush's copies are done */
         if (tid == 0) {
             if (flush) stage.n = 0;
+            if (nj.item != job.item) stage.full = 0;
             s_job[t & 1] = src.grab(t + 2);
         }
         job = nj;

@@ -232,7 +232,7 @@ struct PendStageN {
     static constexpr uint32_t cap = N;
     Pend rec[N];
     uint32_t n;
-    uint32_t pad;
+    uint32_t full; /* the pending list was found full: no more is tested */
     unsigned long long base;
 };
 typedef PendStageN<PEND_LDS> PendStage;
@@ -299,7 +299,10 @@ __device__ __forceinline__ PushSlots push_reserve(const CountArgs &g, PS &ps, ui
             const unsigned long long q = st_add(&g.st->pend_count, (unsigned long long)rest);
             lo = (uint32_t)q;
             hi = (uint32_t)(q >> 32);
-            if (q + rest > g.pcap) mark_full(g);
+            if (q + rest > g.pcap) {
+                mark_full(g);
+                ps.full = 1;
+            }
         }
         lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)lo);
         hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)hi);
@@ -331,7 +334,14 @@ __device__ __forceinline__ void push_pending(const CountArgs &g, PS &ps, PushSlo
  * barrier) and after the last push, respectively.                          */
 template <class PS>
 __device__ __forceinline__ void stage_init(PS &ps) {
-    if (threadIdx.x == 0) ps.n = 0;
+    if (threadIdx.x == 0) {
+        ps.n = 0;
+        ps.full = 0;
+    }
+}
+template <class PS>
+__device__ __forceinline__ bool stage_full(PS &ps) {
+    return __hip_atomic_load(&ps.full, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != 0u;
 }
 
 /* The flush proper: every push is complete (the caller has passed a
@@ -445,6 +455,7 @@ template <int FFUN, class PS>
 __device__ __forceinline__ void push_mask(const CountArgs &g, PS &ps, const FilterConsts &fc,
                                           int32_t A, int32_t B, const int32_t (&c)[2][3][3],
                                           uint32_t mask) {
+    if (stage_full(ps)) return; /* the band is redone */
     const int32_t y = c[0][2][2], z = c[1][2][2];
     /* body(bit, w, x) for the evaluations in mb4, row pair by row pair */
     auto walk = [&](uint32_t mb4, auto body) {
