@@ -243,7 +243,7 @@ inline int32_t pairs_from(int64_t n_tiles) { return n_tiles >= 2048 ? (int32_t)s
  * fourfold, a host round trip (40 us) and a selection between two: 1,024 x
  * 256 0.73 -> 0.13 ms (5 bands -> 1), 3,001 x 777 Fisher 1.44 -> 0.29, 20,000
  * x 2,048 3.69 -> 2.38 (10 -> 3), 8,000 x 20,001 3.84 -> 2.50.               */
-constexpr double GUESS_ENTROPY = 8.0;
+constexpr double GUESS_ENTROPY = 7.5; /* 8: 1,024 x 256 top-100 selects for 54 us, 7.5: 47 */
 /* Fisher: 16 for the 100 best, where a few variants decide, down to 4 for long
  * rankings, whose count varies less: each guessed evaluation that passes the
  * bound costs a walk over its tables (3,000 x 2,000 top-10,000 1.85 -> 0.7 ms,
