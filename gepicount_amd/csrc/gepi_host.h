@@ -281,6 +281,7 @@ struct BandPlan {
     double factor = 1.0; /* survivors measured over survivors expected       */
     double spread = 16.0; /* survivors a list takes over those expected (room) */
     double walks = 65536; /* records scored in little more than one's time     */
+    double limit = 1048576.0; /* tiles of one band at most (longest)           */
 
     /* Expected survivors of the chi-square bound per evaluation under the
      * threshold that admits a share q: its cut is h/2 of the quantile (a few
@@ -352,6 +353,15 @@ struct BandPlan {
     unsigned long long room_again(unsigned long long pcap) const {
         return std::min<unsigned long long>(pcap, (unsigned long long)std::max(4.0 * aim(), gepi::TILE_EVALS_MAX + 1024.0));
     }
+    /* Tiles of one band at most: an eighth of the scan, or what takes about 2
+     * ms (0.7 ns for 64 x 32 pairs and 128 samples).  A few linked variants
+     * late in a band can fill its list, and the time before that is lost: with
+     * the last band as 85% of the scan, 40,000 x 4,096 in linked blocks, five
+     * of them with an effect, entropy top-100, took 20.5 ms and 14.6 now (16.0
+     * in bands that grow without a guess).                                  */
+    static double longest(int64_t n_tiles, int64_t n_ks) {
+        return std::min(1048576.0, std::max((double)n_tiles / 8, 3.0e6 / (double)std::max<int64_t>(1, n_ks)));
+    }
     /* the threshold that lets through what is expected after `done` tiles */
     double share_after(int64_t done) const { return 1.3 * k / ((double)done * evals_tile); }
     /* survivors found in n tiles under the threshold that admits a share q */
@@ -368,7 +378,7 @@ struct BandPlan {
         const double per = survivors(1, share_after(done));
         const double cheap = std::min(std::max(250000.0 / per, 3.0 * (double)done),
                                       (entropy ? 8.0 : 3.0) * (double)done);
-        const double tiles = std::min({cheap, most / per, 1048576.0, (double)left});
+        const double tiles = std::min({cheap, most / per, limit, (double)left});
         /* a remainder below a fifth of the band goes with it */
         if ((double)left < 1.2 * tiles && (double)left * per < most) return left;
         return std::max<int64_t>(1, (int64_t)tiles);

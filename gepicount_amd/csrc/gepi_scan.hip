@@ -582,6 +582,7 @@ int run_scan(gepi_panel *p, const uint64_t *mask_ctrl, const uint64_t *mask_case
     const int64_t first = plan.first(n_tiles);
     const bool planned = fp4 && n_ks > 0 && !hooks && !par->intermediate && par->max_grid_area <= 0 &&
                          plan.sound(first, cap) && short_ranking;
+    if (planned) plan.limit = BandPlan::longest(n_tiles, n_ks);
     if (!planned && !noalloc) {
         cap = cap_full;
         pcap = pend_cap(cap);

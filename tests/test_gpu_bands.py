@@ -86,3 +86,20 @@ def test_tiny_panels(n_var, n, k, ffun):
         got, st = panel.scan(m0, m1, topmost=k, ffun=ffun)
     assert st["bands"] <= 2, st
     assert_same(got, orc.gold_scan(orc.Panel(bits, valid, m0, m1, n), k, ffun=ffun), "tiny")
+
+
+@pytest.mark.parametrize("ffun", [0, 1])
+def test_long_bands(monkeypatch, ffun):
+    """No planned band of a long scan is much more than an eighth of it: what
+    one that turns out to pass too much has cost is small."""
+    print("case long bands ffun=%d" % ffun, flush=True)
+    rng = np.random.default_rng(75)
+    byte = np.array([a | b << 2 | c << 4 | d << 6 for a in (0, 2, 3) for b in (0, 2, 3) for c in (0, 2, 3) for d in (0, 2, 3)], np.uint8)
+    n_var, n = 40000, 4096
+    payload = byte[rng.integers(0, 81, (n_var, n // 4), np.uint8)]
+    m0, m1 = orc.masks_from_classes(rng.integers(0, 2, n))
+    with ge.Panel.from_bed(payload, n_var, n) as panel:
+        got, st = panel.scan(m0, m1, topmost=100, ffun=ffun)
+        ref, _ = band_by_band(monkeypatch, panel, m0, m1, 100, ffun, 65536)
+    assert st["bands"] >= 6, st
+    assert_same(got, ref, "long bands")
