@@ -59,6 +59,8 @@ struct ScanItem {
     bool guessed = false; /* the first band runs under a guessed threshold    */
     BandPlan plan{};
     int64_t first = 0;    /* tiles of that band                               */
+    double q = 0;           /* the share of evaluations its threshold admits   */
+    bool looser = false;    /* ... after one that admitted too few             */
     bool misjudged = false; /* it overflowed a list: it is redone in parts */
     unsigned long long room() const { /* in the pending list of the next band */
         if (!guessed || t0 >= first) return pcap;

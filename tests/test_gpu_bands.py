@@ -103,3 +103,28 @@ def test_long_bands(monkeypatch, ffun):
         ref, _ = band_by_band(monkeypatch, panel, m0, m1, 100, ffun, 65536)
     assert st["bands"] >= 6, st
     assert_same(got, ref, "long bands")
+
+
+def test_batch_guess_too_strict():
+    """With 8 cases few tables are as improbable as the guess assumes: the
+    scans of a batch go on under a looser one, not from a single tile."""
+    print("case batch guess too strict", flush=True)
+    rng = np.random.default_rng(77)
+    codes = np.array([0, 2, 3], np.uint8)
+    items, refs = [], []
+    for j in range(4):
+        f = rng.uniform(0.05, 0.5, (3000, 1, 1))
+        dose = (rng.random((3000, 400, 2)) < f).sum(2)
+        bits, valid = orc.planes_from_codes(codes[dose])
+        cls = np.zeros(400, np.int64)
+        cls[rng.choice(400, 8, replace=False)] = 1
+        m0, m1 = orc.masks_from_classes(cls)
+        items.append(dict(panel=ge.Panel.from_planes(bits, valid, 400), mask_ctrl=m0, mask_case=m1, topmost=100, ffun=1))
+        refs.append(items[-1]["panel"].scan(m0, m1, topmost=100, ffun=1)[0])
+    eng = ge.Engine()
+    res, bs = eng.scan_batch(items)
+    eng.close()
+    for j in range(4):
+        items[j]["panel"].close()
+        assert_same(res[j][0], refs[j], "batch %d" % j)
+    assert bs["rounds"] <= 4, bs
