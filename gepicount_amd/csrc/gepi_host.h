@@ -353,14 +353,15 @@ struct BandPlan {
     unsigned long long room_again(unsigned long long pcap) const {
         return std::min<unsigned long long>(pcap, (unsigned long long)std::max(4.0 * aim(), gepi::TILE_EVALS_MAX + 1024.0));
     }
-    /* Tiles of one band at most: an eighth of the scan, or what takes about 2
-     * ms (0.7 ns for 64 x 32 pairs and 128 samples).  A few linked variants
+    /* Tiles of one band at most: a third of the scan (100,000 x 8,192
+     * ran 1.5% slower with an eighth, 0.3-0.8% with a quarter, 0-0.5% so), or what
+     * takes about 2 ms (0.7 ns for 64 x 32 pairs and 128 samples).  A few linked variants
      * late in a band can fill its list, and the time before that is lost: with
      * the last band as 85% of the scan, 40,000 x 4,096 in linked blocks, five
-     * of them with an effect, entropy top-100, took 20.5 ms and 14.6 now (16.0
+     * of them with an effect, entropy top-100, took 20.5 ms and 15.8 now (16.1
      * in bands that grow without a guess).                                  */
     static double longest(int64_t n_tiles, int64_t n_ks) {
-        return std::min(1048576.0, std::max((double)n_tiles / 8, 3.0e6 / (double)std::max<int64_t>(1, n_ks)));
+        return std::min(1048576.0, std::max((double)n_tiles / 3, 3.0e6 / (double)std::max<int64_t>(1, n_ks)));
     }
     /* the threshold that lets through what is expected after `done` tiles */
     double share_after(int64_t done) const { return 1.3 * k / ((double)done * evals_tile); }

@@ -90,7 +90,7 @@ def test_tiny_panels(n_var, n, k, ffun):
 
 @pytest.mark.parametrize("ffun", [0, 1])
 def test_long_bands(monkeypatch, ffun):
-    """No planned band of a long scan is much more than an eighth of it: what
+    """No planned band of a long scan is much more than a third of it: what
     one that turns out to pass too much has cost is small."""
     print("case long bands ffun=%d" % ffun, flush=True)
     rng = np.random.default_rng(75)
