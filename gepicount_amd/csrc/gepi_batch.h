@@ -1,8 +1,9 @@
 /*
  * gepi_batch.h -- kernels of the batched scan engine.  Many scans (panels
  * and phenotype vectors of different sizes) advance together in rounds; a
- * round is three kinds of launch whatever the number of scans (one count
- * launch per objective and job shape present):
+ * round is four kinds of launch whatever the number of scans (one count
+ * launch per objective and job shape present, k_pairs_batch only where scans
+ * put pairs off):
  *
  *   k_count_f4_batch  one band of fp4 count tiles per scan in one persistent
  *                     grid: workgroups take (scan, tile) slots from per-XCD
@@ -10,7 +11,10 @@
  *   k_count_f4w_batch the same for scans on wave tiles (Fisher's, and long
  *                     entropy scans): one (scan, unit of two tiles) slot per
  *                     workgroup
- *   k_count_f4g_batch the same on genotype planes (every .bed panel's)
+ *   k_count_f4g_batch the same on genotype planes (every .bed panel's, unless
+ *                     its classes are too uneven for the screen), where no
+ *                     call is missing k_count_f4c_batch
+ *   k_pairs_batch     the tests of the pairs that those two put off
  *   k_exact_batch     exact scores of each scan's filter survivors
  *                     (blockIdx.y = scan)
  *   k_topk_wg         one 1024-thread workgroup per scan: radix select of

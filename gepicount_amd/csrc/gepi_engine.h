@@ -1,13 +1,14 @@
 /*
  * gepi_engine.h -- the batched scan engine (host side).  Scans are added at
  * any time and advance together in rounds; a round is one count launch per
- * objective and job shape present, one exact-score launch and one top-k
- * launch for all active
- * scans, then a single read of their reports; with GEPI_ENGINE_GRAPH=1 a
- * round's launches are replayed from two captured HIP graphs.  The batch C
- * ABI runs rounds
- * until every scan is done; the serving loop admits new requests between
- * rounds.  All device work runs on the engine's stream.
+ * objective and job shape present (and one of k_pairs_batch for each on
+ * genotype planes), one exact-score launch and one top-k launch
+ * for all active scans, then a single read of their reports; with
+ * GEPI_ENGINE_GRAPH=1 a round's launches are replayed from two captured HIP
+ * graphs.  A scan's first band runs under a guessed threshold and the others
+ * are sized as in a planned single scan (BandPlan).  The batch C ABI runs
+ * rounds until every scan is done; the serving loop admits new requests
+ * between rounds.  All device work runs on the engine's stream.
  */
 #ifndef GEPI_ENGINE_H
 #define GEPI_ENGINE_H
@@ -131,7 +132,7 @@ class Engine {
      * groups in bit mask part: bit g = objective (g & 1: 0 entropy, 1
      * Fisher) and job shape (g >> 1: 0 whole tiles, 1 half tiles)), part
      * NGRAPH_COUNT into gx_finish_ (exact + top-k launches).  Wave-tile
-     * groups (4-7) have no persistent form and are never captured: with
+     * groups (4-9) have no persistent form and are never captured: with
      * graphs on, scans keep whole tiles instead.                          */
     int capture_graph(int part, int per_cu);
     /* One count launch of group g (as in capture_graph). */

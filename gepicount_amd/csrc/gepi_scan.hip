@@ -14,15 +14,22 @@
  *   classes  [n_var_pad][3][wc] u32 per scan: samples reordered so that class
  *            0 (controls) then class 1 (cases) are contiguous, each segment
  *            zero-padded to 128 bits; class masks become word ranges.
- *   classes_k [n_ks][n_var_pad][3] u64 (MFMA path): the same bits K-major.
- *   pend     [cap] 16-byte filter survivors; cand [2][cap] 32-byte candidates.
+ *   classes_k [n_ks][n_var_pad][3] u64 (MFMA path): the same bits K-major
+ *            (fp4 paths: in super-steps, allele or genotype planes).
+ *   pend     16-byte filter survivors; cand 32-byte candidates, a second list
+ *            of them only for rankings that one workgroup does not select.
+ *   pairs    48-byte variant pairs that the count kernel puts off (genotype
+ *            planes, short rankings; left out where memory is short).
  *
  * A scan walks the lower triangle of variant tiles in bands: count kernel
- * (filter survivors -> pend), k_exact (exact score, admit keys <= threshold
- * -> cand), then, when more than k candidates exist, a radix select of the
- * k-th key, compaction to exactly k records and a new threshold.  The host
- * synchronises once per band to read the state and size the next band; only
- * the final k records are copied to the host.
+ * (filter survivors -> pend), k_pairs (the tests put off), k_exact (exact
+ * score, admit keys <= threshold -> cand), then, when more than k candidates
+ * exist, a select of the k-th key, compaction to exactly k records and a new
+ * threshold.  Short rankings on the fp4 paths run as planned bands: a first
+ * one under a guessed threshold, then all others enqueued at once, one
+ * synchronisation after each (BandPlan).  Otherwise the host synchronises
+ * once per band to read the state and size the next.  Only the final k
+ * records are copied to the host.
  */
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>

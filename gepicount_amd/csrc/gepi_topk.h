@@ -6,8 +6,11 @@
  *
  * Keys are (order_bits(score), idx) as 128-bit unsigned values; idx orders
  * like (sA, sB, fun), so the key order is the canonical (score, sA, sB, fun).
- * The select is an MSB-first radix select with 8-bit digits that finishes
- * with a bitonic sort in LDS once at most SEL_SMALL keys share the prefix.
+ * Two selects of the k-th key: for lists of at most WG_SELECT_MAX records one
+ * workgroup (12-bit digits of the score, and the idx of those that tie), for
+ * longer ones a chain of launches, an MSB-first radix select with 8-bit digits
+ * that finishes with a bitonic sort in LDS once at most SEL_SMALL keys share
+ * the prefix.
  */
 #ifndef GEPI_TOPK_H
 #define GEPI_TOPK_H

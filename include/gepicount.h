@@ -70,8 +70,12 @@ typedef struct gepi_params {
     int32_t gpu_num;       /* -G: HIP device ordinal                           */
     int32_t ffun;          /* -f: gepi_ffunc                                   */
     int64_t topmost;       /* -N: results to keep                              */
-    int32_t count_path;    /* 0 = fastest (3 from 10 K steps of 128 samples or
-                            * about 2,900 variants, else 4; in
+    int32_t count_path;    /* 0 = fastest (3 from 10 K steps of 128 samples on;
+                            * where classes and genotypes suit the screen
+                            * of path 3, also from about 1,000 variants, for
+                            * Fisher about 2,900 and 4 for rankings of more
+                            * than one in 800,000 evaluations, 400,000
+                            * without missing calls; else 4; in
                             * gepi_scan_noalloc 3 from 10 K steps, 4 for
                             * Fisher),
                             * 1 = popcount (VALU), 2 = int8 MFMA, 3 = fp4
@@ -198,7 +202,7 @@ int gepi_panel_filter(gepi_panel *panel, float max_miss_snps, float max_miss_sam
 
 /* ---- batched scans ---------------------------------------------------------
  * Many scans (panels of any size, phenotype vectors) advance together in
- * rounds of three launches, so small scans share the GPU instead of
+ * rounds of a few launches, so small scans share the GPU instead of
  * running one after another.  No counterpart in the reference, which runs
  * one process_gpu_1 per process (src/gEpiCount.cpp:84-87); each item's
  * result is identical to gepi_scan's on the same input (fp4 count path).
@@ -265,8 +269,10 @@ typedef struct gepi_tune_class {
  * CU, or wave tiles; x 5e8, 2e9 or 8e9 evaluations per band), repeats times
  * each, and keeps the fastest (the default unless another is more than 3%
  * faster).  The default schedule: 2 persistent workgroups per CU, 2e9
- * evaluations per band, entropy scans of at least 48 K steps or about 1,000
- * variants on wave tiles and smaller ones on 64 x 32 tiles.  The engine uses the table from then
+ * evaluations per band, entropy scans of at least 48 K steps, or of about 1,000
+ * variants whose classes and genotypes suit the screen, on wave tiles and others
+ * on 64 x 32 tiles; a class whose best job shape is the default's keeps the
+ * default for each scan (reserved = 1).  The engine uses the table from then
  * on: a scan's job shape and band size by its class, a round's launch form
  * by the class with the most count work in it.  A table that differs from
  * the default is kept only if it is also 1% faster on all 16 trial scans
@@ -303,7 +309,9 @@ typedef struct gepi_server_params {
                                 before the first request                      */
     int64_t hbm_budget;      /* scan workspace admitted at once, bytes; 0 = 3/4
                                 of the device memory free at creation; a
-                                request larger than the budget runs alone      */
+                                request larger than the budget runs alone;
+                                lists that only save time are left out of a
+                                scan where they do not fit                     */
     int64_t round_wg_budget; /* workgroups per count round; 0 = 262,144: bounds
                                 how long a new request waits to join          */
 } gepi_server_params;
